@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 
 namespace reef {
 
@@ -30,6 +31,19 @@ int prog_index(int kind, int gcv)
 }
 
 }  // namespace
+
+// The engine of this process whose on-chip launch was the last one on each GPU.  Blocks of an
+// on-chip launch wait for each other, so two launches must not share the CUs half and half:
+// an engine whose stream is not the last one's makes its stream wait for that launch first.
+static std::mutex g_chip_mu;
+static std::map<int, std::pair<const Engine*, hipEvent_t>> g_chip_last;
+
+static void chip_leave(const Engine* e)
+{
+    std::lock_guard<std::mutex> lk(g_chip_mu);
+    for(auto it = g_chip_last.begin(); it != g_chip_last.end();)
+        it = it->second.first == e ? g_chip_last.erase(it) : std::next(it);
+}
 
 // ------------------------------------------------------------------ device pool
 DevicePool::~DevicePool()
@@ -153,6 +167,9 @@ Engine::~Engine()
 {
     if(stream) (void)hipStreamSynchronize(stream);
     drop_graphs();
+    chip_leave(this);
+    if(chip_ev_) (void)hipEventDestroy(chip_ev_);
+    if(d_chip_) (void)hipFree(d_chip_);
     for(auto& r : ranges_)
     {
         (void)hipEventDestroy(r.a);
@@ -378,6 +395,7 @@ int Engine::add_built(TankBuild& b, int* id)
         D.gnops[q] = b.nop[q];
     }
     D.shape = shape_of(h);
+    t.chip_h.fill(-1);
     // slot
     int slot = -1;
     for(size_t q = 0; q < tanks.size(); ++q)
@@ -506,6 +524,8 @@ int Engine::sync_tables()
         if(tanks[q].used && tanks[q].active) act.push_back(q);
     all_ = make_sets(act);
     cur_ = &all_;
+    for(TankHost& t : tanks) t.chip_h.fill(-1);   // plans may have changed
+    all_chip_ = chip_plan(act);
     solving_key_.clear();
     solving_sets_.clear();
     last_state.resize(nslot, BiState{});
@@ -892,11 +912,168 @@ static const char* const BICG_NAMES[5] = {"bicg_p", "bicg_v", "bicg_t", "bicg_x"
 static const char* const MIX_NAMES[4] = {"mix_v", "bicg32_t", "bicg32_x", "mix_ru"};
 static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 
-// 8 iterations of the tanks of the current sets, then their states gathered into ring
-// slot `ring` and copied to the host.  Iterations after a tank's end are no-ops for it.
+// ------------------------------------------------------------------ on-chip solves
+// Blocks of tank t with at most per_block tiles each: the smallest power of two, at most 256
+// and the tank's items; 0 when the tank does not fit or its sums are taken in another order
+// (a 2-D tank with cpt > 1 walks its rows in the streaming v and t phases).
+int Engine::chip_blocks(TankHost& t, int per_block) const
+{
+    const TileShape& s = t.dev.shape;
+    if(s.ntiles > CHIP_TILES || s.cpt > CHIP_CPT_MAX || (t.hg.jdir == 0 && s.cpt > 1)) return 0;
+    // items a block's two groups hold at four tile slots each, within per_block tiles
+    const int most = std::max(1, std::min(2 * (CHIP_TILES_PER_BLOCK / 2 / s.cpt), per_block / s.cpt));
+    for(int q = 0, nb = 1; nb <= CHIP_BLOCKS && nb <= s.nitems; ++q, nb *= 2)
+    {
+        if((s.nitems + nb - 1) / nb > most) continue;
+        if(t.chip_h[q] < 0) t.chip_h[q] = chip_halo(s, nb);
+        if(t.chip_h[q] <= CHIP_HALO_MAX) return nb;
+    }
+    return 0;
+}
+
+// On-chip launches for the slots: a launch holds tanks of at most 256 blocks together.  Two
+// tiles per block where everything then fits one launch (an exchange among fewer blocks is
+// cheaper, but so is less work per thread), else four, else eight and several launches.
+Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots)
+{
+    ChipPlan P;
+    auto pack = [&](int per_block) {
+        P.launches.clear();
+        P.rest.clear();
+        for(int q : slots)
+        {
+            TankHost& t = tanks[q];
+            const int nb = chip_off_ ? 0 : chip_blocks(t, per_block);
+            if(nb == 0)
+            {
+                P.rest.push_back(q);
+                continue;
+            }
+            ChipSet* S = nullptr;
+            for(ChipSet& L : P.launches)
+                if(L.d3 == t.hg.jdir && L.n < CHIP_TANKS && L.blk0[L.n] + nb <= CHIP_BLOCKS) S = &L;
+            if(!S)
+            {
+                P.launches.emplace_back();
+                S = &P.launches.back();
+                std::memset(S, 0, sizeof(*S));
+                S->d3 = t.hg.jdir;
+            }
+            S->tanks = d_tanks_;
+            S->slot[S->n] = q;
+            S->tile0[S->n] = S->blk0[S->n] * CHIP_TILES_PER_BLOCK;
+            S->blk0[S->n + 1] = S->blk0[S->n] + nb;
+            S->hmax = std::max(S->hmax, t.chip_h[31 - __builtin_clz((unsigned)nb)]);
+            S->slots = std::max(S->slots, (chip_items(t.dev.shape, nb, 0) + 1) / 2 * t.dev.shape.cpt);
+            S->n += 1;
+        }
+    };
+    pack(CHIP_TILES_PER_BLOCK);
+    const size_t rest = P.rest.size();
+    for(int per_block = CHIP_FIRST; per_block <= CHIP_TILES_PER_BLOCK; per_block *= 2)
+    {
+        pack(per_block);
+        if(P.launches.size() <= 1 && P.rest.size() == rest) break;
+    }
+    P.stream_all = P.launches.empty();
+    if(!P.stream_all && !P.rest.empty()) P.rest_sets = make_sets(P.rest);
+    return P;
+}
+
+int Engine::chip_alloc()
+{
+    if(d_chip_) return 0;
+    const int rc = chip_prepare();
+    if(rc) return fail(rc, "on-chip solver: dynamic LDS limit not accepted");
+    const size_t bytes = (CHIP_HALO_WORDS + (size_t)CHIP_TANKS * CHIP_ACC_WORDS) * 8 + CHIP_CTL * sizeof(unsigned);
+    unsigned long long* d = nullptr;
+    EHIP(hipMalloc(&d, bytes));
+    if(!chip_ev_)
+    {
+        const hipError_t e = hipEventCreateWithFlags(&chip_ev_, hipEventDisableTiming);
+        if(e != hipSuccess)
+        {
+            (void)hipFree(d);
+            return fail(REEF_E_HIP, std::string("hipEventCreateWithFlags: ") + hipGetErrorString(e));
+        }
+    }
+    const hipError_t e = hipMemsetAsync(d, 0, bytes, stream);
+    if(e != hipSuccess)
+    {
+        (void)hipFree(d);
+        return fail(REEF_E_HIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
+    }
+    d_chip_ = d;
+    chip_epoch_ = 1;
+    chip_ctl_ = 0;
+    return 0;
+}
+
+// the on-chip launches of the plan, each up to cap iterations
+int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
+{
+    int rc;
+    if((rc = chip_alloc())) return rc;
+    unsigned long long* acc = d_chip_ + CHIP_HALO_WORDS;
+    unsigned* ctl = (unsigned*)(acc + (size_t)CHIP_TANKS * CHIP_ACC_WORDS);
+    int dev = 0;
+    EHIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_chip_mu);
+    auto& last = g_chip_last[dev];
+    if(last.first && last.first != this) EHIP(hipStreamWaitEvent(stream, last.second, 0));
+    for(ChipSet& S : P.launches)
+    {
+        // tags and commit words are never used twice without clearing the workspace
+        if(chip_epoch_ > 0xffffffffu - 2 * CHIP_EPOCHS || chip_ctl_ + S.n > CHIP_CTL)
+        {
+            const bool tags = chip_epoch_ > 0xffffffffu - 2 * CHIP_EPOCHS;
+            if(tags) EHIP(hipMemsetAsync(d_chip_, 0, (CHIP_HALO_WORDS + (size_t)CHIP_TANKS * CHIP_ACC_WORDS) * 8, stream));
+            EHIP(hipMemsetAsync(ctl, 0, CHIP_CTL * sizeof(unsigned), stream));
+            if(tags) chip_epoch_ = 1;
+            chip_ctl_ = 0;
+        }
+        S.halo = d_chip_;
+        S.acc = acc;
+        S.ctl = ctl + chip_ctl_;
+        S.epoch = chip_epoch_;
+        S.cap = cap;
+        tbegin("chip");
+        bl_chip_solve(S, kind, x, rhs, stream);
+        tend();
+        const hipError_t e = hipGetLastError();
+        if(e != hipSuccess) return fail(REEF_E_HIP, std::string("on-chip solver launch: ") + hipGetErrorString(e));
+        chip_epoch_ += CHIP_EPOCHS;
+        chip_ctl_ += S.n;
+    }
+    EHIP(hipEventRecord(chip_ev_, stream));
+    last = {this, chip_ev_};
+    return 0;
+}
+
+// Iterations of the current sets' tanks: `iters` by the streaming phases; the tanks that fit
+// the on-chip solver run there instead, up to chip_cap iterations in one launch.  Iterations
+// after a tank's end are no-ops for it.
+int Engine::enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap)
+{
+    ChipPlan* P = cur_ == &all_ ? &all_chip_ : cur_ == &solving_sets_ ? &solving_chip_ : nullptr;
+    if(P && !chip_off_ && !P->stream_all)
+    {
+        int rc = chip_launch(*P, kind, x, rhs, chip_cap);
+        if(rc || P->rest.empty()) return rc;
+        const std::vector<TankSet>* keep = cur_;
+        const bool lockstep = cur_ == &all_;
+        cur_ = &P->rest_sets;
+        rc = stream_iterations(kind, x, rhs, iters, lockstep);
+        cur_ = keep;
+        return rc;
+    }
+    return stream_iterations(kind, x, rhs, iters, cur_ == &all_);
+}
+
+// `iters` streaming iterations of the current sets (8 launches of two parts each).
 // kind: SOLVE_FP64 (the Poisson operator), SOLVE_MIXED, or SOLVE_MAT (the explicit
 // 7-diagonal operator; rhs is then the FLEXLOOP var)
-int Engine::enqueue_batch(int kind, int x, int rhs, int ring, int iters)
+int Engine::stream_iterations(int kind, int x, int rhs, int iters, bool lockstep)
 {
     const int nph = 4;
     const char* const* names = kind == SOLVE_MIXED ? MIX_NAMES : kind == SOLVE_MAT ? MAT_NAMES : BICG_NAMES;
@@ -922,12 +1099,12 @@ int Engine::enqueue_batch(int kind, int x, int rhs, int ring, int iters)
     int rc;
     // the lockstep sets only change with the tables; the scheduler's solving sets change
     // from round to round, and a set's batch graph is captured when the set comes back
-    if(cur_ == &all_)
-        rc = replay({1, kind, x, rhs * 64 + iters}, body);
-    else if(graphs && !timing && cur_ == &solving_sets_)
+    if(lockstep)
+        rc = replay({1, kind, x, (rhs * 64 + iters) * 2 + (cur_ == &all_)}, body);
+    else if(graphs && !timing)
     {
         std::vector<int> key(solving_key_);
-        key.insert(key.end(), {-1, kind, x, rhs, iters});
+        key.insert(key.end(), {-1, kind, x, rhs, iters, cur_ == &solving_sets_});
         // a full cache captures no more sets (their batches launch directly) rather than
         // destroying executable graphs in the middle of a run: graph execs are destroyed only
         // when the tables change (drop_graphs, after a stream synchronisation) and at teardown
@@ -950,7 +1127,15 @@ int Engine::enqueue_batch(int kind, int x, int rhs, int ring, int iters)
     }
     else
         rc = body();
-    if(rc) return rc;
+    return rc;
+}
+
+// one batch: the iterations, then the states of the current sets gathered into ring slot
+// `ring` and copied to the host
+int Engine::enqueue_batch(int kind, int x, int rhs, int ring, int iters)
+{
+    int rc;
+    if((rc = enqueue_iterations(kind, x, rhs, iters, CHIP_CAP))) return rc;
     BiState* dst = d_status_ + (size_t)ring * cap_tanks_;
     each([&](const TankSet& S) { bl_gather_states(S, dst, stream); });
     EHIP(hipMemcpyAsync(h_status_ + (size_t)ring * cap_tanks_, dst, sizeof(BiState) * tanks.size(),
@@ -968,20 +1153,27 @@ int Engine::run_iterations(int kind, int x, int rhs, int maxiter)
     for(const TankSet& S : *cur_)
         for(int p = 0; p < S.n; ++p) members.push_back(S.slot[p]);
     int rc;
+    // an on-chip batch usually is the whole solve: nothing is enqueued behind it
+    auto ahead = [&] { return chip_off_ || cur_ != &all_ || all_chip_.stream_all || !all_chip_.rest.empty(); };
     if((rc = enqueue_batch(kind, x, rhs, 0, 8))) return rc;
+    bool queued = false;   // batch k is behind batch k - 1
     for(long k = 1;; ++k)
     {
-        if((rc = enqueue_batch(kind, x, rhs, (int)(k & 1), 8))) return rc;
+        if((queued = ahead()) && (rc = enqueue_batch(kind, x, rhs, (int)(k & 1), 8))) return rc;
         EHIP(hipEventSynchronize(st_ev_[(k - 1) & 1]));
         const BiState* hs = h_status_ + (size_t)((k - 1) & 1) * cap_tanks_;
         bool all = true;
         for(int q : members)
+        {
             if(!hs[q].done) all = false;
+            if(hs[q].chip_fail) chip_off_ = true;   // the solve goes on streaming
+        }
         if(all)
         {
             for(int q : members) last_state[q] = hs[q];
             break;
         }
+        if(!queued && (rc = enqueue_batch(kind, x, rhs, (int)(k & 1), 8))) return rc;
         if(timing && ranges_.size() > 2048) tcollect();
         if(k * 8 > 4L * (maxiter + 16)) return fail(REEF_E_HIP, "BiCGStab did not terminate");
     }
@@ -1521,6 +1713,7 @@ int Engine::read_batch(const Inflight& f)
         TankHost& t = tanks[m.first];
         if(!t.used || t.seq != m.second || !solving_pc(t.pc)) continue;
         const BiState& st = hs[m.first];
+        if(st.chip_fail) chip_off_ = true;
         if(!st.done) continue;
         t.iters_step += st.iter;
         last_state[m.first] = st;
@@ -1590,6 +1783,7 @@ int Engine::pump(std::vector<int>& stepped)
         if(solving != solving_key_)
         {
             solving_sets_ = make_sets(solving);
+            solving_chip_ = chip_plan(solving);
             solving_key_ = solving;
         }
         const int ring = (int)(batch_no_++ & 1);
@@ -1714,16 +1908,7 @@ int Engine::probe(double& stencil_ms, double& solver_ms)
         bl_fill(S, REEF_PCORR, 0.0, stream);
     });
     if((rc = solve_begin(REEF_PCORR, A_RHS, 1e-300, 16, mixed))) return rc;
-    for(int it = 0; it < 16; ++it)
-        for(int ph = 0; ph < 4; ++ph)
-            for(int part = 0; part < 2; ++part)
-                each([&](const TankSet& S) {
-                    if(mixed)
-                        bl_mixed_phase(S, REEF_PCORR, A_RHS, ph, part, stream);
-                    else
-                        bl_bicg_phase(S, REEF_PCORR, A_RHS, ph, part, stream);
-                });
-    if(mixed) each([&](const TankSet& S) { bl_mixed_settle(S, stream); });
+    if((rc = enqueue_iterations(mixed ? SOLVE_MIXED : SOLVE_FP64, REEF_PCORR, A_RHS, 16, 16))) return rc;
     if((rc = solve_end(REEF_PCORR, mixed))) return rc;
     EHIP(hipEventRecord(ev[2].e, stream));
     EHIP(hipEventSynchronize(ev[2].e));

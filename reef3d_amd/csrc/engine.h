@@ -14,9 +14,10 @@
 // A tank's arithmetic is the same either way, alone or with any other tanks.
 #pragma once
 
-#include "batch.h"
+#include "chip.h"
 
 #include <array>
+#include <atomic>
 #include <deque>
 #include <map>
 #include <string>
@@ -66,6 +67,8 @@ struct TankHost
     std::vector<void*> mem;         // pool blocks
     size_t bytes = 0;               // device bytes of the tank
     std::vector<double> staging;
+    // on-chip solver (Engine::chip_plan): largest halo of a block with 2^q blocks, -1 unknown
+    std::array<int, 9> chip_h;
     // iteration-level scheduling (start_steps / pump)
     int pc = -1;                    // -1 idle; 0, 2, 4, 6: segment pc / 2 next; 1, 3, 5: solving
     int seq = 0;                    // solves started
@@ -297,6 +300,29 @@ private:
     template<class Body>
     int replay(const GraphKey& key, Body body);
     int enqueue_batch(int kind, int x, int rhs, int ring, int iters);
+    // On-chip solves (kernels_chip.hip).  chip_plan splits slots into launches of the on-chip
+    // solver and the tanks that stay with the streaming phases; the plan of the current sets is
+    // kept with them.  The workspace belongs to the engine's stream: launches of one engine
+    // follow each other, those of another engine of the process wait for them (chip_order).
+    struct ChipPlan
+    {
+        std::vector<ChipSet> launches;
+        std::vector<int> rest;              // slots that stream
+        std::vector<TankSet> rest_sets;
+        bool stream_all = false;            // every slot streams: the caller's sets are used
+    };
+    ChipPlan all_chip_, solving_chip_;
+    unsigned long long* d_chip_ = nullptr;  // halo words, then accumulator words, then commit words
+    unsigned chip_epoch_ = 0;
+    int chip_ctl_ = 0;                      // next unused commit word
+    bool chip_off_ = false;                 // a launch gave up waiting: another process shares the GPU
+    hipEvent_t chip_ev_ = nullptr;
+    int chip_blocks(TankHost& t, int per_block) const;
+    ChipPlan chip_plan(const std::vector<int>& slots);
+    int chip_alloc();
+    int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);
+    int enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap);
+    int stream_iterations(int kind, int x, int rhs, int iters, bool lockstep);
     int drain();
     int read_batch(const Inflight& b);
     int run_iterations(int kind, int x, int rhs, int maxiter);

@@ -12,6 +12,7 @@
 // stencil results are bit-identical to the reference whatever the set.
 #include "batch.h"
 #include "cell_ops.h"
+#include "solver_state.h"
 
 #include <algorithm>
 #include <mutex>
@@ -20,19 +21,6 @@ namespace reef {
 namespace bk {
 
 // ------------------------------------------------------------------ work walk
-// The tank table is never written by a kernel: reading it through the constant address
-// space lets the compiler use scalar loads (the tank's pointers and sizes stay in SGPRs).
-// Kernels take the tank by reference there and copy only its DevGrid: indexing a local
-// copy of the pointer table with a run-time array id would keep the whole table in
-// registers.
-// (the host compilation pass of this file never runs device code and has no such
-// address space)
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef __attribute__((address_space(4))) const TankDev CTank;
-#else
-typedef const TankDev CTank;
-#endif
-
 // index p with a[p] <= g < a[p + 1] in a set's prefix array a[0..n]
 __device__ __forceinline__ int set_find(const int* a, int n, int g)
 {
@@ -204,43 +192,10 @@ __device__ __forceinline__ void tank_totals(CTank& T, const TankSet& b, double (
     sum_partials<M>(b.partials + (size_t)T.item0 * M, T.shape.nitems, tot);
 }
 
-// ------------------------------------------------------------------ reliable-update outcome
-// The state that a reliable update (mode 3) or restart (mode 1) of the mixed solve leaves,
-// from the FP64 sums of its residual phase tot = {|r|^2, (r0, r)} (kb_mix_ru).  The phase
-// has no finalize launch of its own: the blocks of the next v phase evaluate the outcome
-// from the same sums (they need beta and the mode), kb_fin_v stores it, and
-// kb_fin_mix_ru stores it after the last iteration of a batch, so the states the host
-// reads are settled.  An idle phase then costs one launch, not two.
-struct RuNext
-{
-    double rn, residual, r_j, norm_r0, beta;
-    int iter, done, mode;
-};
-
+// the sums of a reliable-update phase (RuNext)
 __device__ __forceinline__ void tank_totals_ru(CTank& T, const TankSet& b, double (&tot)[2])
 {
     sum_partials<2>(b.partials_ru + (size_t)T.item0 * 2, T.shape.nitems, tot);
-}
-
-__device__ __forceinline__ RuNext ru_next(const BiState* st, const double (&tot)[2])
-{
-    RuNext n;
-    n.rn = sqrt(tot[0]);
-    n.residual = n.rn / double(st->ncell);
-    n.iter = st->iter + (st->mode == 1 ? 1 : 0);   // a restart counts as an iteration (bicgstab_ijk.cpp:183-191)
-    n.done = !((n.residual >= st->stop) && (n.iter < st->maxiter));
-    n.mode = st->mode == 1 ? 2 : 0;
-    n.r_j = tot[1];
-    n.norm_r0 = st->norm_r0;
-    n.beta = st->beta;
-    if(st->mode == 1)
-        n.norm_r0 = sqrt(tot[1]);
-    else
-    {
-        const double wr = st->w * st->r_j_prev;
-        n.beta = st->alpha * tot[1] / (wr == 0 ? 1.0e-15 : wr);
-    }
-    return n;
 }
 
 // the outcome as the v phase needs it: mode (0 or 2; 4 for done) in the high word, the FP32
@@ -264,36 +219,6 @@ __device__ __noinline__ int restart_done(const double* __restrict__ parts, int n
     sum_partials<1>(parts, nitems, tot);
     const double residual = sqrt(tot[0]) / double(st->ncell);
     return !((residual >= st->stop) && (st->iter + 1 < st->maxiter));
-}
-
-__device__ __forceinline__ void restart_store(BiState* st, double rr)
-{
-    st->r_j = rr;
-    st->rr = rr;
-    st->norm_r0 = sqrt(rr);
-    st->residual = sqrt(rr) / double(st->ncell);
-    st->iter += 1;
-    if(!((st->residual >= st->stop) && (st->iter < st->maxiter))) st->done = 1;
-    st->mode = 2;
-}
-
-// stores the outcome (one thread)
-__device__ __forceinline__ void ru_store(BiState* st, const RuNext& n)
-{
-    st->residual = n.residual;
-    st->nru += 1;
-    st->pending = 1;
-    st->rmax = n.rn;
-    st->iter = n.iter;
-    if(n.done)
-    {
-        st->done = 1;
-        return;
-    }
-    st->r_j = n.r_j;
-    st->norm_r0 = n.norm_r0;
-    st->beta = n.beta;
-    st->mode = n.mode;
 }
 
 // ------------------------------------------------------------------ per-precision views
@@ -1160,6 +1085,7 @@ __global__ void kb_setup(TankSet b, double stop, int maxiter, int mixed, double 
     st->pending = 0;
     st->nru = 0;
     st->buf = 0;
+    st->chip_fail = 0;
     st->ncell = (long)T.g.nx * T.g.ny * T.g.nz;
 }
 
@@ -1251,13 +1177,7 @@ __global__ void kb_fin_p(TankSet b)
     tank_totals<1>(T, b, tot);
     if(threadIdx.x == 0)
     {
-        st->r_j = tot[0];
-        st->rr = tot[0];
-        st->norm_r0 = sqrt(tot[0]);
-        st->residual = sqrt(tot[0]) / double(st->ncell);
-        st->iter += 1;
-        if(!((st->residual >= st->stop) && (st->iter < st->maxiter))) st->done = 1;
-        st->mode = 2;
+        restart_store(st, tot[0]);
     }
 }
 
@@ -1507,26 +1427,7 @@ __global__ void kb_fin_v(TankSet b, int rr_state)
             restart_store(st, stot[0]);
             if(st->done) return;
         }
-        const double sigma = tot[0];
-        const double norm_vj = sqrt(tot[1]);
-        const double norm_rj = sqrt(rr_state ? st->rr : tot[2]);
-        const double alpha = st->r_j / sigma;
-        st->sigma = sigma;
-        st->norm_vj = norm_vj;
-        st->norm_rj = norm_rj;
-        st->alpha = alpha;
-        if(st->mixed)
-        {
-            // the fused v phase wrote p and v into the other half and added x32
-            st->buf ^= 1;
-            st->pending = 0;
-        }
-        if(fabs(sigma) <= (1.0e-12 * (norm_vj * st->norm_r0)))
-            st->mode = 1;
-        else if((fabs(alpha) * norm_vj / (norm_rj == 0 ? 1.0e-15 : norm_rj)) <= 0.08)
-            st->mode = 1;
-        else
-            st->mode = 0;
+        v_store(st, tot[0], tot[1], rr_state ? st->rr : tot[2]);
     }
 }
 
@@ -1636,11 +1537,7 @@ __global__ void kb_fin_t(TankSet b)
     if(done || mode == 1 || mode == 3) return;
     if(threadIdx.x == 0)
     {
-        st->w1 = tot[0];
-        st->w2 = tot[1];
-        st->norm_sj = sqrt(tot[2]);
-        st->branch = st->norm_sj > st->stop ? 1 : 0;
-        st->w = st->branch ? tot[0] / (tot[1] == 0 ? 1.0e-15 : tot[1]) : st->w;
+        t_store(st, tot);
     }
 }
 
@@ -1708,34 +1605,10 @@ __global__ void kb_fin_x(TankSet b)
     CTank& T = tank_at(b, blockIdx.x);
     BiState* st = T.st;
     const int done = st->done, mode = st->mode;
-    const double alpha = st->alpha, w = st->w;
-    const int branch = st->branch;
     double tot[2];
     tank_totals<2>(T, b, tot);
     if(done || mode == 1 || mode == 3) return;
-    if(threadIdx.x == 0)
-    {
-        const double r_j1 = tot[0];
-        st->r_j_prev = st->r_j;
-        if(branch) st->beta = alpha * r_j1 / (w * st->r_j == 0 ? 1.0e-15 : (w * st->r_j));
-        st->r_j1 = r_j1;
-        st->r_j = r_j1;
-        st->rr = tot[1];
-        st->residual = sqrt(tot[1]) / double(st->ncell);
-        st->iter += 1;
-        st->mode = 0;
-        if(!st->mixed)
-        {
-            if(!((st->residual >= st->stop) && (st->iter < st->maxiter))) st->done = 1;
-            return;
-        }
-        const double rn = sqrt(tot[1]);
-        if(rn > st->rmax) st->rmax = rn;
-        if(!branch)
-            st->mode = 1;
-        else if(!(st->residual >= st->stop) || st->iter >= st->maxiter || rn < st->delta * st->rmax)
-            st->mode = 3;
-    }
+    if(threadIdx.x == 0) x_store(st, tot);
 }
 
 // ------------------------------------------------------------------ mixed precision

@@ -1,0 +1,68 @@
+"""The on-chip BiCGStab (tanks of up to 2048 tiles) at the edges of its blocks: one tile, ragged
+tiles in every direction, one block and many, one and two tiles per work item, the largest
+tank, and the first size above it, which the streaming phases solve.
+
+The first iterations follow the oracle's, as those of the streaming solver do.  Tolerance:
+the device adds its dot products in another order than the oracle's serial loop, about
+sqrt(N) eps = 1.6e-13 relative for the largest tank, and 12 iterations amplify that by less
+than the 1e-10 that the first 40 iterations on the reference's fixture are held to."""
+import numpy as np
+import pytest
+
+from tests._cases import inner
+from tests.test_gpu_mixed import TOL, _system
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(64, 1, 4, 0), (65, 1, 9, 0), (37, 1, 130, 0), (1150, 1, 157, 0), (2048, 1, 256, 0), (2049, 1, 256, 0),
+          (16, 6, 12, 1), (65, 5, 33, 1), (130, 33, 37, 1), (192, 39, 64, 1)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_first_iterations_follow_the_oracle(shape):
+    nx, ny, nz, jdir = shape
+    O, D, M, b = _system(nx, ny, nz, jdir, seed=77 + nx)
+    print(shape, flush=True)
+    for it in (1, 3, 12):
+        D.zero("work0")
+        n, _ = D.solver("work0", "work1", 1e-300, it)
+        x = np.zeros(O.shape)
+        O.bicgstab(x, M, b.copy(), 1e-300, it)
+        assert n == it
+        got, ref = inner(D.get("work0")), inner(x)
+        np.testing.assert_allclose(got, ref, rtol=0, atol=1e-10 * np.abs(ref).max(), err_msg=f"it={it}")
+
+
+@pytest.mark.parametrize("shape", [(64, 1, 4, 0), (1150, 1, 157, 0), (65, 5, 33, 1), (192, 39, 64, 1)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_solution_and_its_scaling(shape, precision):
+    """The oracle's residual of the solution meets the stop criterion (1.5 times it in FP64,
+    whose iterated residual drifts from the true one), and the right-hand side 2b gives
+    exactly 2x: a power of two changes no rounding, so a lost or stale value breaks it."""
+    nx, ny, nz, jdir = shape
+    O, D, M, b = _system(nx, ny, nz, jdir, seed=5 + nz)
+    solve = D.solver if precision == "fp64" else D.solver_mixed
+    print(shape, precision, flush=True)
+    out = []
+    for scale in (1.0, 2.0):
+        rhs = np.zeros(O.shape)
+        inner(rhs)[...] = scale * b.reshape(nx, ny, nz).transpose(2, 1, 0)
+        D.put("work1", rhs)
+        D.zero("work0")
+        solve("work0", "work1", -TOL, 20000)
+        out.append(D.get("work0"))
+    assert O.residual(out[0], M, b.copy()) <= (1.5 if precision == "fp64" else 1.0) * TOL * np.linalg.norm(b)
+    assert np.array_equal(inner(out[1]), 2.0 * inner(out[0]))
+
+
+def test_iterations_beyond_one_launch():
+    """More iterations than one launch runs (1024): the solve goes on where it stopped, in the
+    same way each time, and stops at the asked count."""
+    _, D, _, _ = _system(65, 5, 33, 1, seed=9)
+    xs = []
+    for _ in range(2):
+        D.zero("work0")
+        n, _ = D.solver("work0", "work1", 0.0, 1500)
+        assert n == 1500
+        xs.append(D.get("work0"))
+    assert np.isfinite(xs[0]).all() and np.array_equal(xs[0], xs[1])
