@@ -11,13 +11,14 @@ enum ChipKind { CHIP_FP64 = 0, CHIP_MIXED = 1, CHIP_MAT = 2 };
 struct ChipSet
 {
     const TankDev* tanks;
-    unsigned long long* halo;      // CHIP_HALO_WORDS: three buffers of CHIP_TILES x 256 cells x 2 words
+    unsigned long long* halo;      // three buffers of halo_words: 256 cells x 2 words per tile slot
+    size_t halo_words;
     unsigned long long* acc;       // CHIP_ACC_WORDS per tank of the launch
     unsigned* ctl;                 // commit word per tank of the launch, 0 before it
     unsigned epoch;                // tag of the launch's first exchange
     int cap;                       // iterations at most
     int hmax;                      // largest halo of a block
-    int d3, slots;                 // 3-D tanks; most tile slots a group uses
+    int d3, ct;                    // 3-D tanks; tile slots per group
     int n;
     int slot[CHIP_TANKS];
     int blk0[CHIP_TANKS + 1];      // first block of each tank

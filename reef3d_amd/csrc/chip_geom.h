@@ -11,54 +11,62 @@
 namespace reef {
 
 constexpr int CHIP_NT = 512;                 // threads per block: two 256-thread groups
-constexpr int CHIP_BLOCKS = 256;             // one block per CU
-constexpr int CHIP_TILES_PER_BLOCK = 8;      // four per group
-constexpr int CHIP_TILES = CHIP_BLOCKS * CHIP_TILES_PER_BLOCK;
-constexpr int CHIP_FIRST = 2;                // tiles per block the plan tries first
+constexpr int CHIP_CUS = 256;                // blocks that run at a time, one per CU
+constexpr int CHIP_BLOCKS = 256;             // blocks of a tank, at most
 constexpr int CHIP_TANKS = 64;               // tanks per launch
-constexpr int CHIP_CPT_MAX = 4;              // tiles per work item
+constexpr int CHIP_TILES = 8192;             // tile slots of all blocks of a launch, at most
 constexpr int CHIP_DIRECT = 64;              // blocks up to which 64 accumulators are added in one hop
 constexpr int CHIP_COPIES = 16;              // places the wave sums of a total are published in
 constexpr int CHIP_COPY_WORDS = 32;          // 4 waves x 3 sums x 2 words, own cache lines
 // per tank two buffers of 256 accumulators x 3 sums x 2 words and the copies
 constexpr int CHIP_ACC_HALF = 3 * 256 * 2 + CHIP_COPIES * CHIP_COPY_WORDS;
 constexpr int CHIP_ACC_WORDS = 2 * CHIP_ACC_HALF;
-constexpr size_t CHIP_HALO_WORDS = (size_t)3 * CHIP_TILES * 256 * 2;
 constexpr int CHIP_LDS_MAX = 152 * 1024;     // dynamic LDS of a block (160 KB less the static arrays)
-constexpr int CHIP_HALO_MAX = 3860;          // halo cells of a block
 constexpr int CHIP_CTL = 4096;               // commit words, used in turn
 // exchanges of a launch are numbered from its epoch; an iteration makes at most five
 constexpr int CHIP_CAP = 1024;               // iterations per launch
 constexpr unsigned CHIP_EPOCHS = 5 * CHIP_CAP + 8;
 
-// operand of the own cells, a zero and the halo (8 bytes each), r, p, v of the halo (sized for
-// FP64) and the exchange index
-constexpr size_t chip_lds_bytes(int hmax) { return (size_t)(CHIP_TILES_PER_BLOCK * 256 + 1 + hmax) * 8 + (size_t)hmax * 28; }
-static_assert(chip_lds_bytes(CHIP_HALO_MAX) <= CHIP_LDS_MAX, "LDS of the on-chip solver");
+// Tile slots per group (ct: 2 or 4; with 8 the FP32 kernel spills and takes 1.2 to 1.9 times
+// as long per iteration, more than it gains in tiles) and the halo cells a thread may keep
+// (sl): both set the registers of a thread, see the kernel's variants.  A 2-D tile has a halo
+// of 136 cells, a 3-D tile of up to 648.
+constexpr int CHIP_CT_MAX = 4;
+constexpr int chip_sl(int d3, int ct) { return d3 ? (ct == 2 ? 6 : 8) : (ct == 2 ? 2 : 3); }
+// dynamic LDS: operand of the own cells, a zero and the halo (8 bytes each, the FP64 residual
+// of the mixed solve uses it too), r, p, v of the halo (vsize bytes each) and its exchange index
+constexpr size_t chip_lds_bytes(int ct, int vsize, int hmax)
+{
+    return (size_t)(2 * ct * 256 + 1 + hmax) * 8 + (size_t)hmax * (3 * vsize + 4);
+}
+// halo cells of a block, at most
+constexpr int chip_halo_max(int d3, int ct, int vsize)
+{
+    const int lds = (int)((CHIP_LDS_MAX - chip_lds_bytes(ct, vsize, 0)) / (8 + 3 * vsize + 4));
+    return lds < chip_sl(d3, ct) * CHIP_NT ? lds : chip_sl(d3, ct) * CHIP_NT;
+}
 
 // ---- geometry of a block, host and device.  Block b of nb keeps the items b, b + nb, ...; its
-// tile slot sl = group * 4 + c holds tile c % cpt of its local item (c / cpt) * 2 + group.
+// tile slot sl = group * ct + c holds tile c % cpt of its local item (c / cpt) * 2 + group.
 // Faces of a tile: 0 +x, 1 -x, 2 +y, 3 -y, 4 +z, 5 -z; a cell of a tile is its thread number.
-constexpr int CHIP_SLOTS = CHIP_TILES_PER_BLOCK / 2;   // tile slots per group
-
 REEF_HD int chip_items(const TileShape& s, int nb, int b) { return (s.nitems - b + nb - 1) / nb; }
 
 // the tile in a slot, -1 empty
-REEF_HD int chip_slot_tile(const TileShape& s, int nb, int b, int sl)
+REEF_HD int chip_slot_tile(const TileShape& s, int ct, int nb, int b, int sl)
 {
-    const int c = sl % CHIP_SLOTS, gr = sl / CHIP_SLOTS, kk = c / s.cpt, li = kk * 2 + gr;
-    if(kk >= CHIP_SLOTS / s.cpt || li >= chip_items(s, nb, b)) return -1;
+    const int c = sl % ct, gr = sl / ct, kk = c / s.cpt, li = kk * 2 + gr;
+    if(kk >= ct / s.cpt || li >= chip_items(s, nb, b)) return -1;
     const int t = (b + li * nb) * s.cpt + (c - kk * s.cpt);
     return t < s.ntiles ? t : -1;
 }
 
 // the slot of a tile in block b, -1 when another block has it
-REEF_HD int chip_tile_slot(const TileShape& s, int nb, int b, int t)
+REEF_HD int chip_tile_slot(const TileShape& s, int ct, int nb, int b, int t)
 {
     const int it = t / s.cpt;
     if(it % nb != b) return -1;
     const int li = it / nb;
-    return (li % 2) * CHIP_SLOTS + (li / 2) * s.cpt + (t - it * s.cpt);
+    return (li % 2) * ct + (li / 2) * s.cpt + (t - it * s.cpt);
 }
 
 // the tile across face f of tile t, -1 at the tank's boundary
@@ -125,7 +133,7 @@ inline int chip_halo(const TileShape& s, int nb)
         for(int f = 0; f < 6; ++f)
         {
             const int nt = chip_face_tile(s, t, f);
-            if(nt >= 0 && chip_tile_slot(s, nb, b, nt) < 0) h[b] += chip_face_size(s, f);
+            if(nt >= 0 && (nt / s.cpt) % nb != b) h[b] += chip_face_size(s, f);
         }
     }
     return *std::max_element(h.begin(), h.end());

@@ -525,7 +525,7 @@ int Engine::sync_tables()
     all_ = make_sets(act);
     cur_ = &all_;
     for(TankHost& t : tanks) t.chip_h.fill(-1);   // plans may have changed
-    all_chip_ = chip_plan(act);
+    for(int m = 0; m < 2; ++m) all_chip_[m] = chip_plan(act, m != 0);
     solving_key_.clear();
     solving_sets_.clear();
     last_state.resize(nslot, BiState{});
@@ -913,99 +913,136 @@ static const char* const MIX_NAMES[4] = {"mix_v", "bicg32_t", "bicg32_x", "mix_r
 static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 
 // ------------------------------------------------------------------ on-chip solves
+// Tile slots per group of the kernel variant for at most per_block tiles per block.
+static int chip_ct(int per_block) { return std::max(2, per_block / 2); }
+
 // Blocks of tank t with at most per_block tiles each: the smallest power of two, at most 256
 // and the tank's items; 0 when the tank does not fit or its sums are taken in another order
 // (a 2-D tank with cpt > 1 walks its rows in the streaming v and t phases).
-int Engine::chip_blocks(TankHost& t, int per_block) const
+int Engine::chip_blocks(TankHost& t, int per_block, bool mixed) const
 {
     const TileShape& s = t.dev.shape;
-    if(s.ntiles > CHIP_TILES || s.cpt > CHIP_CPT_MAX || (t.hg.jdir == 0 && s.cpt > 1)) return 0;
-    // items a block's two groups hold at four tile slots each, within per_block tiles
-    const int most = std::max(1, std::min(2 * (CHIP_TILES_PER_BLOCK / 2 / s.cpt), per_block / s.cpt));
+    const int ct = chip_ct(per_block), d3 = t.hg.jdir;
+    if(s.cpt > ct || (d3 == 0 && s.cpt > 1) || s.ntiles > CHIP_BLOCKS * per_block) return 0;
+    const int most = std::max(1, std::min(2 * (ct / s.cpt), per_block / s.cpt));   // items per block
+    const int hmax = chip_halo_max(d3, ct, mixed ? 4 : 8);
     for(int q = 0, nb = 1; nb <= CHIP_BLOCKS && nb <= s.nitems; ++q, nb *= 2)
     {
         if((s.nitems + nb - 1) / nb > most) continue;
         if(t.chip_h[q] < 0) t.chip_h[q] = chip_halo(s, nb);
-        if(t.chip_h[q] <= CHIP_HALO_MAX) return nb;
+        if(t.chip_h[q] <= hmax) return nb;
     }
     return 0;
 }
 
-// On-chip launches for the slots: a launch holds tanks of at most 256 blocks together.  Two
-// tiles per block where everything then fits one launch (an exchange among fewer blocks is
-// cheaper, but so is less work per thread), else four, else eight and several launches.
-Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots)
+// On-chip launches for the slots.  A launch runs up to 256 blocks at a time, one per CU; of
+// more blocks the later ones start in order as CUs come free.  Few tiles per block keep an
+// iteration short, many keep more tanks on the chip at once.  The launch takes the tiles per
+// block (2, 4 or 8) with the shortest end of all tanks, estimated from the time of an iteration
+// (measured, 2-D tanks: 11, 16 and 17.5 us with 2, 4 and 8 tiles per block, 3-D: 15, 19 and
+// 25 us) and
+// iterations in proportion to the tank's longest side, the longest first.
+Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
 {
     ChipPlan P;
-    auto pack = [&](int per_block) {
-        P.launches.clear();
-        P.rest.clear();
-        for(int q : slots)
-        {
-            TankHost& t = tanks[q];
-            const int nb = chip_off_ ? 0 : chip_blocks(t, per_block);
-            if(nb == 0)
-            {
-                P.rest.push_back(q);
-                continue;
-            }
-            ChipSet* S = nullptr;
-            for(ChipSet& L : P.launches)
-                if(L.d3 == t.hg.jdir && L.n < CHIP_TANKS && L.blk0[L.n] + nb <= CHIP_BLOCKS) S = &L;
-            if(!S)
-            {
-                P.launches.emplace_back();
-                S = &P.launches.back();
-                std::memset(S, 0, sizeof(*S));
-                S->d3 = t.hg.jdir;
-            }
-            S->tanks = d_tanks_;
-            S->slot[S->n] = q;
-            S->tile0[S->n] = S->blk0[S->n] * CHIP_TILES_PER_BLOCK;
-            S->blk0[S->n + 1] = S->blk0[S->n] + nb;
-            S->hmax = std::max(S->hmax, t.chip_h[31 - __builtin_clz((unsigned)nb)]);
-            S->slots = std::max(S->slots, (chip_items(t.dev.shape, nb, 0) + 1) / 2 * t.dev.shape.cpt);
-            S->n += 1;
-        }
-    };
-    pack(CHIP_TILES_PER_BLOCK);
-    const size_t rest = P.rest.size();
-    for(int per_block = CHIP_FIRST; per_block <= CHIP_TILES_PER_BLOCK; per_block *= 2)
+    P.stream_all = true;
+    if(chip_off_) return P;
+    static const double US[2][3] = {{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}};
+    struct Tank
     {
-        pack(per_block);
-        if(P.launches.size() <= 1 && P.rest.size() == rest) break;
+        int slot, side, per[3], nb[3];   // blocks and tiles per block for 2, 4, 8 (or the next that fits)
+    };
+    std::vector<Tank> fit;
+    for(int q : slots_in)
+    {
+        TankHost& t = tanks[q];
+        Tank k;
+        k.slot = q;
+        k.side = std::max(t.hg.nx, std::max(t.hg.ny, t.hg.nz));
+        int nb = 0, per = 2;
+        for(int l = 2; l >= 0; --l)
+        {
+            const int here = chip_blocks(t, 2 << l, mixed);
+            if(here) nb = here, per = l;
+            k.nb[l] = nb;
+            k.per[l] = per;
+        }
+        if(k.nb[2])
+            fit.push_back(k);
+        else
+            P.rest.push_back(q);
     }
-    P.stream_all = P.launches.empty();
-    if(!P.stream_all && !P.rest.empty()) P.rest_sets = make_sets(P.rest);
+    if(fit.empty()) return P;
+    P.stream_all = false;
+    std::stable_sort(fit.begin(), fit.end(), [](const Tank& a, const Tank& b) { return a.side > b.side; });
+    int best = 0;
+    double best_end = 0.0;
+    for(int l = 0; l < 3; ++l)
+    {
+        std::multimap<double, int> running;   // end time, blocks
+        int free_cus = CHIP_CUS;
+        double now = 0.0, end = 0.0;
+        for(const Tank& k : fit)
+        {
+            while(free_cus < k.nb[l])
+            {
+                now = std::max(now, running.begin()->first);
+                free_cus += running.begin()->second;
+                running.erase(running.begin());
+            }
+            const double e = now + k.side * US[tanks[k.slot].hg.jdir][k.per[l]];
+            running.emplace(e, k.nb[l]);
+            free_cus -= k.nb[l];
+            end = std::max(end, e);
+        }
+        if(l == 0 || end < best_end) best = l, best_end = end;
+    }
+    for(const Tank& k : fit)
+    {
+        const TankHost& t = tanks[k.slot];
+        const int nb = k.nb[best], ct = chip_ct(2 << k.per[best]);
+        ChipSet* S = nullptr;
+        for(ChipSet& L : P.launches)
+            if(L.d3 == t.hg.jdir && L.ct == ct && L.n < CHIP_TANKS && (L.blk0[L.n] + nb) * 2 * ct <= CHIP_TILES) S = &L;
+        if(!S)
+        {
+            P.launches.emplace_back();
+            S = &P.launches.back();
+            std::memset(S, 0, sizeof(*S));
+            S->d3 = t.hg.jdir;
+            S->ct = ct;
+        }
+        S->tanks = d_tanks_;
+        S->slot[S->n] = k.slot;
+        S->tile0[S->n] = S->blk0[S->n] * 2 * ct;
+        S->blk0[S->n + 1] = S->blk0[S->n] + nb;
+        S->hmax = std::max(S->hmax, t.chip_h[31 - __builtin_clz((unsigned)nb)]);
+        S->n += 1;
+    }
+    if(!P.rest.empty()) P.rest_sets = make_sets(P.rest);
     return P;
 }
 
-int Engine::chip_alloc()
+// workspace of the on-chip solver for at least `tiles` tile slots
+int Engine::chip_alloc(size_t tiles)
 {
-    if(d_chip_) return 0;
+    if(d_chip_ && tiles <= chip_tiles_) return 0;
     const int rc = chip_prepare();
     if(rc) return fail(rc, "on-chip solver: dynamic LDS limit not accepted");
-    const size_t bytes = (CHIP_HALO_WORDS + (size_t)CHIP_TANKS * CHIP_ACC_WORDS) * 8 + CHIP_CTL * sizeof(unsigned);
-    unsigned long long* d = nullptr;
-    EHIP(hipMalloc(&d, bytes));
-    if(!chip_ev_)
+    if(!chip_ev_) EHIP(hipEventCreateWithFlags(&chip_ev_, hipEventDisableTiming));
+    if(d_chip_)
     {
-        const hipError_t e = hipEventCreateWithFlags(&chip_ev_, hipEventDisableTiming);
-        if(e != hipSuccess)
-        {
-            (void)hipFree(d);
-            return fail(REEF_E_HIP, std::string("hipEventCreateWithFlags: ") + hipGetErrorString(e));
-        }
+        EHIP(hipStreamSynchronize(stream));
+        (void)hipFree(d_chip_);
+        d_chip_ = nullptr;
     }
-    const hipError_t e = hipMemsetAsync(d, 0, bytes, stream);
-    if(e != hipSuccess)
-    {
-        (void)hipFree(d);
-        return fail(REEF_E_HIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
-    }
-    d_chip_ = d;
+    tiles = std::max(tiles, (size_t)2048);
+    const size_t bytes = ((size_t)CHIP_TANKS * CHIP_ACC_WORDS + 3 * tiles * 512) * 8 + CHIP_CTL * sizeof(unsigned);
+    EHIP(hipMalloc(&d_chip_, bytes));
+    chip_tiles_ = tiles;
     chip_epoch_ = 1;
     chip_ctl_ = 0;
+    EHIP(hipMemsetAsync(d_chip_, 0, bytes, stream));
     return 0;
 }
 
@@ -1013,9 +1050,11 @@ int Engine::chip_alloc()
 int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
 {
     int rc;
-    if((rc = chip_alloc())) return rc;
-    unsigned long long* acc = d_chip_ + CHIP_HALO_WORDS;
-    unsigned* ctl = (unsigned*)(acc + (size_t)CHIP_TANKS * CHIP_ACC_WORDS);
+    size_t tiles = 0;
+    for(const ChipSet& S : P.launches) tiles = std::max(tiles, (size_t)S.blk0[S.n] * 2 * S.ct);
+    if((rc = chip_alloc(tiles))) return rc;
+    unsigned* ctl = (unsigned*)(d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS);
+    unsigned long long* halo = d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS + CHIP_CTL / 2;
     int dev = 0;
     EHIP(hipGetDevice(&dev));
     std::lock_guard<std::mutex> lk(g_chip_mu);
@@ -1027,13 +1066,18 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
         if(chip_epoch_ > 0xffffffffu - 2 * CHIP_EPOCHS || chip_ctl_ + S.n > CHIP_CTL)
         {
             const bool tags = chip_epoch_ > 0xffffffffu - 2 * CHIP_EPOCHS;
-            if(tags) EHIP(hipMemsetAsync(d_chip_, 0, (CHIP_HALO_WORDS + (size_t)CHIP_TANKS * CHIP_ACC_WORDS) * 8, stream));
             EHIP(hipMemsetAsync(ctl, 0, CHIP_CTL * sizeof(unsigned), stream));
-            if(tags) chip_epoch_ = 1;
             chip_ctl_ = 0;
+            if(tags)
+            {
+                EHIP(hipMemsetAsync(d_chip_, 0, (size_t)CHIP_TANKS * CHIP_ACC_WORDS * 8, stream));
+                EHIP(hipMemsetAsync(halo, 0, 3 * chip_tiles_ * 512 * 8, stream));
+                chip_epoch_ = 1;
+            }
         }
-        S.halo = d_chip_;
-        S.acc = acc;
+        S.halo = halo;
+        S.halo_words = chip_tiles_ * 512;
+        S.acc = d_chip_;
         S.ctl = ctl + chip_ctl_;
         S.epoch = chip_epoch_;
         S.cap = cap;
@@ -1055,7 +1099,8 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
 // after a tank's end are no-ops for it.
 int Engine::enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap)
 {
-    ChipPlan* P = cur_ == &all_ ? &all_chip_ : cur_ == &solving_sets_ ? &solving_chip_ : nullptr;
+    const int m = kind == SOLVE_MIXED;
+    ChipPlan* P = cur_ == &all_ ? &all_chip_[m] : cur_ == &solving_sets_ ? &solving_chip_[m] : nullptr;
     if(P && !chip_off_ && !P->stream_all)
     {
         int rc = chip_launch(*P, kind, x, rhs, chip_cap);
@@ -1154,7 +1199,8 @@ int Engine::run_iterations(int kind, int x, int rhs, int maxiter)
         for(int p = 0; p < S.n; ++p) members.push_back(S.slot[p]);
     int rc;
     // an on-chip batch usually is the whole solve: nothing is enqueued behind it
-    auto ahead = [&] { return chip_off_ || cur_ != &all_ || all_chip_.stream_all || !all_chip_.rest.empty(); };
+    const ChipPlan& P = all_chip_[kind == SOLVE_MIXED];
+    auto ahead = [&] { return chip_off_ || cur_ != &all_ || P.stream_all || !P.rest.empty(); };
     if((rc = enqueue_batch(kind, x, rhs, 0, 8))) return rc;
     bool queued = false;   // batch k is behind batch k - 1
     for(long k = 1;; ++k)
@@ -1783,7 +1829,7 @@ int Engine::pump(std::vector<int>& stepped)
         if(solving != solving_key_)
         {
             solving_sets_ = make_sets(solving);
-            solving_chip_ = chip_plan(solving);
+            solving_chip_[mixed] = chip_plan(solving, mixed);
             solving_key_ = solving;
         }
         const int ring = (int)(batch_no_++ & 1);

@@ -311,15 +311,17 @@ private:
         std::vector<TankSet> rest_sets;
         bool stream_all = false;            // every slot streams: the caller's sets are used
     };
-    ChipPlan all_chip_, solving_chip_;
-    unsigned long long* d_chip_ = nullptr;  // halo words, then accumulator words, then commit words
+    ChipPlan all_chip_[2], solving_chip_[2];   // [1]: mixed precision (FP32 vectors)
+    size_t chip_tiles_ = 0;                 // tile slots the workspace holds
+    // accumulator words, commit words, then the halo words of chip_tiles_ tile slots
+    unsigned long long* d_chip_ = nullptr;
     unsigned chip_epoch_ = 0;
     int chip_ctl_ = 0;                      // next unused commit word
     bool chip_off_ = false;                 // a launch gave up waiting: another process shares the GPU
     hipEvent_t chip_ev_ = nullptr;
-    int chip_blocks(TankHost& t, int per_block) const;
-    ChipPlan chip_plan(const std::vector<int>& slots);
-    int chip_alloc();
+    int chip_blocks(TankHost& t, int per_block, bool mixed) const;
+    ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);
+    int chip_alloc(size_t tiles);
     int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);
     int enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap);
     int stream_iterations(int kind, int x, int rhs, int iters, bool lockstep);

@@ -33,9 +33,7 @@ namespace bk {
 typedef unsigned long long u64;
 
 constexpr int CG = CHIP_NT / NT;           // 256-thread groups
-constexpr int CS = CHIP_TILES_PER_BLOCK;   // tile slots per block
-constexpr int CQ = CHIP_SLOTS;             // tile slots per group
-static_assert(CG == 2 && CG * CQ == CS, "tile slots of a block");
+static_assert(CG == 2, "groups of a block");
 constexpr unsigned ABORT = 0x80000000u;
 constexpr long WAIT_TICKS = 5000000;   // 50 ms of the 100 MHz wall clock
 
@@ -171,10 +169,11 @@ __device__ __forceinline__ double wave_sum(double v)
 template<class V, int KIND, bool d3, int CT, int SL>
 __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
 {
+    constexpr int CS = CG * CT;           // tile slots per group and block
     constexpr bool MIXED = KIND == CHIP_MIXED, MAT = KIND == CHIP_MAT;
     extern __shared__ __align__(16) char lds[];
     __shared__ BiState st;
-    __shared__ double ws[CG][NT / 64][CQ][3];      // wave sums per item
+    __shared__ double ws[CG][NT / 64][CT][3];      // wave sums per item
     __shared__ double wt[3][NT / 64];              // its wave sums
     __shared__ double acc1[NT][3];                 // the accumulators of a one-block tank
     __shared__ int fnb[CS][6], foff[CS][6], ftile[CS][6], stile[CS];
@@ -190,8 +189,8 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
     const int cpt = sh.cpt, nitems = sh.nitems;
     const int tid = threadIdx.x, grp = tid >> 8, ct = tid & (NT - 1), wave = ct >> 6, lane = ct & 63;
     u64* const halo0 = S.halo;
-    u64* const halo1 = S.halo + (size_t)CHIP_TILES * NT * 2;
-    u64* const halo2 = S.halo + (size_t)CHIP_TILES * NT * 4;
+    u64* const halo1 = S.halo + S.halo_words;
+    u64* const halo2 = S.halo + 2 * S.halo_words;
     u64* const accw = S.acc + (size_t)p * CHIP_ACC_WORDS;
     unsigned* const ctl = S.ctl + p;
     const int xt0 = S.tile0[p];
@@ -209,7 +208,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
         st = *T.st;
         dead = 0;
     }
-    if(tid < CS) stile[tid] = chip_slot_tile(sh, NB, b, tid);
+    if(tid < CS) stile[tid] = chip_slot_tile(sh, CT, NB, b, tid);
     __syncthreads();
     if(st.done) return;
     // the neighbour tile of each face (+x, -x, +y, -y, +z, -z): in this block (its slot), in
@@ -220,7 +219,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
         int nb = -1, nt = -1;
         if(tl >= 0 && (nt = chip_face_tile(sh, tl, f)) >= 0)
         {
-            nb = chip_tile_slot(sh, NB, b, nt);
+            nb = chip_tile_slot(sh, CT, NB, b, nt);
             if(nb < 0) nb = -2;
         }
         fnb[sl][f] = nb;
@@ -308,7 +307,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
         cidx[c] = 0;
         if constexpr(MIXED) x64[c] = 0.0;
         if(c >= nc) continue;
-        const int sl = grp * CQ + c, tl = stile[sl];
+        const int sl = grp * CT + c, tl = stile[sl];
         if(tl < 0) continue;
         int i, j, k;
         if(!cell_of(tl, ct, i, j, k)) continue;
@@ -409,7 +408,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             if(c < nc && pub[c] && act[c])
             {
                 auto w = val(c);
-                Wire<decltype(w)>::put(buf + ((size_t)(xt0 + stile[grp * CQ + c]) * NT + ct) * 2, w, tg);
+                Wire<decltype(w)>::put(buf + ((size_t)(xt0 + stile[grp * CT + c]) * NT + ct) * 2, w, tg);
             }
     };
     // receives the neighbours' values of this thread's halo cells: got(s, q, value)
@@ -487,7 +486,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             double s = 0.0;
             for(int li = q; li < nloc; li += naccs)
             {
-                const double(*w4)[CQ][3] = ws[li % CG];
+                const double(*w4)[CT][3] = ws[li % CG];
                 const int kk = li / CG;
                 s += ((w4[0][kk][m] + w4[1][kk][m]) + w4[2][kk][m]) + w4[3][kk][m];
             }
@@ -589,7 +588,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
     auto no_send = [](unsigned) {};
     auto stencil = [&](int c, const auto* o, const auto& m) {
         using W = std::remove_cv_t<std::remove_reference_t<decltype(o[0])>>;
-        const int sl = grp * CQ + c;
+        const int sl = grp * CT + c;
         const W yw = d3 ? o[nx23[c] & 0xffffu] : W(0), ye = d3 ? o[nx23[c] >> 16] : W(0);
         return coef_apply<W>(m, d3, o[sl * NT + ct], o[nx01[c] & 0xffffu], o[nx01[c] >> 16], yw, ye, o[nx45[c] & 0xffffu],
                              o[nx45[c] >> 16]);
@@ -607,7 +606,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             publish(halo1, [&](int c) { return x[c]; }, tg);
             #pragma unroll
             for(int c = 0; c < CT; ++c)
-                if(c < nc) op[(grp * CQ + c) * NT + ct] = x[c];
+                if(c < nc) op[(grp * CT + c) * NT + ct] = x[c];
             receive(halo1, tg, V(0), [&](int, int q, V val) { op[HALO + q] = val; });
             #pragma unroll
             for(int s = 0; s < SL; ++s)
@@ -671,7 +670,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             }
         #pragma unroll
         for(int c = 0; c < CT; ++c)
-            if(c < nc) op[(grp * CQ + c) * NT + ct] = pv[c] * a[c];
+            if(c < nc) op[(grp * CT + c) * NT + ct] = pv[c] * a[c];
         #pragma unroll
         for(int s = 0; s < SL; ++s)
         {
@@ -710,7 +709,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             const V alpha = (V)st.alpha;
             #pragma unroll
             for(int c = 0; c < CT; ++c)
-                if(c < nc) op[(grp * CQ + c) * NT + ct] = (r[c] - alpha * v[c]) * a[c];
+                if(c < nc) op[(grp * CT + c) * NT + ct] = (r[c] - alpha * v[c]) * a[c];
             #pragma unroll
             for(int s = 0; s < SL; ++s)
             {
@@ -795,7 +794,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
                 publish(halo1, [&](int c) { return x64[c] + (double)x[c]; }, tg);
                 #pragma unroll
                 for(int c = 0; c < CT; ++c)
-                    if(c < nc) op64[(grp * CQ + c) * NT + ct] = x64[c] + (double)x[c];
+                    if(c < nc) op64[(grp * CT + c) * NT + ct] = x64[c] + (double)x[c];
                 if(tid == 0) op64[ZERO] = 0.0;
                 receive(halo1, tg, 0.0, [&](int, int q, double val) { op64[HALO + q] = val; });
                 #pragma unroll
@@ -817,7 +816,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
                     rv[c] = r0v[c] = 0.0;
                     if(c >= nc || !act[c]) continue;
                     int i, j, k;
-                    cell_of(stile[grp * CQ + c], ct, i, j, k);
+                    cell_of(stile[grp * CT + c], ct, i, j, k);
                     const Coef<double> m =
                         poisson_coef(g, couplings(g, T.f[A_RFX], T.f[A_RFY], T.f[A_RFZ], (long)cidx[c], i, j, k), i, j, k);
                     rv[c] = b64[cidx[c]] - stencil(c, op64, m);
@@ -904,20 +903,18 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
 
 }  // namespace bk
 
-// The variants of the kernel: registers for two or four tile slots per group, and for the
-// halo cells that go with them (2-D: 136 a tile; 3-D: up to 648)
+// the variant of the kernel for a launch (chip_geom.h: ct tile slots, chip_sl halo cells)
 template<class F>
-static void chip_variant(int kind, bool d3, int slots, int hmax, F f)
+static void chip_variant(int kind, bool d3, int ct, F f)
 {
     auto pick = [&](auto V_, auto K_) {
         using V = decltype(V_);
         constexpr int K = decltype(K_)::value;
-        if(!d3)
-            slots <= 2 ? f(bk::kc_solve<V, K, false, 2, 2>) : f(bk::kc_solve<V, K, false, 4, 3>);
+        if(ct == 2)
+            d3 ? f(bk::kc_solve<V, K, true, 2, chip_sl(1, 2)>) : f(bk::kc_solve<V, K, false, 2, chip_sl(0, 2)>);
         else
-            slots <= 2 && hmax <= 6 * CHIP_NT ? f(bk::kc_solve<V, K, true, 2, 6>) : f(bk::kc_solve<V, K, true, 4, 8>);
+            d3 ? f(bk::kc_solve<V, K, true, 4, chip_sl(1, 4)>) : f(bk::kc_solve<V, K, false, 4, chip_sl(0, 4)>);
     };
-    static_assert(8 * CHIP_NT >= CHIP_HALO_MAX && 2 * CHIP_NT >= 4 * 136 && 3 * CHIP_NT >= 8 * 136, "halo cells");
     if(kind == CHIP_FP64)
         pick(0.0, std::integral_constant<int, CHIP_FP64>());
     else if(kind == CHIP_MAT)
@@ -931,8 +928,8 @@ int chip_prepare()
     int bad = 0;
     for(int kind : {CHIP_FP64, CHIP_MIXED, CHIP_MAT})
         for(int d3 = 0; d3 < 2; ++d3)
-            for(int slots : {2, 4})
-                chip_variant(kind, d3 != 0, slots, 0, [&](auto k) {
+            for(int ct = 2; ct <= CHIP_CT_MAX; ct *= 2)
+                chip_variant(kind, d3 != 0, ct, [&](auto k) {
                     bad |= hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, CHIP_LDS_MAX) !=
                            hipSuccess;
                 });
@@ -941,8 +938,9 @@ int chip_prepare()
 
 void bl_chip_solve(const ChipSet& S, int kind, int x, int rhs, hipStream_t s)
 {
-    chip_variant(kind, S.d3 != 0, S.slots, S.hmax, [&](auto k) {
-        hipLaunchKernelGGL(k, dim3((unsigned)S.blk0[S.n]), dim3(CHIP_NT), chip_lds_bytes(S.hmax), s, S, x, rhs);
+    const size_t lds = chip_lds_bytes(S.ct, kind == CHIP_MIXED ? 4 : 8, S.hmax);
+    chip_variant(kind, S.d3 != 0, S.ct, [&](auto k) {
+        hipLaunchKernelGGL(k, dim3((unsigned)S.blk0[S.n]), dim3(CHIP_NT), lds, s, S, x, rhs);
     });
 }
 
