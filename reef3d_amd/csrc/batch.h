@@ -30,6 +30,13 @@ constexpr int NPROG = 13;
 constexpr int PROG_KIND_GCV[NPROG][2] = {{4, 52}, {4, 1}, {4, 40}, {1, 10}, {2, 11}, {3, 12}, {1, 7},
                                          {2, 8},  {3, 9}, {2, 12}, {4, 50}, {1, 14}, {3, 16}};
 
+enum RowClass
+{
+    ROW_MIXED = 0,
+    ROW_WATER = 1,
+    ROW_AIR = 2
+};
+
 struct TankDev
 {
     DevGrid g;                     // geometry and metadata (base relative to each array)
@@ -43,6 +50,14 @@ struct TankDev
     const GhostOp* gops[NPROG];    // compiled ghost programs
     int gnops[NPROG];
     BiState* st;                   // solver state (FP64 or mixed)
+    // density class of each 64-cell row (bx, j, k), at (bx ny + j) nz + k: ROW_WATER / ROW_AIR
+    // when the six faces of all its cells have that density, else ROW_MIXED (kb_aii, kb_coef32)
+    unsigned char* cls;
+    // couplings of the two row classes along each axis: entries 2 ((class - 1) n + index) and the
+    // next are those across the + and the - face, 1 / (rho DP DN) in FP64, the FP32 conductance
+    // times the FP32 1/DN in ct32
+    const double* ct[3];
+    const float* ct32[3];
     double* vol;                   // volume1, volume2 of the last fluid update
     // explicit 7-diagonal operator of the matrix solve (solver::start with the caller's
     // a->M) in field layout: M.p, M.n, M.s, M.w, M.e, M.t, M.b, the right-hand side, and the
@@ -64,6 +79,7 @@ struct TankSet
     double* partials;              // reduction partials: [TankDev::item0 + item] * 4
     double* partials_ru;           // partials of the mixed solve's reliable-update phase:
                                    // [TankDev::item0 + item] * 2, read by the next v phase
+    double rw, ra;                 // W1, W3: the densities of the row classes
     int n;                         // tanks in the set
     int ntiles, nitems;            // tiles and work items of the set
     int has_pw, has_direct;        // tanks walked by the 3-D plane walk / by the direct stencil

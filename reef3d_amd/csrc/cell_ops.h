@@ -404,29 +404,6 @@ __device__ __forceinline__ V diag_of(const DevGrid& g, const CouplingV<V>& q)
 // neighbours (pressure-correction ghosts are 0) drop out, the diagonal keeps them.
 // Summation order of matvec_std (bicgstab_ijk.cpp:296-310); 5 points in 2-D
 // (bicgstab_ijk_2D.cpp:308-320).  xv(cc) gives the value of x at element cc.
-// the same sum from the seven values (xn/xs: i+-1, xw/xe: j+-1, xt/xb: k+-1), values
-// outside the domain are ignored
-template<class V>
-__device__ __forceinline__ V stencil7(const DevGrid& g, const CouplingV<V>& q, V xc, V xn_, V xs_, V xw_, V xe_, V xt_,
-                                      V xb_, int i, int j, int k)
-{
-    const V Mp = diag_of(g, q);
-    const V Mn = i == g.nx - 1 ? V(0) : -q.T[0];
-    const V Ms = i == 0 ? V(0) : -q.T[1];
-    const V Mt = k == g.nz - 1 ? V(0) : -q.T[4];
-    const V Mb = k == 0 ? V(0) : -q.T[5];
-    const V xn = i == g.nx - 1 ? V(0) : xn_;
-    const V xs = i == 0 ? V(0) : xs_;
-    const V xt = k == g.nz - 1 ? V(0) : xt_;
-    const V xb = k == 0 ? V(0) : xb_;
-    const V yd = (V)g.ydir;
-    const V Mw = j == g.ny - 1 ? V(0) : -q.T[2] * yd;
-    const V Me = j == 0 ? V(0) : -q.T[3] * yd;
-    const V xw = j == g.ny - 1 ? V(0) : xw_;
-    const V xe = j == 0 ? V(0) : xe_;
-    return Mp * xc + Mn * xn + Ms * xs + Mw * xw + Me * xe + Mt * xt + Mb * xb;
-}
-
 // the 2-D (x-z) operator of apply_A_fn from the five values (xn/xs: i+-1, xt/xb: k+-1)
 template<class V>
 __device__ __forceinline__ V stencil5(const DevGrid& g, const CouplingV<V>& q, V xc, V xn_, V xs_, V xt_, V xb_, int i,
@@ -442,6 +419,38 @@ __device__ __forceinline__ V stencil5(const DevGrid& g, const CouplingV<V>& q, V
     const V xt = k == g.nz - 1 ? V(0) : xt_;
     const V xb = k == 0 ? V(0) : xb_;
     return Mp * xc + Mn * xn + Ms * xs + Mt * xt + Mb * xb;
+}
+
+// (A y)(c) from the seven coefficients of the cell, in matvec_std's order (the sums of
+// apply_A_fn, stencil5 and mat_apply); neighbours outside the domain have coefficient 0 and
+// the caller gives 0 for them
+template<class V>
+struct Coef
+{
+    V p, n, s, w, e, t, b;
+};
+
+template<class V>
+__device__ __forceinline__ V coef_apply(const Coef<V>& m, bool d3, V yc, V yn, V ys, V yw, V ye, V yt, V yb)
+{
+    if(d3) return m.p * yc + m.n * yn + m.s * ys + m.w * yw + m.e * ye + m.t * yt + m.b * yb;
+    return m.p * yc + m.n * yn + m.s * ys + m.t * yt + m.b * yb;
+}
+
+// the coefficients apply_A_fn forms from the couplings of cell (i, j, k)
+template<class V>
+__device__ __forceinline__ Coef<V> poisson_coef(const DevGrid& g, const CouplingV<V>& q, int i, int j, int k)
+{
+    Coef<V> m;
+    m.p = diag_of(g, q);
+    m.n = i == g.nx - 1 ? V(0) : -q.T[0];
+    m.s = i == 0 ? V(0) : -q.T[1];
+    m.t = k == g.nz - 1 ? V(0) : -q.T[4];
+    m.b = k == 0 ? V(0) : -q.T[5];
+    const V yd = (V)g.ydir;
+    m.w = j == g.ny - 1 ? V(0) : -q.T[2] * yd;
+    m.e = j == 0 ? V(0) : -q.T[3] * yd;
+    return m;
 }
 
 template<class V, class XV>

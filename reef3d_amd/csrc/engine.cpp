@@ -188,6 +188,8 @@ Engine::~Engine()
 // device bytes add_built takes for a build: the pool blocks of the FP64 and FP32 arrays,
 // the metadata block (tables, FP32 1/DN, ghost programs), the solver state and the
 // time-step block, each rounded to the pool's granule
+static size_t class_bytes(const HostGrid& h) { return (size_t)((h.nx + TILE_X - 1) / TILE_X) * h.ny * h.nz; }
+
 static size_t meta_block_bytes(const TankBuild& b)
 {
     return up(b.meta.size() * 8) + up(b.inv.size() * 4) + b.ops.size() * sizeof(GhostOp);
@@ -197,7 +199,7 @@ size_t Engine::built_bytes(const TankBuild& b)
 {
     const size_t n = (size_t)b.hg.nalloc;
     return (size_t)NARR64 * up(n * 8) + (size_t)NARR32 * up(n * 4) + up(meta_block_bytes(b)) + up(sizeof(BiState)) +
-           up(8 * sizeof(double));
+           up(8 * sizeof(double)) + up(class_bytes(b.hg));
 }
 
 size_t Engine::tank_bytes(const reef_grid_desc& gd)
@@ -270,6 +272,25 @@ int Engine::build_tank(const reef_grid_desc& gd, const reef_params& p, TankBuild
     {
         b.offinv[a] = b.inv.size();
         for(double d : h.DN[a]) b.inv.push_back(d != 0.0 ? (float)(1.0 / d) : 0.0f);
+    }
+    // couplings of rows of one density (W1 water, W3 air) with the operations of couplings() and
+    // of kb_coef32 / coupling_of
+    for(int a = 0; a < 3; ++a)
+    {
+        const int n = a == 0 ? h.nx : a == 1 ? h.ny : h.nz;
+        b.offct[a] = b.meta.size();
+        b.offct32[a] = b.inv.size();
+        for(int cl = 0; cl < 2; ++cl)
+        {
+            const double rho = cl == 0 ? p.W1 : p.W3;
+            for(int q = 0; q < n; ++q)
+                for(int side = 0; side < 2; ++side)
+                {
+                    const double DP = h.DP[a][q + MARGE - side], DN = h.DN[a][q + MARGE];
+                    b.meta.push_back((1.0 * 1.0) / (rho * DP * DN));
+                    b.inv.push_back((float)(1.0 / (rho * DP)) * b.inv[b.offinv[a] + (size_t)(q + MARGE)]);
+                }
+        }
     }
     return 0;
 }
@@ -351,6 +372,9 @@ int Engine::add_built(TankBuild& b, int* id)
     if((rc = take(sizeof(BiState), &stb))) return release(), rc;
     EHIP(hipMemsetAsync(stb, 0, sizeof(BiState), stream));
     D.st = (BiState*)stb;
+    void* clb;
+    if((rc = take(class_bytes(h), &clb))) return release(), rc;
+    D.cls = (unsigned char*)clb;
     // the time-step block: dt, the velocity maxima of the last time-step pass, and the
     // smallest cell width MIN over the cells of MIN3(DXN, DYN, DZN) (ietimestep.cpp:180-184)
     void* tsb;
@@ -389,6 +413,11 @@ int Engine::add_built(TankBuild& b, int* id)
     D.iDXN32 = invd + b.offinv[0];
     D.iDYN32 = invd + b.offinv[1];
     D.iDZN32 = invd + b.offinv[2];
+    for(int a = 0; a < 3; ++a)
+    {
+        D.ct[a] = md + b.offct[a];
+        D.ct32[a] = invd + b.offct32[a];
+    }
     for(int q = 0; q < NPROG; ++q)
     {
         D.gops[q] = opd + b.op0[q];
@@ -554,6 +583,8 @@ std::vector<TankSet> Engine::make_sets(const std::vector<int>& slots_in) const
         S.tanks = d_tanks_;
         S.partials = d_partials_;
         S.partials_ru = d_partials_ + cap_partials_ / 2;
+        S.rw = shared() ? shared()->W1 : 1000.0;
+        S.ra = shared() ? shared()->W3 : 1.205;
         const size_t b = std::min(slots.size(), a + (size_t)SET_MAX);
         int nt = 0, ni = 0;
         for(size_t q = a; q < b; ++q)

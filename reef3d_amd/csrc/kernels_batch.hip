@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 namespace reef {
 namespace bk {
@@ -124,6 +125,18 @@ struct TileWalk
 __device__ __forceinline__ TileWalk item_walk(CTank& T, const TankSet& b, const ItemIter& q)
 {
     const int li = item_at(T.shape, q.q - b.item0[q.p]);
+    TileWalk w;
+    w.s = T.shape;
+    w.t = li * T.shape.cpt;
+    w.t1 = min(w.t + T.shape.cpt, T.shape.ntiles);
+    w.gi = T.item0 + li;
+    return w;
+}
+
+// the same in item_spread order (the class phases)
+__device__ __forceinline__ TileWalk class_item(CTank& T, const TankSet& b, const ItemIter& q)
+{
+    const int li = item_spread(T.shape, q.q - b.item0[q.p]);
     TileWalk w;
     w.s = T.shape;
     w.t = li * T.shape.cpt;
@@ -562,6 +575,17 @@ __global__ void __launch_bounds__(NT) kb_poisson_rhs(TankSet b, int u_, int v_, 
     }
 }
 
+// the class of the wavefront's row of a tile (TankDev::cls): a wavefront holds one row of
+// every tile shape, so j and k are its own; cells outside the grid count as any class
+__device__ __forceinline__ void store_row_class(CTank& T, const TankSet& b, const DevGrid& g, bool in, double f0, double f1,
+                                                double f2, double f3, double f4, double f5, int i, int j, int k)
+{
+    auto all_are = [&](double r) { return f0 == r && f1 == r && f2 == r && f3 == r && f4 == r && f5 == r; };
+    const bool water = __all(!in || all_are(b.rw)), air = __all(!in || all_are(b.ra));
+    if(in && (threadIdx.x & 63) == 0)
+        T.cls[((long)(i / TILE_X) * g.ny + j) * g.nz + k] = water ? ROW_WATER : air ? ROW_AIR : ROW_MIXED;
+}
+
 // face densities of the "+" faces of the interior and of the -1 layer, optionally the
 // Jacobi diagonal aii = -1/(M.p + 1e-19) (needs all faces: second pass)
 __global__ void __launch_bounds__(NT) kb_face_rho(TankSet b, double rw, double ra)
@@ -609,7 +633,11 @@ __global__ void __launch_bounds__(NT) kb_aii(TankSet b)
         {
             int i, j, k;
             long c;
-            if(!tile_cell(g, tw, t, i, j, k, c)) continue;
+            // every lane of the wavefront takes part in its row's class
+            const bool in = tile_cell(g, tw, t, i, j, k, c);
+            if(!in) c = g.base;
+            store_row_class(T, b, g, in, rfx[c], rfx[c - 1], rfy[c], rfy[c - g.sx], rfz[c], rfz[c - g.sxy], i, j, k);
+            if(!in) continue;
             const Coupling cq = couplings(g, rfx, rfy, rfz, c, i, j, k);
             aii[c] = -1.0 / (diag_of(g, cq) + 1e-19);
         }
@@ -643,39 +671,13 @@ __global__ void __launch_bounds__(NT) kb_correct(TankSet b, double rw, double ra
 // plane walk and the FP32 / elementwise kernels; 5 for the kernels that apply the FP64
 // operator cell by cell (about 100 registers), whose grids are sized to match.
 constexpr int OCC_FULL = 8, OCC_A64 = 5;
-// plane walk: 4 blocks per CU for 4-byte operands (two planes of loads in flight per
-// block); the default plan of a 3-D tank gives it one work item per block.  8-byte operands
-// keep PW64_DEPTH planes of loads in flight at OCC_PW64 blocks per CU: the FP64 walk is
-// bound by the latency of its loads, and a deeper prefetch at a lower occupancy keeps more
-// bytes in flight per CU than one plane at four blocks per CU
-#ifndef REEF_PW64_DEPTH
-#define REEF_PW64_DEPTH 1
-#endif
-#ifndef REEF_OCC_PW64
-#define REEF_OCC_PW64 4
-#endif
-constexpr int OCC_PW = REEF_OCC_PW;
-constexpr int PW64_DEPTH = REEF_PW64_DEPTH;
-constexpr int OCC_PW64 = REEF_OCC_PW64;
-template<class V>
-constexpr int occ_pw() { return sizeof(V) == 4 ? OCC_PW : OCC_PW64; }
+// class walk: 4 blocks per CU (the default plan of a 3-D tank gives it one work item per
+// block)
+constexpr int OCC_PW = REEF_OCC_PW, OCC_CX = REEF_OCC_PW;
 
 // The state machine of bicgstab_ijk::solve (bicgstab_ijk.cpp:125-278) per tank: mode 1 = a
 // restart is pending, 2 = p and ph were just set from the residual, 3 = reliable update
 // pending (mixed precision).  Dot products are accumulated in FP64 for both precisions.
-
-// plane walk of the 3-D stencil kernels (tanks with 64 x 4 x 1 tiles): a block walks up
-// the k planes of its item's column; the stencil input of plane k (rows j-1 .. j+4,
-// columns i-1 .. i+64) and the +x / +y faces sit in LDS, planes k-1, k+1 of the own cell
-// and the -z face stay in registers, so every array crosses HBM about once per cell.
-// The LDS planes are double buffered: one barrier per plane.
-template<class V>
-struct PlaneLDS
-{
-    V x[TY + 2][TX + 2];
-    V fx[TY][TX + 1];
-    V fy[TY + 1][TX];
-};
 
 // element e of an array through a 32-bit byte offset from its (uniform) base, so the load
 // takes the scalar-base + 32-bit vector-offset form (a tank's arrays are below 4 GiB)
@@ -690,267 +692,408 @@ __device__ __forceinline__ void st32(T* __restrict__ p, unsigned e, T v)
     *(T*)((char*)p + e * (unsigned)sizeof(T)) = v;
 }
 
-// Loads of one plane of the walk, issued one plane ahead: the operand's raw inputs at one
-// halo cell of the block and at the cell above (k + 1), the faces, and the epilogue's
-// inputs.  Halo cells are spread over the threads: thread h < 64 loads the south row
-// (j0-1, i0+h), 64 <= h < 128 the north row (j0+TY, i0+h-64), 128 <= h < 132 the west
-// column (j0+h-128, i0-1), 132 <= h < 136 the east column (j0+h-132, i0+TX); the halo
-// faces: thread h < 64 the -y face of column i0+h, 128 <= h < 132 the -x face of row
-// j0+h-128.
-template<class V, class R, class E, class AF>
-struct PlaneIn
-{
-    R h, xu;
-    V f0, f2, f4, fh;
-    AF az;
-    E e;
-};
-
 struct NoEpi
 {
 };
 
-// raw(cc) -> R: the loads of the stencil operand at cc; val(R, V& aux) -> V: the operand
+// ------------------------------------------------------------------ class walk (3-D tanks)
+// Plane walk of the 3-D stencil phases (tanks with 64 x 4 x 1 tiles): a block walks up the k
+// planes of its item's column; the operand of plane k (rows j-1 .. j+4, columns i-1 .. i+64)
+// sits in a double-buffered LDS plane (one barrier per plane), planes k-1 and k+1 of the own
+// cell in registers.
+//
+// The operator comes from the density class of each 64-cell row (TankDev::cls): away from the
+// interface band every face of a row has the density of water or of air exactly, so the six
+// couplings of its cells are functions of one axis each: two table entries per axis, index and
+// class (TankDev::ct, formed with the assembly's operations, so they are the same bits).  x and
+// y entries stay in registers along a column, the z entries load through the scalar unit, and
+// the Jacobi factor is one division of their sum.  Only rows of mixed class read the three
+// face arrays and aii and form the couplings with six divisions.
+// What bounds it: HBM bytes.  On the 512x64x128 wave tank 91 % of the rows have one class and
+// read neither faces nor aii.
+
+// table entries through the constant address space (scalar loads at a uniform index)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(4))) const double CDouble;
+typedef __attribute__((address_space(4))) const float CFloat;
+#else
+typedef const double CDouble;
+typedef const float CFloat;
+#endif
+
+// the couplings of a row class along one axis at index ix
+template<class V>
+struct Pair
+{
+    V p, m;
+};
+__device__ __forceinline__ Pair<double> class_pair64(CTank& T, int axis, int n, int c, int ix)
+{
+    const double* t = T.ct[axis] + 2 * ((c - 1) * n + ix);
+    return {t[0], t[1]};
+}
+template<class V>
+__device__ __forceinline__ Pair<V> class_pair(CTank& T, int axis, int n, int c, int ix)
+{
+    const int e = 2 * ((c - 1) * n + ix);
+    if constexpr(sizeof(V) == 8)
+        return {T.ct[axis][e], T.ct[axis][e + 1]};
+    else
+        return {T.ct32[axis][e], T.ct32[axis][e + 1]};
+}
+
+// the classes of one row in up to 64 planes from k on: lane l holds plane k + l
+struct RowClasses
+{
+    int k0, v;
+    __device__ __forceinline__ void open(const unsigned char* row, int nz, int k)
+    {
+        k0 = k;
+        v = row[min(k + (int)(threadIdx.x & 63), nz - 1)];
+    }
+    __device__ __forceinline__ int at(int k) const { return __builtin_amdgcn_readlane(v, k - k0); }
+};
+
+// Loads of one plane of the walk, issued D planes ahead: the operand's raw inputs at one halo
+// cell of the block and at the cell above, the epilogue's inputs; of mixed rows also the
+// faces, aii above and aii of the halo cell.  Halo cells are spread over the threads: thread
+// h < 64 the south row (j0-1, i0+h), 64 <= h < 128 the north row (j0+TY, i0+h-64), 128 <= h <
+// 132 the west column (j0+h-128, i0-1), 132 <= h < 136 the east column (j0+h-132, i0+TX).
+template<class V, class R, class E>
+struct ClassIn
+{
+    R h, xu;
+    V f[6], ah, au;
+    E e;
+};
+
+// Where the operand's aii comes from: none needed (the operand is stored), loaded with the
+// operand (4 bytes cost less than the FP64 division), or from the row class
+enum
+{
+    AII_NONE = 0,
+    AII_LOAD = 1,
+    AII_CLASS = 2
+};
+
+// For the planes of a column run and the one below and above, in LDS: the z entries of both
+// classes, {water +, -, air +, -}, and the row classes (rows j0 .. j0+3, j0-1, j0+4, the west
+// and the east neighbours of the first four).  They are not loaded where they are used: a
+// global load in the plane loop that is used at once, on any path, waits for the loads in flight.
+constexpr int ZPLANES = 66, CROWS = 2 + 3 * TY;
+template<class V>
+struct ClassLDS
+{
+    V x[2][TY + 2][TX + 2];
+    double z[ZPLANES][4];
+    float z32[sizeof(V) == 4 ? ZPLANES : 1][4];
+    unsigned char c[CROWS][ZPLANES + 2];
+    // grid factors of the mixed rows' couplings
+    using AF = AxisFactor<std::conditional_t<sizeof(V) == 8, SolverOp64, SolverOp32>>;
+    AF ax[TX], ay[TY], az[ZPLANES];
+};
+
+// raw(cc) -> R: the loads of the stencil operand at cc; val(R, aii, V& aux) -> V: the operand
 // (aux: what the epilogue needs of the centre); pre(c) -> E: the epilogue's loads;
-// post(c, Ax, aux, E): the epilogue.  The loads of planes t+1 .. t+D are in flight while
-// plane t is staged, synchronised and computed: D = 2 for 4-byte operands, 1 for 8-byte
-// ones.  Every load of a plane is issued unconditionally at a clamped (valid) address
-// and masked afterwards, and the loop is unrolled over D+1 plane buffers, so no plane's
-// loads wait for the next plane's to be issued.
-template<class V, class Op, class Raw, class Val, class Pre, class Post>
-__device__ __forceinline__ void plane_walk(const DevGrid& g, const Op& op, const TileWalk& tw, Raw raw, Val val, Pre pre,
-                                           Post post)
+// post(c, Ax, aux, E): the epilogue.  Every load's address is valid (clamped) and its value
+// masked afterwards.  A column run is at most 64 planes (cpt <= 64).
+template<class V, int AII, int D, class Raw, class Val, class Pre, class Post>
+__device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const TileWalk& tw, Raw raw, Val val, Pre pre, Post post)
 {
     using R = decltype(raw(0u));
     using E = decltype(pre(0u));
-    using AF = AxisFactor<Op>;
-    using In = PlaneIn<V, R, E, AF>;
-    constexpr int D = sizeof(V) == 4 ? 2 : PW64_DEPTH;
-    static_assert(D == 1 || D == 2, "plane walk prefetch depth");
-    __shared__ PlaneLDS<V> L[2];
-    const V* __restrict__ fxa = face_x(op);
-    const V* __restrict__ fya = face_y(op);
-    const V* __restrict__ fza = face_z(op);
+    using In = ClassIn<V, R, E>;
+    constexpr bool DIV = AII == AII_CLASS, LOAD = AII == AII_LOAD;
+    __shared__ ClassLDS<V> S;
+    std::conditional_t<sizeof(V) == 8, SolverOp64, SolverOp32> op{};
+    if constexpr(sizeof(V) == 4) op = SolverOp32{nullptr, nullptr, nullptr, T.iDXN32, T.iDYN32, T.iDZN32};
+    const V *fxa, *fya, *fza, *aiia;
+    if constexpr(sizeof(V) == 8)
+    {
+        fxa = T.f[A_RFX];
+        fya = T.f[A_RFY];
+        fza = T.f[A_RFZ];
+        aiia = T.f[A_AII];
+    }
+    else
+    {
+        fxa = T.s[S_KX];
+        fya = T.s[S_KY];
+        fza = T.s[S_KZ];
+        aiia = T.s[S_AII];
+    }
     const int h = threadIdx.x;
-    // one tile row per wavefront: the row (and with it j and the column's y grid factors)
-    // is wave-uniform and lives in scalar registers
+    // one tile row per wavefront: the row (and with it j) is wave-uniform
     const int lane = h & (TX - 1), row = __builtin_amdgcn_readfirstlane(h >> 6);
-    // the halo cell of thread h relative to the tile origin (h < 136), and its LDS slot:
-    // h < 64 the south row (j0-1, i0+h), 64 <= h < 128 the north row (j0+TY, i0+h-64),
-    // 128 <= h < 132 the west column (j0+h-128, i0-1), 132 <= h < 136 the east column
-    // (j0+h-132, i0+TX); the halo faces: h < 64 the -y face of column i0+h,
-    // 128 <= h < 132 the -x face of row j0+h-128
-    int hi = 0, hj = 0, hrow = 0, hcol = 0;
+    // halo cell relative to the tile, its LDS slot, its row's classes
+    int hi = 0, hj = 0, hslot = 0, hrow = 0;
     if(h < TX)
     {
         hi = h;
         hj = -1;
-        hrow = 0;
-        hcol = h + 1;
+        hslot = h + 1;
+        hrow = TY;
     }
     else if(h < 2 * TX)
     {
         hi = h - TX;
         hj = TY;
+        hslot = (TY + 1) * (TX + 2) + h - TX + 1;
         hrow = TY + 1;
-        hcol = h - TX + 1;
     }
     else if(h < 2 * TX + TY)
     {
         hi = -1;
         hj = h - 2 * TX;
-        hrow = h - 2 * TX + 1;
-        hcol = 0;
+        hslot = (h - 2 * TX + 1) * (TX + 2);
+        hrow = TY + 2 + hj;
     }
     else if(h < 2 * TX + 2 * TY)
     {
         hi = TX;
         hj = h - 2 * TX - TY;
-        hrow = h - 2 * TX - TY + 1;
-        hcol = TX + 1;
+        hslot = (h - 2 * TX - TY + 1) * (TX + 2) + TX + 1;
+        hrow = 2 * TY + 2 + hj;
     }
     const bool has_halo = h < 2 * TX + 2 * TY;
-    const bool fh_y = h < TX, fh_x = h >= 2 * TX && h < 2 * TX + TY;
-    // position of a tile of the walk: plane k of column col = (bx, by).  The walk moves one
-    // tile at a time, so positions advance by increments (one division per item, at its
-    // start, instead of one per plane)
-    struct Pos
-    {
-        int k, col, bx, by;
+    const unsigned sxy = (unsigned)g.sxy, sx = (unsigned)g.sx;
+
+    // ---- column state
+    int k = 0, kend = 0, zk0 = 0;   // current plane, planes [k, kend) of this run, first z plane in LDS
+    int ic = 0, jc = 0;
+    bool in = false, hval = false;
+    unsigned coff = 0, hoff = 0;    // element offsets within plane k = 0
+    auto own = [&](int kk) { return __builtin_amdgcn_readfirstlane((int)S.c[row][kk - zk0]); };
+    // of the class each belongs to: the own cell's x coefficients and coupling sum over x and y,
+    // the same sum for the next own cell and for the halo cell
+    V cn = V(0), cs = V(0), s4 = V(0);
+    double s4N = 0.0, s4H = 0.0;
+    int keyC = 0, keyN = 0, keyH = 0;
+    auto sum_xy = [&](int c, int ci, int cj) {
+        const Pair<double> px = class_pair64(T, 0, g.nx, c, ci), py = class_pair64(T, 1, g.ny, c, cj);
+        return px.p + px.m + py.p + py.m;
     };
-    auto pos_of = [&](int tt) {
-        Pos q;
-        q.col = tt / tw.s.nbz;
-        q.k = tt - q.col * tw.s.nbz;
-        q.by = q.col / tw.s.nbx;
-        q.bx = q.col - q.by * tw.s.nbx;
-        return q;
+    // aii of a cell of class c in plane kk from its x and y sum (diag_of's order)
+    auto jacobi = [&](double sxy4, int c, int kk) -> V {
+        const double* const z = &S.z[kk - zk0][2 * c - 2];
+        return (V)(-1.0 / ((sxy4 + z[0] + z[1]) + 1e-19));
     };
-    auto adv = [&](Pos q) {
-        if(++q.k == tw.s.nbz)
+    auto own_a = [&](int kk, int c, V loaded) -> V {
+        if(!DIV || c == ROW_MIXED) return loaded;
+        if(c != keyN)
         {
-            q.k = 0;
-            ++q.col;
-            if(++q.bx == tw.s.nbx)
-            {
-                q.bx = 0;
-                ++q.by;
-            }
+            s4N = sum_xy(c, ic, jc);
+            keyN = c;
         }
-        return q;
-    };
-    // per-column state: the thread's cell, which halo/face loads are real
-    int i0, j0, k, col, i, j;
-    bool in = false, hval = false, fhval = false;
-    unsigned coff = 0, hoff = 0, fhoff = 0;   // element offsets within plane k = 0
-    auto column_setup = [&]() {
-        i = i0 + lane;
-        j = j0 + row;
-        in = i < g.nx && j < g.ny;
-        const int ic = min(i, g.nx - 1), jc = min(j, g.ny - 1);
-        coff = (unsigned)(g.base + ic + g.sx * jc);
-        const int ih = i0 + hi, jh = j0 + hj;
-        hval = has_halo && ih >= 0 && ih < g.nx && jh >= 0 && jh < g.ny;
-        hoff = (unsigned)(g.base + max(0, min(ih, g.nx - 1)) + g.sx * max(0, min(jh, g.ny - 1)));
-        const int jr = j0 + (h - 2 * TX);
-        fhval = (fh_y && i < g.nx && j0 < g.ny) || (fh_x && jr < g.ny);
-        if(fh_y)
-            fhoff = (unsigned)(g.base + ic + g.sx * (min(j0, g.ny - 1) - 1));
-        else if(fh_x)
-            fhoff = (unsigned)(g.base + i0 - 1 + g.sx * min(jr, g.ny - 1));
-        else
-            fhoff = coff;
+        return jacobi(s4N, c, kk);
     };
     auto fetch = [&](int kk, In& P) {
-        const unsigned pk = (unsigned)(g.sxy * kk);
-        const unsigned c = coff + pk;
-        P.h = raw(hoff + pk);
-        P.fh = ld32(fh_y ? fya : fxa, fhoff + pk);
-        P.f0 = ld32(fxa, c);
-        P.f2 = ld32(fya, c);
-        P.f4 = ld32(fza, c);
-        P.xu = raw(c + (unsigned)g.sxy);   // k + 1 <= nz: a ghost plane at worst
-        P.az = axis_factor(g, op, 2, kk);
+        const unsigned c = coff + sxy * (unsigned)kk;
+        const int ku = min(kk + 1, g.nz - 1);
+        const int co = own(kk), cu = own(ku), ch = S.c[hrow][kk - zk0];
+        P.h = raw(hoff + sxy * (unsigned)kk);
+        P.xu = raw(c + sxy);   // kk + 1 <= nz: a ghost plane at worst
         P.e = pre(c);
+        if(LOAD)
+        {
+            P.au = ld32(aiia, coff + sxy * (unsigned)ku);
+            P.ah = ld32(aiia, hoff + sxy * (unsigned)kk);
+        }
+        if(co == ROW_MIXED)
+        {
+            P.f[0] = ld32(fxa, c);
+            P.f[1] = ld32(fxa, c - 1u);
+            P.f[2] = ld32(fya, c);
+            P.f[3] = ld32(fya, c - sx);
+            P.f[4] = ld32(fza, c);
+            P.f[5] = ld32(fza, c - sxy);
+        }
+        if(DIV && cu == ROW_MIXED) P.au = ld32(aiia, coff + sxy * (unsigned)ku);
+        if(DIV && has_halo && ch == ROW_MIXED) P.ah = ld32(aiia, hoff + sxy * (unsigned)kk);
     };
-    // k-window of the operand: xd (k-1), xc (k) and the centre's aux; fzd: the -z face;
-    // ax, ay: the column's x and y grid factors
-    V xd, xc, auxc, fzd;
-    AF ax, ay;
+    V xd = V(0), xc = V(0), auxc = V(0);
     int t = tw.t;
-    if(t >= tw.t1) return;
-    Pos pc = pos_of(t);   // plane t
-    i0 = pc.bx * TX;
-    j0 = pc.by * TY;
-    k = pc.k;
-    col = pc.col;
-    bool v1 = false;   // D = 2: the buffer after the current one holds plane t+1
+    bool v1 = false;   // D = 2: the buffer after the current one holds plane k + 1
+    // start of a column run at tile t
     auto start = [&](In& P0, In& P1) {
-        column_setup();
-        const unsigned c = coff + (unsigned)(g.sxy * k);
+        const int col = t / tw.s.nbz;
+        k = t - col * tw.s.nbz;
+        const int by = col / tw.s.nbx, bx = col - by * tw.s.nbx;
+        kend = min(tw.s.nbz, k + (tw.t1 - t));
+        zk0 = max(k - 1, 0);
+        const int i0 = bx * TX, j0 = by * TY;
+        __syncthreads();   // the last run's entries have been read
+        for(int q = h; q < 4 * ZPLANES; q += NT)
+        {
+            const int kk = min(zk0 + (q >> 2), g.nz - 1), e = 2 * (((q >> 1) & 1) * g.nz + kk) + (q & 1);
+            S.z[q >> 2][q & 3] = T.ct[2][e];
+            if constexpr(sizeof(V) == 4) S.z32[q >> 2][q & 3] = T.ct32[2][e];
+        }
+        for(int q = h; q < CROWS * ZPLANES; q += NT)
+        {
+            const int rr = q / ZPLANES, kk = min(zk0 + q - rr * ZPLANES, g.nz - 1);
+            const int jr = rr < TY ? j0 + rr : rr == TY ? j0 - 1 : rr == TY + 1 ? j0 + TY : j0 + (rr - 2) % TY;
+            const int br = rr < TY + 2 ? bx : rr < 2 * TY + 2 ? bx - 1 : bx + 1;
+            const int jq = max(0, min(jr, g.ny - 1)), bq = max(0, min(br, tw.s.nbx - 1));
+            S.c[rr][q - rr * ZPLANES] = T.cls[((long)bq * g.ny + jq) * g.nz + kk];
+        }
+        if(h < TX)
+            S.ax[h] = axis_factor(g, op, 0, min(i0 + h, g.nx - 1));
+        else if(h < TX + TY)
+            S.ay[h - TX] = axis_factor(g, op, 1, min(j0 + h - TX, g.ny - 1));
+        else if(h >= 2 * TX && h < 2 * TX + ZPLANES)
+            S.az[h - 2 * TX] = axis_factor(g, op, 2, min(zk0 + h - 2 * TX, g.nz - 1));
+        __syncthreads();
+        const int i = i0 + lane, j = j0 + row;
+        in = i < g.nx && j < g.ny;
+        ic = min(i, g.nx - 1);
+        jc = min(j, g.ny - 1);
+        coff = (unsigned)(g.base + ic + g.sx * jc);
+        int ih = i0 + hi, jh = j0 + hj;
+        hval = has_halo && ih >= 0 && ih < g.nx && jh >= 0 && jh < g.ny;
+        ih = max(0, min(ih, g.nx - 1));
+        jh = max(0, min(jh, g.ny - 1));
+        hoff = (unsigned)(g.base + ih + g.sx * jh);
+        keyC = keyN = keyH = 0;
+        const unsigned c = coff + sxy * (unsigned)k;
         V d;
-        xd = (in && k > 0) ? val(raw(c - (unsigned)g.sxy), d) : V(0);
-        auxc = V(0);
-        xc = in ? val(raw(c), auxc) : V(0);
-        fzd = in ? ld32(fza, c - (unsigned)g.sxy) : V(0);
-        ax = axis_factor(g, op, 0, min(i, g.nx - 1));
-        ay = axis_factor(g, op, 1, min(j, g.ny - 1));
+        xd = xc = auxc = V(0);
+        if(k > 0)
+        {
+            const int cd = own(k - 1);
+            const V a = own_a(k - 1, cd, LOAD || (DIV && cd == ROW_MIXED) ? ld32(aiia, c - sxy) : V(0));
+            const V x = val(raw(c - sxy), a, d);
+            xd = in ? x : V(0);
+        }
+        {
+            const int cc = own(k);
+            const V a = own_a(k, cc, LOAD || (DIV && cc == ROW_MIXED) ? ld32(aiia, c) : V(0));
+            const V x = val(raw(c), a, auxc);
+            xc = in ? x : V(0);
+        }
         fetch(k, P0);
         v1 = false;
         if constexpr(D == 2)
-            if(t + 1 < tw.t1)
+            if(k + 1 < kend)
             {
-                const Pos q = D == 1 ? adv(pc) : pos_of(t + 1);
-                if(q.col == col)
-                {
-                    fetch(q.k, P1);
-                    v1 = true;
-                }
+                fetch(k + 1, P1);
+                v1 = true;
             }
     };
     int buf = 0;
-    // one plane: cur is plane t, n1 plane t+1 (D = 2), nf receives plane t+D; false at the end
+    // one plane: cur is plane k, nf receives plane k + D; n1: plane k + 1 (D = 2); false at the end
     auto step = [&](In& cur, In& n1, In& nf) -> bool {
-        PlaneLDS<V>& P = L[buf];
+        V* const P = &S.x[buf][0][0];
+        const int at = (row + 1) * (TX + 2) + lane + 1;
+        P[at] = xc;
+        if(has_halo)
         {
-            V d;
-            const V hv = val(cur.h, d);
-            P.x[row + 1][lane + 1] = xc;
-            if(has_halo) P.x[hrow][hcol] = hval ? hv : V(0);
-            P.fx[row][lane + 1] = in ? cur.f0 : V(0);
-            P.fy[row + 1][lane] = in ? cur.f2 : V(0);
-            const V fh = fhval ? cur.fh : V(0);
-            if(fh_y)
-                P.fy[0][h] = fh;
-            else if(fh_x)
-                P.fx[h - 2 * TX][0] = fh;
+            V a = cur.ah, d;
+            const int ch = S.c[hrow][k - zk0];
+            if(DIV && ch != ROW_MIXED)
+            {
+                if(ch != keyH)
+                {
+                    s4H = sum_xy(ch, (int)((hoff - (unsigned)g.base) % sx), (int)((hoff - (unsigned)g.base) / sx));
+                    keyH = ch;
+                }
+                a = jacobi(s4H, ch, k);
+            }
+            const V hv = val(cur.h, a, d);
+            P[hslot] = hval ? hv : V(0);
         }
         bool vf = false;
-        if(t + D < tw.t1 && (D == 1 || v1))
+        if(k + D < kend && (D == 1 || v1))
         {
-            const Pos q = D == 1 ? adv(pc) : pos_of(t + 2);
-            if(q.col == col)
-            {
-                fetch(q.k, nf);
-                vf = true;
-            }
+            fetch(k + D, nf);
+            vf = true;
         }
         __syncthreads();
-        V auxu = V(0);
-        const V xu = (in && k + 1 < g.nz) ? val(cur.xu, auxu) : V(0);
-        if(!(in && k + 1 < g.nz)) auxu = V(0);
-        if(in)
+        V auxu = V(0), xu = V(0);
+        if(k + 1 < g.nz)
         {
-            const unsigned c = coff + (unsigned)(g.sxy * k);
-            const CouplingV<V> cq =
-                coupling_axes(op, cur.f0, P.fx[row][lane], cur.f2, P.fy[row][lane], cur.f4, fzd, ax, ay, cur.az);
-            const V Ax = stencil7(g, cq, xc, P.x[row + 1][lane + 2], P.x[row + 1][lane], P.x[row + 2][lane + 1],
-                                  P.x[row][lane + 1], xu, xd, i, j, k);
-            post(c, Ax, auxc, cur.e);
+            const V a = own_a(k + 1, DIV ? own(k + 1) : 0, cur.au);
+            const V x = val(cur.xu, a, auxu);
+            xu = in ? x : V(0);
         }
-        buf ^= 1;
-        if(t + 1 >= tw.t1) return false;
-        ++t;
-        pc = D == 1 ? adv(pc) : pos_of(t);
-        if(pc.col == col)
+        const int c = own(k);
+        V Ax;
+        if(c == ROW_MIXED)
         {
-            xd = xc;
-            xc = xu;
-            auxc = auxu;
-            fzd = in ? cur.f4 : V(0);
-            k = pc.k;
-            v1 = vf;
+            const Coef<V> cf = poisson_coef(g,
+                                            coupling_axes(op, cur.f[0], cur.f[1], cur.f[2], cur.f[3], cur.f[4], cur.f[5],
+                                                          S.ax[lane], S.ay[row], S.az[k - zk0]),
+                                            ic, jc, k);
+            Ax = coef_apply(cf, true, xc, P[at + 1], P[at - 1], P[at + TX + 2], P[at - TX - 2], xu, xd);
         }
         else
         {
-            i0 = pc.bx * TX;
-            j0 = pc.by * TY;
-            k = pc.k;
-            col = pc.col;
-            // the next step's current buffer (and its successor) restart the column
-            if constexpr(D == 1)
-                start(nf, n1);
+            const int ey = 2 * ((c - 1) * g.ny + jc);
+            V yp, ym, zp, zm;
+            if constexpr(sizeof(V) == 8)
+            {
+                yp = ((CDouble*)T.ct[1])[ey];
+                ym = ((CDouble*)T.ct[1])[ey + 1];
+                zp = S.z[k - zk0][2 * c - 2];
+                zm = S.z[k - zk0][2 * c - 1];
+            }
             else
-                start(n1, nf);
+            {
+                yp = ((CFloat*)T.ct32[1])[ey];
+                ym = ((CFloat*)T.ct32[1])[ey + 1];
+                zp = S.z32[k - zk0][2 * c - 2];
+                zm = S.z32[k - zk0][2 * c - 1];
+            }
+            if(c != keyC)
+            {
+                const Pair<V> px = class_pair<V>(T, 0, g.nx, c, ic);
+                s4 = px.p + px.m + yp + ym;
+                cn = ic == g.nx - 1 ? V(0) : -px.p;
+                cs = ic == 0 ? V(0) : -px.m;
+                keyC = c;
+            }
+            const Coef<V> cf{s4 + zp + zm,
+                             cn,
+                             cs,
+                             jc == g.ny - 1 ? V(0) : -yp,
+                             jc == 0 ? V(0) : -ym,
+                             k == g.nz - 1 ? V(0) : -zp,
+                             k == 0 ? V(0) : -zm};
+            Ax = coef_apply(cf, true, xc, P[at + 1], P[at - 1], P[at + TX + 2], P[at - TX - 2], xu, xd);
         }
+        if(in) post(coff + sxy * (unsigned)k, Ax, auxc, cur.e);
+        buf ^= 1;
+        ++t;
+        if(t >= tw.t1) return false;
+        if(k + 1 < kend)
+        {
+            ++k;
+            xd = xc;
+            xc = xu;
+            auxc = auxu;
+            v1 = vf;
+        }
+        else if constexpr(D == 1)
+            start(nf, n1);
+        else
+            start(n1, nf);
         return true;
     };
+    if(t >= tw.t1) return;
+    In X, Y;
     if constexpr(D == 1)
     {
-        // one buffer ahead: the next plane lands in nx and is moved into cur (registers
-        // allow no second buffer for 8-byte operands at this occupancy)
-        In cur, nx;
-        start(cur, nx);
+        start(X, Y);
         #pragma unroll 1
         for(;;)
         {
-            if(!step(cur, nx, nx)) break;
-            cur = nx;
+            if(!step(X, Y, Y)) break;
+            if(!step(Y, X, X)) break;
         }
     }
     else
     {
-        In X, Y, Z;
+        In Z;
         start(X, Y);
         #pragma unroll 1
         for(;;)
@@ -959,6 +1102,73 @@ __device__ __forceinline__ void plane_walk(const DevGrid& g, const Op& op, const
             if(!step(Y, Z, X)) break;
             if(!step(Z, X, Y)) break;
         }
+    }
+}
+
+// Elementwise pass over an item of a plane-walked tank with aii from the row classes (mixed
+// rows load it): load(u, c) and use(u, c, aii) for each cell, U tiles at a time so that their
+// loads are in flight together; the cells of a thread come in tile order.
+template<class V, int U, class Load, class Use>
+__device__ __forceinline__ void class_cells(CTank& T, const DevGrid& g, const TileWalk& tw, Load load, Use use)
+{
+    const V* aii;
+    if constexpr(sizeof(V) == 8)
+        aii = T.f[A_AII];
+    else
+        aii = T.s[S_AII];
+    const int lane = threadIdx.x & 63, row = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    int t = tw.t;
+    #pragma unroll 1
+    while(t < tw.t1)
+    {
+        // a run of at most 64 tiles of one column
+        const int col = t / tw.s.nbz, k0 = t - col * tw.s.nbz, by = col / tw.s.nbx, bx = col - by * tw.s.nbx;
+        const int k1 = min(tw.s.nbz, k0 + (tw.t1 - t));
+        const int i = bx * TX + lane, j = by * TY + row;
+        const bool in = i < g.nx && j < g.ny;
+        const int ic = min(i, g.nx - 1), jc = min(j, g.ny - 1);
+        const unsigned c0 = (unsigned)(g.base + ic + g.sx * jc);
+        RowClasses own;
+        own.open(T.cls + ((long)bx * g.ny + jc) * g.nz, g.nz, k0);
+        int key = 0;
+        double s4 = 0.0;
+        #pragma unroll 1
+        for(int k = k0; k < k1; k += U)
+        {
+            V ae[U];
+            int cl[U];
+            double zs[U][2];
+            #pragma unroll
+            for(int u = 0; u < U; ++u)
+            {
+                const int kk = min(k + u, k1 - 1);
+                const unsigned c = c0 + (unsigned)(g.sxy * kk);
+                cl[u] = own.at(kk);
+                load(u, c);
+                CDouble* const z = (CDouble*)T.ct[2] + 2 * (max(cl[u] - 1, 0) * g.nz + kk);
+                zs[u][0] = z[0];
+                zs[u][1] = z[1];
+                ae[u] = V(0);
+                if(cl[u] == ROW_MIXED) ae[u] = ld32(aii, c);
+            }
+            #pragma unroll
+            for(int u = 0; u < U; ++u)
+            {
+                if(k + u >= k1) break;
+                if(cl[u] != ROW_MIXED)
+                {
+                    if(cl[u] != key)
+                    {
+                        const Pair<double> px = class_pair64(T, 0, g.nx, cl[u], ic), py = class_pair64(T, 1, g.ny, cl[u], jc);
+                        s4 = px.p + px.m + py.p + py.m;
+                        key = cl[u];
+                    }
+                    ae[u] = (V)(-1.0 / ((s4 + zs[u][0] + zs[u][1]) + 1e-19));
+                }
+                if(in) use(u, c0 + (unsigned)(g.sxy * (k + u)), ae[u]);
+            }
+        }
+        t += k1 - k0;
     }
 }
 
@@ -1132,7 +1342,7 @@ __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int r
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 2)
+        if(st->done || st->mode == 2 || plane_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1166,6 +1376,52 @@ __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int r
     }
 }
 
+// kb_bicg_p of the plane-walked tanks, aii from the row classes: 40 bytes per cell (r, p, v / p,
+// ph)
+__global__ void __launch_bounds__(NT, OCC_CX) kb_class_p(TankSet b, int x, int rhs)
+{
+    #pragma unroll 1
+    for(ItemIter q = set_items(b, 0, b.pw_items); q.q < q.hi; next_item(q, b))
+    {
+        CTank& T = tank_at(b, q.p);
+        const DevGrid g = T.g;
+        const BiState* st = T.st;
+        if(st->done || st->mode == 2)
+        {
+            skip_tank(q, b);
+            continue;
+        }
+        const BiVec<double> v = Prec<double>::vec(T, x, rhs);
+        const TileWalk tw = class_item(T, b, q);
+        if(st->mode == 1)
+        {
+            double vals[1] = {0.0};
+            restart_body(g, Prec<double>::op(T), v, tw, vals[0]);
+            block_sum_to<1>(vals, b.partials_ru + (size_t)tw.gi);
+            continue;
+        }
+        const double beta = st->beta, w = st->w;
+        const double* __restrict__ r = v.r;
+        const double* __restrict__ vv = v.v;
+        double* __restrict__ p = v.p;
+        double* __restrict__ ph = v.ph;
+        constexpr int U = 4;
+        double rr[U], pp[U], ve[U];
+        class_cells<double, U>(
+            T, g, tw,
+            [&](int u, unsigned c) {
+                rr[u] = ld32(r, c);
+                pp[u] = ld32(p, c);
+                ve[u] = ld32(vv, c);
+            },
+            [&](int u, unsigned c, double a) {
+                const double pn = rr[u] + beta * (pp[u] - w * ve[u]);
+                st32(p, c, pn);
+                st32(ph, c, pn * a);
+            });
+    }
+}
+
 // totals of a restart of the explicit-operator solve (km_p): ++solveriter, residual = |r|/N
 // (bicgstab_ijk.cpp:183-191); the Poisson solve's restarts are finalized by its v phase
 __global__ void kb_fin_p(TankSet b)
@@ -1184,18 +1440,17 @@ __global__ void kb_fin_p(TankSet b)
 // v = A ph; sigma = (v, r0), |v|^2 (bicgstab_ijk.cpp:151-160).  |r|^2 of the same loop is
 // the square norm of the residual the x phase (or the restart) has just formed and summed:
 // kb_fin_v takes it from the state instead of reading r again here.
-// PW: items of the tanks walked by the plane walk, else the others (direct stencil)
-template<class V, bool PW>
-__global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_FULL : OCC_A64)) kb_bicg_v(TankSet b, int x,
-                                                                                               int rhs)
+// Tanks without a plane walk; kb_class_v takes the others.
+template<class V>
+__global__ void __launch_bounds__(NT, sizeof(V) == 4 ? OCC_FULL : OCC_A64) kb_bicg_v(TankSet b, int x, int rhs)
 {
     #pragma unroll 1
-    for(ItemIter q = set_items_of<PW>(b); q.q < q.hi; next_item(q, b))
+    for(ItemIter q = set_items_of<false>(b); q.q < q.hi; next_item(q, b))
     {
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 3 || plane_walk_ok(T) != PW)
+        if(st->done || st->mode == 3 || plane_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1221,23 +1476,7 @@ __global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_F
             vals[0] += vd * double(r0[c]);
             vals[1] += vd * vd;
         };
-        if constexpr(PW)
-        {
-            struct EpiIn
-            {
-                V r0;
-            };
-            plane_walk<V>(
-                g, op, tw, [&](unsigned cc) { return ld32(ph, cc); }, [](V x, V&) { return x; },
-                [&](unsigned c) { return EpiIn{ld32(r0, c)}; },
-                [&](unsigned c, V Ax, V, const EpiIn& e) {
-                    st32(vo, c, Ax);
-                    const double vd = Ax;
-                    vals[0] += vd * double(e.r0);
-                    vals[1] += vd * vd;
-                });
-        }
-        else if(row_walk_ok(g, tw))
+        if(row_walk_ok(g, tw))
         {
             struct EpiIn
             {
@@ -1264,6 +1503,51 @@ __global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_F
                 epilogue(c, apply_A(g, cq, ph, c, i, j, k));
             }
         block_sum_to<3>(vals, b.partials + (size_t)item_slot(T, b, q) * 3);
+    }
+}
+
+// v = A ph of the plane-walked tanks (24 bytes per cell: ph, r0 / v).  The p update stays a
+// pass of its own (kb_class_p): fused into this walk, as the FP32 v phase has it, the FP64
+// operand needs r, p, v and aii at every stencil point, and the walk spills at 4 blocks per CU.
+__global__ void __launch_bounds__(NT, OCC_PW) kb_class_v(TankSet b, int x, int rhs)
+{
+    #pragma unroll 1
+    for(ItemIter q = set_items_of<true>(b); q.q < q.hi; next_item(q, b))
+    {
+        CTank& T = tank_at(b, q.p);
+        const DevGrid g = T.g;
+        const BiState* st = T.st;
+        if(st->done || st->mode == 3 || !plane_walk_ok(T))
+        {
+            skip_tank(q, b);
+            continue;
+        }
+        // mode 1: this iteration's p phase has restarted the tank (ph = aii r, fresh)
+        if(st->mode == 1
+           && __builtin_amdgcn_readfirstlane(restart_done(b.partials_ru + (size_t)T.item0, T.shape.nitems, st)))
+        {
+            skip_tank(q, b);
+            continue;
+        }
+        const BiVec<double> bv = Prec<double>::vec(T, x, rhs);
+        const TileWalk tw = class_item(T, b, q);
+        double vals[3] = {0.0, 0.0, 0.0};
+        const double* __restrict__ ph = bv.ph;
+        const double* __restrict__ r0 = bv.r0;
+        double* __restrict__ vo = bv.v;
+        struct EpiIn
+        {
+            double r0;
+        };
+        class_walk<double, AII_NONE, 2>(
+            T, g, tw, [&](unsigned cc) { return ld32(ph, cc); }, [](double z, double, double&) { return z; },
+            [&](unsigned c) { return EpiIn{ld32(r0, c)}; },
+            [&](unsigned c, double Ax, double, const EpiIn& e) {
+                st32(vo, c, Ax);
+                vals[0] += Ax * e.r0;
+                vals[1] += Ax * Ax;
+            });
+        block_sum_to<3>(vals, b.partials + (size_t)tw.gi * 3);
     }
 }
 
@@ -1319,8 +1603,52 @@ __global__ void __launch_bounds__(NT, PW ? OCC_PW : OCC_FULL) kb_mix_v(TankSet b
         float* __restrict__ ph = T.s[S_PH];
         float* __restrict__ x32 = T.s[S_X];
         double* __restrict__ x64 = T.f[x];
-        const TileWalk tw = item_walk(T, b, q);
+        const TileWalk tw = PW ? class_item(T, b, q) : item_walk(T, b, q);
         double vals[3] = {0.0, 0.0, 0.0};
+        if constexpr(PW)
+        {
+            // the operator and aii from the row classes; ph is not stored, the x phase forms it
+            struct EpiIn
+            {
+                float r0, r;
+            };
+            struct Rp
+            {
+                float r, p, v;
+            };
+            auto cpre = [&](unsigned c) { return EpiIn{ld32(r0, c), ld32(r, c)}; };
+            auto cpost = [&](unsigned c, float Ax, float pv, const EpiIn& e) {
+                st32(vn, c, Ax);
+                st32(pn, c, pv);
+                if(pend)
+                {
+                    st32(x64, c, ld32(x64, c) + (double)ld32(x32, c));
+                    st32(x32, c, 0.0f);
+                }
+                const double vd = Ax, rc = e.r;
+                vals[0] += vd * double(e.r0);
+                vals[1] += vd * vd;
+                vals[2] += rc * rc;
+            };
+            if(upd)
+                class_walk<float, AII_LOAD, 2>(
+                    T, g, tw, [&](unsigned cc) { return Rp{ld32(r, cc), ld32(pc, cc), ld32(vc, cc)}; },
+                    [&](const Rp& z, float a, float& pv) {
+                        pv = z.r + beta * (z.p - w * z.v);
+                        return pv * a;
+                    },
+                    cpre, cpost);
+            else
+                class_walk<float, AII_LOAD, 2>(
+                    T, g, tw, [&](unsigned cc) { return ld32(pc, cc); },
+                    [&](float z, float a, float& pv) {
+                        pv = z;
+                        return z * a;
+                    },
+                    cpre, cpost);
+            block_sum_to<3>(vals, b.partials + (size_t)tw.gi * 3);
+            continue;
+        }
         struct Epi
         {
             float r0, r, a, p;
@@ -1357,14 +1685,7 @@ __global__ void __launch_bounds__(NT, PW ? OCC_PW : OCC_FULL) kb_mix_v(TankSet b
         };
         auto raw_f = [&](unsigned cc) { return ld32(ph, cc); };
         auto val_f = [](float z, float&) { return z; };
-        if constexpr(PW)
-        {
-            if(upd)
-                plane_walk<float>(g, op, tw, raw_u, val_u, pre, post);
-            else
-                plane_walk<float>(g, op, tw, raw_f, val_f, pre, post);
-        }
-        else if(row_walk_ok(g, tw))
+        if(row_walk_ok(g, tw))
         {
             if(upd)
                 row_walk<float>(g, op, tw, raw_u, val_u, pre, post);
@@ -1391,7 +1712,7 @@ __global__ void __launch_bounds__(NT, PW ? OCC_PW : OCC_FULL) kb_mix_v(TankSet b
                     Ax = apply_A(g, cq, (const float*)ph, c, i, j, k);
                 post((unsigned)c, Ax, pnew, pre((unsigned)c));
             }
-        block_sum_to<3>(vals, b.partials + (size_t)item_slot(T, b, q) * 3);
+        block_sum_to<3>(vals, b.partials + (size_t)tw.gi * 3);
     }
 }
 
@@ -1427,13 +1748,13 @@ __global__ void kb_fin_v(TankSet b, int rr_state)
             restart_store(st, stot[0]);
             if(st->done) return;
         }
-        v_store(st, tot[0], tot[1], rr_state ? st->rr : tot[2]);
+        v_store(st, tot[0], tot[1], rr_state ? st->rr : tot[2], st->mixed);
     }
 }
 
 // s = r - alpha v, sh = aii s, t = A sh; (t,s), (t,t), (s,s) (bicgstab_ijk.cpp:193-221)
 template<class V, bool PW>
-__global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_FULL : OCC_A64)) kb_bicg_t(TankSet b, int x,
+__global__ void __launch_bounds__(NT, PW ? OCC_PW : (sizeof(V) == 4 ? OCC_FULL : OCC_A64)) kb_bicg_t(TankSet b, int x,
                                                                                                int rhs)
 {
     #pragma unroll 1
@@ -1449,7 +1770,7 @@ __global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_F
         }
         const BiVec<V> bv = Prec<V>::vec(T, x, rhs);
         const typename Prec<V>::Op op = Prec<V>::op(T);
-        const TileWalk tw = item_walk(T, b, q);
+        const TileWalk tw = PW ? class_item(T, b, q) : item_walk(T, b, q);
         double vals[3] = {0.0, 0.0, 0.0};
         const V alpha = (V)st->alpha;
         const V* __restrict__ r = bv.r;
@@ -1469,15 +1790,17 @@ __global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_F
         };
         if constexpr(PW)
         {
+            // t into the half of v's buffer that is not current
+            if constexpr(sizeof(V) == 4) to = T.s[st->buf ? S_V : S_V2];
             struct Rin
             {
-                V r, v, a;
+                V r, v;
             };
-            plane_walk<V>(
-                g, op, tw, [&](unsigned cc) { return Rin{ld32(r, cc), ld32(v, cc), ld32(a, cc)}; },
-                [&](const Rin& q, V& sv) {
+            class_walk<V, sizeof(V) == 8 ? AII_CLASS : AII_LOAD, sizeof(V) == 8 ? 1 : 2>(
+                T, g, tw, [&](unsigned cc) { return Rin{ld32(r, cc), ld32(v, cc)}; },
+                [&](const Rin& q, V aq, V& sv) {
                     sv = q.r - alpha * q.v;
-                    return sv * q.a;
+                    return sv * aq;
                 },
                 [](unsigned) { return NoEpi{}; },
                 [&](unsigned c, V Ax, V s, const NoEpi&) {
@@ -1523,7 +1846,7 @@ __global__ void __launch_bounds__(NT, PW ? occ_pw<V>() : (sizeof(V) == 4 ? OCC_F
                 const V t = apply_A_fn(g, cq, [&](long cc) { return cc == c ? shc : shv(cc, dummy); }, c, i, j, k);
                 epilogue(c, t, s);
             }
-        block_sum_to<3>(vals, b.partials + (size_t)item_slot(T, b, q) * 3);
+        block_sum_to<3>(vals, b.partials + (size_t)tw.gi * 3);
     }
 }
 
@@ -1551,7 +1874,7 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 1 || st->mode == 3)
+        if(st->done || st->mode == 1 || st->mode == 3 || plane_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1598,6 +1921,69 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
     }
 }
 
+// kb_bicg_x of the plane-walked tanks, aii from the row classes: 64 bytes per cell in FP64 (x,
+// ph, r, v, t, r0 / x, r); FP32 forms ph = aii p from the current p
+template<class V>
+__global__ void __launch_bounds__(NT, OCC_CX) kb_class_x(TankSet b, int x, int rhs)
+{
+    #pragma unroll 1
+    for(ItemIter q = set_items(b, 0, b.pw_items); q.q < q.hi; next_item(q, b))
+    {
+        CTank& T = tank_at(b, q.p);
+        const DevGrid g = T.g;
+        const BiState* st = T.st;
+        if(st->done || st->mode == 1 || st->mode == 3)
+        {
+            skip_tank(q, b);
+            continue;
+        }
+        const BiVec<V> bv = Prec<V>::vec(T, x, rhs);
+        const TileWalk tw = class_item(T, b, q);
+        const V alpha = (V)st->alpha, w = (V)st->w;
+        const int branch = st->branch;
+        double vals[2] = {0.0, 0.0};
+        V* __restrict__ xv = bv.x;
+        V* __restrict__ r = bv.r;
+        const V* __restrict__ vv = bv.v;
+        const V* __restrict__ pv = sizeof(V) == 8 ? bv.ph : bv.p;
+        const V* __restrict__ tv = bv.t;
+        if constexpr(sizeof(V) == 4) tv = T.s[st->buf ? S_V : S_V2];
+        const V* __restrict__ r0 = bv.r0;
+        constexpr int U = 4;
+        V xx[U], pp[U], rr[U], ve[U], te[U], r0e[U];
+        class_cells<V, U>(
+            T, g, tw,
+            [&](int u, unsigned c) {
+                xx[u] = ld32(xv, c);
+                pp[u] = ld32(pv, c);
+                rr[u] = ld32(r, c);
+                ve[u] = ld32(vv, c);
+                te[u] = ld32(tv, c);
+                r0e[u] = ld32(r0, c);
+            },
+            [&](int u, unsigned c, V a) {
+                const V ph = sizeof(V) == 8 ? pp[u] : pp[u] * a, s = rr[u] - alpha * ve[u];
+                V rn;
+                if(branch)
+                {
+                    const V sh = s * a;
+                    st32(xv, c, xx[u] + (alpha * ph + w * sh));
+                    rn = s - w * te[u];
+                }
+                else
+                {
+                    st32(xv, c, xx[u] + alpha * ph);
+                    rn = s;
+                }
+                st32(r, c, rn);
+                const double rd = rn;
+                vals[0] += rd * double(r0e[u]);
+                vals[1] += rd * rd;
+            });
+        block_sum_to<2>(vals, b.partials + (size_t)tw.gi * 2);
+    }
+}
+
 // beta, residual, iteration count; the mixed form asks for reliable updates instead of
 // ending on the iterated residual
 __global__ void kb_fin_x(TankSet b)
@@ -1634,7 +2020,10 @@ __global__ void __launch_bounds__(NT) kb_coef32(TankSet b)
         {
             int i, j, k;
             long c;
-            if(!tile_cell(g, tw, t, i, j, k, c)) continue;
+            const bool in = tile_cell(g, tw, t, i, j, k, c);
+            if(!in) c = g.base;
+            store_row_class(T, b, g, in, rfx[c], rfx[c - 1], rfy[c], rfy[c - g.sx], rfz[c], rfz[c - g.sxy], i, j, k);
+            if(!in) continue;
             const int ip = i + MARGE, jp = j + MARGE, kp = k + MARGE;
             kx[c] = (float)(1.0 / (rfx[c] * g.DXP[ip]));
             ky[c] = (float)(1.0 / (rfy[c] * g.DYP[jp]));
@@ -2665,18 +3054,24 @@ void bl_bicg_phase(const TankSet& b, int x, int rhs, int phase, int part, hipStr
     {
         switch(phase)
         {
-            case 0: hipLaunchKernelGGL(kb_bicg_p<double>, grid64, dim3(NT), 0, s, b, x, rhs); break;
+            case 0:
+                if(b.has_pw) hipLaunchKernelGGL(kb_class_p, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_p<double>, grid64, dim3(NT), 0, s, b, x, rhs);
+                break;
             case 1:
-                if(b.has_pw) hipLaunchKernelGGL((kb_bicg_v<double, true>), pgrid_pw(b, OCC_PW64), dim3(NT), 0, s, b, x, rhs);
+                if(b.has_pw) hipLaunchKernelGGL(kb_class_v, pgrid_pw(b, OCC_PW), dim3(NT), 0, s, b, x, rhs);
                 if(b.has_direct)
-                    hipLaunchKernelGGL((kb_bicg_v<double, false>), pgrid_direct(b, OCC_A64), dim3(NT), 0, s, b, x, rhs);
+                    hipLaunchKernelGGL(kb_bicg_v<double>, pgrid_direct(b, OCC_A64), dim3(NT), 0, s, b, x, rhs);
                 break;
             case 2:
-                if(b.has_pw) hipLaunchKernelGGL((kb_bicg_t<double, true>), pgrid_pw(b, OCC_PW64), dim3(NT), 0, s, b, x, rhs);
+                if(b.has_pw) hipLaunchKernelGGL((kb_bicg_t<double, true>), pgrid_pw(b, OCC_PW), dim3(NT), 0, s, b, x, rhs);
                 if(b.has_direct)
                     hipLaunchKernelGGL((kb_bicg_t<double, false>), pgrid_direct(b, OCC_A64), dim3(NT), 0, s, b, x, rhs);
                 break;
-            default: hipLaunchKernelGGL(kb_bicg_x<double>, grid, dim3(NT), 0, s, b, x, rhs); break;
+            default:
+                if(b.has_pw) hipLaunchKernelGGL(kb_class_x<double>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_x<double>, grid, dim3(NT), 0, s, b, x, rhs);
+                break;
         }
         return;
     }
@@ -2769,7 +3164,10 @@ void bl_mixed_phase(const TankSet& b, int x, int rhs, int phase, int part, hipSt
                 if(b.has_direct)
                     hipLaunchKernelGGL((kb_bicg_t<float, false>), pgrid_direct(b, OCC_FULL), dim3(NT), 0, s, b, x, rhs);
                 break;
-            case 2: hipLaunchKernelGGL(kb_bicg_x<float>, grid, dim3(NT), 0, s, b, x, rhs); break;
+            case 2:
+                if(b.has_pw) hipLaunchKernelGGL(kb_class_x<float>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_x<float>, grid, dim3(NT), 0, s, b, x, rhs);
+                break;
             default: hipLaunchKernelGGL(kb_mix_ru, pgrid(b, OCC_A64), dim3(NT), 0, s, b, x, rhs); break;
         }
         return;

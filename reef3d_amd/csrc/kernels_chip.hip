@@ -98,37 +98,6 @@ struct Guard
     }
 };
 
-// (A y)(c) from the coefficients in matvec_std's order (stencil7 / stencil5 / mat_apply):
-// outside the domain the operand is 0
-template<class V>
-struct Coef
-{
-    V p, n, s, w, e, t, b;
-};
-
-template<class V>
-__device__ __forceinline__ V coef_apply(const Coef<V>& m, bool d3, V yc, V yn, V ys, V yw, V ye, V yt, V yb)
-{
-    if(d3) return m.p * yc + m.n * yn + m.s * ys + m.w * yw + m.e * ye + m.t * yt + m.b * yb;
-    return m.p * yc + m.n * yn + m.s * ys + m.t * yt + m.b * yb;
-}
-
-// the coefficients stencil7 / stencil5 form from the couplings of cell (i, j, k)
-template<class V>
-__device__ __forceinline__ Coef<V> poisson_coef(const DevGrid& g, const CouplingV<V>& q, int i, int j, int k)
-{
-    Coef<V> m;
-    m.p = diag_of(g, q);
-    m.n = i == g.nx - 1 ? V(0) : -q.T[0];
-    m.s = i == 0 ? V(0) : -q.T[1];
-    m.t = k == g.nz - 1 ? V(0) : -q.T[4];
-    m.b = k == 0 ? V(0) : -q.T[5];
-    const V yd = (V)g.ydir;
-    m.w = j == g.ny - 1 ? V(0) : -q.T[2] * yd;
-    m.e = j == 0 ? V(0) : -q.T[3] * yd;
-    return m;
-}
-
 // wavefront sum by the butterfly off = 32, 16, .. 1 of block_sum_to and sum_partials, lane 0's
 // (and every lane's) bits: the swaps give both halves to all lanes, and the rotations within
 // 16 lanes reach the partner lane because the values already repeat with the previous offset
@@ -690,14 +659,14 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
         auto vrecv = [&](unsigned tg) { receive(halo0, tg, V(0), [&](int, int q, V val) { hv[q] = val; }); };
         if constexpr(KIND == CHIP_FP64)
             exchange(std::integral_constant<int, 2>(), vsums, vsend, vrecv,
-                     [&](const double* tot) { v_store(&st, tot[0], tot[1], st.rr); });
+                     [&](const double* tot) { v_store(&st, tot[0], tot[1], st.rr, false); });
         else
             exchange(std::integral_constant<int, 3>(),
                      [&](int c, double* s) {
                          vsums(c, s);
                          s[2] = double(r[c]) * double(r[c]);
                      },
-                     vsend, vrecv, [&](const double* tot) { v_store(&st, tot[0], tot[1], tot[2]); });
+                     vsend, vrecv, [&](const double* tot) { v_store(&st, tot[0], tot[1], tot[2], MIXED); });
         if(dead)
         {
             gone = true;

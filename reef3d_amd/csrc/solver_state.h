@@ -88,8 +88,9 @@ __device__ __forceinline__ void ru_store(BiState* st, const RuNext& n)
 }
 
 // alpha and the restart tests from the v phase's sums: sigma = (v, r0), vv = |v|^2, rr = |r|^2
-// (bicgstab_ijk.cpp:162-191)
-__device__ __forceinline__ void v_store(BiState* st, double sigma, double vv, double rr)
+// (bicgstab_ijk.cpp:162-191); swap: the phase wrote p and v into the other halves of their
+// buffers
+__device__ __forceinline__ void v_store(BiState* st, double sigma, double vv, double rr, bool swap)
 {
     const double norm_vj = sqrt(vv);
     const double norm_rj = sqrt(rr);
@@ -98,12 +99,8 @@ __device__ __forceinline__ void v_store(BiState* st, double sigma, double vv, do
     st->norm_vj = norm_vj;
     st->norm_rj = norm_rj;
     st->alpha = alpha;
-    if(st->mixed)
-    {
-        // the fused v phase wrote p and v into the other half and added x32
-        st->buf ^= 1;
-        st->pending = 0;
-    }
+    if(swap) st->buf ^= 1;
+    if(st->mixed) st->pending = 0;   // the fused v phase added x32
     if(fabs(sigma) <= (1.0e-12 * (norm_vj * st->norm_r0)))
         st->mode = 1;
     else if((fabs(alpha) * norm_vj / (norm_rj == 0 ? 1.0e-15 : norm_rj)) <= 0.08)

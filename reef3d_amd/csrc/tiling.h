@@ -86,6 +86,19 @@ REEF_HD int item_at(const TileShape& s, int l)
     return (l - zc * ncol) * s.zslab + zc;
 }
 
+// the item at position l for the phases whose work depends on the row classes: rows of mixed
+// class lie in one or two z-slabs, and z-slab-major order would give all of them to one XCD.
+// Here each XCD group's share is a group of whole columns, z-slab by z-slab within it, so the
+// blocks that share a CU (positions 32 apart) walk different slabs.
+REEF_HD int item_spread(const TileShape& s, int l)
+{
+    if(s.zslab == 0) return l;
+    const int ncol = s.nbx * s.nby, per = (ncol + 7) / 8;
+    const int x = l / (per * s.zslab), c0 = x * per, n = ncol - c0 < per ? ncol - c0 : per;
+    const int q = l - c0 * s.zslab, zc = q / n;
+    return (c0 + q - zc * n) * s.zslab + zc;
+}
+
 // items [lo, hi) walked by block group `xcd` (0..7) of a launch over nitems items
 REEF_HD void group_range(int nitems, int xcd, int& lo, int& hi)
 {
