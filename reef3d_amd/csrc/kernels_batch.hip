@@ -887,19 +887,21 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
         }
         return jacobi(s4N, c, kk);
     };
-    auto fetch = [&](int kk, In& P) {
+    // the loads of a plane that need no class, then those that do
+    auto fetch_raw = [&](int kk, In& P) {
         const unsigned c = coff + sxy * (unsigned)kk;
-        const int ku = min(kk + 1, g.nz - 1);
-        const int co = own(kk), cu = own(ku), ch = S.c[hrow][kk - zk0];
         P.h = raw(hoff + sxy * (unsigned)kk);
         P.xu = raw(c + sxy);   // kk + 1 <= nz: a ghost plane at worst
         P.e = pre(c);
         if(LOAD)
         {
-            P.au = ld32(aiia, coff + sxy * (unsigned)ku);
+            P.au = ld32(aiia, coff + sxy * (unsigned)min(kk + 1, g.nz - 1));
             P.ah = ld32(aiia, hoff + sxy * (unsigned)kk);
         }
-        if(co == ROW_MIXED)
+    };
+    auto fetch_mixed = [&](int kk, In& P) {
+        const unsigned c = coff + sxy * (unsigned)kk;
+        if(own(kk) == ROW_MIXED)
         {
             P.f[0] = ld32(fxa, c);
             P.f[1] = ld32(fxa, c - 1u);
@@ -908,8 +910,16 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
             P.f[4] = ld32(fza, c);
             P.f[5] = ld32(fza, c - sxy);
         }
-        if(DIV && cu == ROW_MIXED) P.au = ld32(aiia, coff + sxy * (unsigned)ku);
-        if(DIV && has_halo && ch == ROW_MIXED) P.ah = ld32(aiia, hoff + sxy * (unsigned)kk);
+        if(DIV)
+        {
+            const int ku = min(kk + 1, g.nz - 1);
+            if(own(ku) == ROW_MIXED) P.au = ld32(aiia, coff + sxy * (unsigned)ku);
+            if(has_halo && S.c[hrow][kk - zk0] == ROW_MIXED) P.ah = ld32(aiia, hoff + sxy * (unsigned)kk);
+        }
+    };
+    auto fetch = [&](int kk, In& P) {
+        fetch_raw(kk, P);
+        fetch_mixed(kk, P);
     };
     V xd = V(0), xc = V(0), auxc = V(0);
     int t = tw.t;
@@ -922,6 +932,26 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
         kend = min(tw.s.nbz, k + (tw.t1 - t));
         zk0 = max(k - 1, 0);
         const int i0 = bx * TX, j0 = by * TY;
+        const int i = i0 + lane, j = j0 + row;
+        in = i < g.nx && j < g.ny;
+        ic = min(i, g.nx - 1);
+        jc = min(j, g.ny - 1);
+        coff = (unsigned)(g.base + ic + g.sx * jc);
+        int ih = i0 + hi, jh = j0 + hj;
+        hval = has_halo && ih >= 0 && ih < g.nx && jh >= 0 && jh < g.ny;
+        ih = max(0, min(ih, g.nx - 1));
+        jh = max(0, min(jh, g.ny - 1));
+        hoff = (unsigned)(g.base + ih + g.sx * jh);
+        // the operand's first loads are in flight while the tables are staged
+        const unsigned c = coff + sxy * (unsigned)k;
+        const R rc = raw(c), rd = raw(k > 0 ? c - sxy : c);
+        V ac = V(0), ad = V(0);
+        if(LOAD)
+        {
+            ac = ld32(aiia, c);
+            ad = ld32(aiia, k > 0 ? c - sxy : c);
+        }
+        fetch_raw(k, P0);
         __syncthreads();   // the last run's entries have been read
         for(int q = h; q < 4 * ZPLANES; q += NT)
         {
@@ -931,7 +961,8 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
         }
         for(int q = h; q < CROWS * ZPLANES; q += NT)
         {
-            const int rr = q / ZPLANES, kk = min(zk0 + q - rr * ZPLANES, g.nz - 1);
+            const int rr = q / ZPLANES, kk = zk0 + q - rr * ZPLANES;
+            if(kk > min(kend, g.nz - 1)) continue;
             const int jr = rr < TY ? j0 + rr : rr == TY ? j0 - 1 : rr == TY + 1 ? j0 + TY : j0 + (rr - 2) % TY;
             const int br = rr < TY + 2 ? bx : rr < 2 * TY + 2 ? bx - 1 : bx + 1;
             const int jq = max(0, min(jr, g.ny - 1)), bq = max(0, min(br, tw.s.nbx - 1));
@@ -944,34 +975,13 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
         else if(h >= 2 * TX && h < 2 * TX + ZPLANES)
             S.az[h - 2 * TX] = axis_factor(g, op, 2, min(zk0 + h - 2 * TX, g.nz - 1));
         __syncthreads();
-        const int i = i0 + lane, j = j0 + row;
-        in = i < g.nx && j < g.ny;
-        ic = min(i, g.nx - 1);
-        jc = min(j, g.ny - 1);
-        coff = (unsigned)(g.base + ic + g.sx * jc);
-        int ih = i0 + hi, jh = j0 + hj;
-        hval = has_halo && ih >= 0 && ih < g.nx && jh >= 0 && jh < g.ny;
-        ih = max(0, min(ih, g.nx - 1));
-        jh = max(0, min(jh, g.ny - 1));
-        hoff = (unsigned)(g.base + ih + g.sx * jh);
         keyC = keyN = keyH = 0;
-        const unsigned c = coff + sxy * (unsigned)k;
         V d;
         xd = xc = auxc = V(0);
-        if(k > 0)
-        {
-            const int cd = own(k - 1);
-            const V a = own_a(k - 1, cd, LOAD || (DIV && cd == ROW_MIXED) ? ld32(aiia, c - sxy) : V(0));
-            const V x = val(raw(c - sxy), a, d);
-            xd = in ? x : V(0);
-        }
-        {
-            const int cc = own(k);
-            const V a = own_a(k, cc, LOAD || (DIV && cc == ROW_MIXED) ? ld32(aiia, c) : V(0));
-            const V x = val(raw(c), a, auxc);
-            xc = in ? x : V(0);
-        }
-        fetch(k, P0);
+        const int cc = own(k), cd = own(max(k - 1, 0));
+        if(DIV && cc == ROW_MIXED) ac = ld32(aiia, c);
+        if(DIV && cd == ROW_MIXED) ad = ld32(aiia, k > 0 ? c - sxy : c);
+        fetch_mixed(k, P0);
         v1 = false;
         if constexpr(D == 2)
             if(k + 1 < kend)
@@ -979,6 +989,13 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
                 fetch(k + 1, P1);
                 v1 = true;
             }
+        if(k > 0)
+        {
+            const V x = val(rd, own_a(k - 1, cd, ad), d);
+            xd = in ? x : V(0);
+        }
+        const V x = val(rc, own_a(k, cc, ac), auxc);
+        xc = in ? x : V(0);
     };
     int buf = 0;
     // one plane: cur is plane k, nf receives plane k + D; n1: plane k + 1 (D = 2); false at the end
