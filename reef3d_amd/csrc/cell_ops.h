@@ -11,6 +11,15 @@ namespace reef {
 
 constexpr int TX = 64, TY = 4, NT = 256;
 
+// tables read through the constant address space (scalar loads at a wave-uniform index)
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __attribute__((address_space(4))) const double CDouble;
+typedef __attribute__((address_space(4))) const float CFloat;
+#else
+typedef const double CDouble;
+typedef const float CFloat;
+#endif
+
 // ------------------------------------------------------------------ WENO5 core
 // Smoothness indicators, (IS+psi)^-2 weights without alpha normalisation and the
 // non-uniform reconstruction, in the operation order of weno_nug_func.h:48-196 and
@@ -23,6 +32,76 @@ constexpr int TX = 64, TY = 4, NT = 256;
 // identically (negation is exact and x - y is x + (-y)).
 // Table entry e of I, C, Q is at [e * st]: st = 1 for a cell's own table row (y, z), the
 // row length for the entry-major x tables.
+// Division without the range scaling of the IEEE sequence: v_rcp_f64, two Newton steps, the
+// quotient and its correction, which round correctly for normal operands whose quotient is
+// normal (the caller's guard).  8 instructions instead of 11.
+__device__ __forceinline__ double div_normal(double a, double b)
+{
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// a / d for a grid width d with r = 1 / d (rounded to nearest): the product is within 1.5 ulp,
+// the first correction makes it faithful, the second rounds correctly (Markstein 1990: with r
+// correctly rounded and q faithful, q + (a - q d) r rounds to a / d).  div_fixup gives the IEEE
+// results for infinities, NaN and zeros.  Operands below 1e-290 may differ in the last bit.  6
+// instructions instead of 11.
+__device__ __forceinline__ double div_width(double a, double d, double r)
+{
+    double q = a * r;
+    q = __builtin_fma(__builtin_fma(-q, d, a), r, q);
+    q = __builtin_fma(__builtin_fma(-q, d, a), r, q);
+    return __builtin_amdgcn_div_fixup(q, d, a);
+}
+
+// the three weights c / (a^2 (c0/a1^2 + c1/a2^2 + c2/a3^2)); the guard keeps every operand and
+// quotient of div_normal between 1e-281 and 1e281
+__device__ __forceinline__ void weno_weights(double c0, double c1, double c2, double a1, double a2, double a3, double& w1,
+                                             double& w2, double& w3)
+{
+    const double b1 = a1 * a1, b2 = a2 * a2, b3 = a3 * a3;
+    auto fine = [](double a) { return a > 1.0e-70 && a < 1.0e70; };
+    auto wide = [](double c) { return c > 1.0e-6 && c < 1.0e6; };
+    if(__all(fine(a1) && fine(a2) && fine(a3) && wide(c0) && wide(c1) && wide(c2)))
+    {
+        const double S = div_normal(c0, b1) + div_normal(c1, b2) + div_normal(c2, b3);
+        w1 = div_normal(c0, 0.0 + b1 * S);
+        w2 = div_normal(c1, 0.0 + b2 * S);
+        w3 = div_normal(c2, 0.0 + b3 * S);
+        return;
+    }
+    w1 = c0 / (0.0 + b1 * (c0 / b1 + c1 / b2 + c2 / b3));
+    w2 = c1 / (0.0 + b2 * (c0 / b1 + c1 / b2 + c2 / b3));
+    w3 = c2 / (0.0 + b3 * (c0 / b1 + c1 / b2 + c2 / b3));
+}
+
+// weno_recon with the side of every lane the same (M: the stencil from below): no selects, and
+// at a wave-uniform table row (CD: the constant address space) the entries load through the
+// scalar unit
+template<bool M, class CD>
+__device__ __forceinline__ double weno_side(CD* __restrict__ I, CD* __restrict__ C, CD* __restrict__ Q, long st, double q1,
+                                            double q2, double q3, double q4, double q5)
+{
+    const double dq12 = q1 - q2, dq23 = q2 - q3, dq32 = q3 - q2, dq34 = q3 - q4, dq43 = q4 - q3, dq54 = q5 - q4;
+    constexpr int r = M ? 0 : 3;
+    CD* I1 = I + (long)(r * 3) * st;
+    const double is1 = I1[0] * dq54 * dq54 + I1[st] * (dq54) * (dq34) + I1[2 * st] * dq34 * dq34;
+    const double is2 = I1[3 * st] * dq23 * dq23 + I1[4 * st] * (dq43) * (dq23) + I1[5 * st] * dq43 * dq43;
+    const double is3 = I1[6 * st] * dq12 * dq12 + I1[7 * st] * (dq32) * (dq12) + I1[8 * st] * dq32 * dq32;
+    double w1, w2, w3;
+    weno_weights(C[r * st], C[(r + 1) * st], C[(r + 2) * st], is1 + 1.0e-6, is2 + 1.0e-6, is3 + 1.0e-6, w1, w2, w3);
+    CD* Qs = Q + (long)(M ? 0 : 6) * st;
+    const double A1 = Qs[0], B1 = M ? -Qs[st] : Qs[st];
+    const double A2 = Qs[2 * st], B2 = Qs[3 * st];
+    const double u2 = M ? dq43 : dq23, v2 = M ? dq23 : dq43;
+    const double A3 = Qs[4 * st], B3 = M ? Qs[5 * st] : -Qs[5 * st];
+    const double u3 = M ? dq12 : dq32, v3 = M ? dq32 : dq12;
+    return w1 * (q4 + A1 * dq34 + B1 * dq54) + w2 * (q3 + A2 * u2 - B2 * v2) + w3 * (q2 + A3 * u3 + B3 * v3);
+}
+
 __device__ __forceinline__ double weno_recon(const double* __restrict__ I, const double* __restrict__ C,
                                              const double* __restrict__ Q, long st, bool minus, double q1, double q2,
                                              double q3, double q4, double q5)
@@ -33,11 +112,8 @@ __device__ __forceinline__ double weno_recon(const double* __restrict__ I, const
     const double is1 = I1[0] * dq54 * dq54 + I1[st] * (dq54) * (dq34) + I1[2 * st] * dq34 * dq34;
     const double is2 = I1[3 * st] * dq23 * dq23 + I1[4 * st] * (dq43) * (dq23) + I1[5 * st] * dq43 * dq43;
     const double is3 = I1[6 * st] * dq12 * dq12 + I1[7 * st] * (dq32) * (dq12) + I1[8 * st] * dq32 * dq32;
-    const double a1 = is1 + 1.0e-6, a2 = is2 + 1.0e-6, a3 = is3 + 1.0e-6;
-    const double c0 = C[r * st], c1 = C[(r + 1) * st], c2 = C[(r + 2) * st];
-    const double w1 = c0 / (0.0 + (a1 * a1) * (c0 / (a1 * a1) + c1 / (a2 * a2) + c2 / (a3 * a3)));
-    const double w2 = c1 / (0.0 + (a2 * a2) * (c0 / (a1 * a1) + c1 / (a2 * a2) + c2 / (a3 * a3)));
-    const double w3 = c2 / (0.0 + (a3 * a3) * (c0 / (a1 * a1) + c1 / (a2 * a2) + c2 / (a3 * a3)));
+    double w1, w2, w3;
+    weno_weights(C[r * st], C[(r + 1) * st], C[(r + 2) * st], is1 + 1.0e-6, is2 + 1.0e-6, is3 + 1.0e-6, w1, w2, w3);
     // minus: w1 (q4 + Q0 (q3 - q4) - Q1 (q5 - q4)) + w2 (q3 + Q2 (q4 - q3) - Q3 (q2 - q3))
     //        + w3 (q2 + Q4 (q1 - q2) + Q5 (q3 - q2))
     // plus:  w1 (q4 + Q6 (q3 - q4) + Q7 (q5 - q4)) + w2 (q3 + Q8 (q2 - q3) - Q9 (q4 - q3))
@@ -51,47 +127,92 @@ __device__ __forceinline__ double weno_recon(const double* __restrict__ I, const
     return w1 * (q4 + A1 * dq34 + B1 * dq54) + w2 * (q3 + A2 * u2 - B2 * v2) + w3 * (q2 + A3 * u3 + B3 * v3);
 }
 
-// HJ gradient along one axis at index ix (stride s) on the side `minus` chosen per lane,
-// given the two central divided differences dd2 = (f0 - fm1) / D(ip-1) and
-// dd3 = (fp1 - f0) / D(ip) (weno_hj_df_nug.cpp:344-396 / ddweno_nug_sf.cpp:186-224): the
-// minus stencil takes (fm2 - fm3) / D(ip-3), dd1, dd2, dd3, dd4, the plus stencil dd1, dd2,
-// dd3, dd4, (fp3 - fp2) / D(ip+2); only the outer quotient of the lane's side is formed
-__device__ __forceinline__ double hj_grad_dd(const DevGrid& g, int axis, const double* __restrict__ f, long c, long s,
-                                             int ix, bool minus, double dd2, double dd3)
+// the reconstruction of the active lanes along one axis: by a wavefront that takes one side,
+// or per lane.  The y and z table rows are the wavefront's (tile_cell_row).
+__device__ __forceinline__ double weno_axis(int axis, const double* I, const double* C, const double* Q, long st, bool minus,
+                                            double q1, double q2, double q3, double q4, double q5)
+{
+    const bool all_m = __all(minus), all_p = !__any(minus);
+    if(all_m || all_p)
+    {
+        if(axis == 0)
+            return all_m ? weno_side<true>(I, C, Q, st, q1, q2, q3, q4, q5) : weno_side<false>(I, C, Q, st, q1, q2, q3, q4, q5);
+        CDouble *i = (CDouble*)I, *c = (CDouble*)C, *q = (CDouble*)Q;
+        return all_m ? weno_side<true>(i, c, q, 1, q1, q2, q3, q4, q5) : weno_side<false>(i, c, q, 1, q1, q2, q3, q4, q5);
+    }
+    return weno_recon(I, C, Q, st, minus, q1, q2, q3, q4, q5);
+}
+
+// The stencil values f(-3) .. f(+3) along one axis (v[3] is the cell).  The momentum flux loads
+// them for the three axes before the sides are known: its two faces per axis share them, and
+// one memory latency covers them (240 -> 220 us on 512x64x128).  The HJ and reinit stages load
+// where they use (LineAt): with the values held they take 90 registers instead of 70 and were
+// 6 % slower.
+struct Line
+{
+    double v[7];
+};
+
+// the same values loaded where they are used
+struct LineAt
+{
+    const double* __restrict__ f;
+    long s;
+    __device__ __forceinline__ double operator()(int q) const { return f[q * s]; }
+    __device__ __forceinline__ double outer(bool minus) const { return f[minus ? -3 * s : 3 * s]; }
+};
+
+__device__ __forceinline__ Line load_line(const double* __restrict__ f, long c, long s)
+{
+    Line l;
+    #pragma unroll
+    for(int q = 0; q < 7; ++q) l.v[q] = f[c + (q - 3) * s];
+    return l;
+}
+
+// HJ gradient along one axis at index ix on the side `minus` chosen per lane, given the two
+// central divided differences dd2 = (f0 - fm1) / D(ip-1) and dd3 = (fp1 - f0) / D(ip)
+// (weno_hj_df_nug.cpp:344-396 / ddweno_nug_sf.cpp:186-224): the minus stencil takes (fm2 - fm3)
+// / D(ip-3), dd1, dd2, dd3, dd4, the plus stencil dd1, dd2, dd3, dd4, (fp3 - fp2) / D(ip+2);
+// only the outer quotient of the lane's side is formed
+template<class L>
+__device__ __forceinline__ double hj_grad_dd(const DevGrid& g, int axis, const L& l, int ix, bool minus, double dd2,
+                                             double dd3)
 {
     const int ip = ix + MARGE;
     const double* D = axis == 0 ? g.DXP : axis == 1 ? g.DYP : g.DZP;
+    const double* R = axis == 0 ? g.RDXP : axis == 1 ? g.RDYP : g.RDZP;
     const long st = axis == 0 ? g.nT : 1;
     const double* I = axis == 0 ? g.isfT + ip : g.isf[axis] + (size_t)ip * 36;
     const double* C = axis == 0 ? g.cfT + ip : g.cf[axis] + (size_t)ip * 12;
     const double* Q = axis == 0 ? g.qfT + ip : g.qf[axis] + (size_t)ip * 24;
-    const double fm2 = f[c - 2 * s], fm1 = f[c - s], fp1 = f[c + s], fp2 = f[c + 2 * s];
-    const double fo = f[minus ? c - 3 * s : c + 3 * s];
-    const double dd1 = (fm1 - fm2) / D[ip - 2];
-    const double dd4 = (fp2 - fp1) / D[ip + 1];
-    const double ddo = (minus ? fm2 - fo : fo - fp2) / D[minus ? ip - 3 : ip + 2];
-    return weno_recon(I, C, Q, st, minus, minus ? ddo : dd1, minus ? dd1 : dd2, minus ? dd2 : dd3, minus ? dd3 : dd4,
-                      minus ? dd4 : ddo);
+    const double dd1 = div_width(l(-1) - l(-2), D[ip - 2], R[ip - 2]);
+    const double dd4 = div_width(l(2) - l(1), D[ip + 1], R[ip + 1]);
+    const int io = minus ? ip - 3 : ip + 2;
+    const double fo = l.outer(minus);
+    const double ddo = div_width(minus ? l(-2) - fo : fo - l(2), D[io], R[io]);
+    return weno_axis(axis, I, C, Q, st, minus, minus ? ddo : dd1, minus ? dd1 : dd2, minus ? dd2 : dd3, minus ? dd3 : dd4,
+                     minus ? dd4 : ddo);
 }
 
 // the HJ gradient upwind of advec (minus for advec > 0, plus for advec < 0, 0 otherwise)
-__device__ __forceinline__ double hj_grad(const DevGrid& g, int axis, const double* __restrict__ f, long c, long s,
-                                          int ix, double advec)
+template<class L>
+__device__ __forceinline__ double hj_grad(const DevGrid& g, int axis, const L& l, int ix, double advec)
 {
     const bool minus = advec > 0.0;
     if(!minus && !(advec < 0.0)) return 0.0;
     const int ip = ix + MARGE;
     const double* D = axis == 0 ? g.DXP : axis == 1 ? g.DYP : g.DZP;
-    const double f0 = f[c];
-    return hj_grad_dd(g, axis, f, c, s, ix, minus, (f0 - f[c - s]) / D[ip - 1], (f[c + s] - f0) / D[ip]);
+    const double* R = axis == 0 ? g.RDXP : axis == 1 ? g.RDYP : g.RDZP;
+    return hj_grad_dd(g, axis, l, ix, minus, div_width(l(0) - l(-1), D[ip - 1], R[ip - 1]),
+                      div_width(l(1) - l(0), D[ip], R[ip]));
 }
 
 // ------------------------------------------------------------------ WENO flux
-// weno_flux_nug::fx/fy/fz with iqmin..kqmax (weno_flux_nug.cpp:136-313): values; the
-// x upwind-from-above stencil repeats f(i+2) (weno_flux_nug.cpp:288-295).  The side is
-// chosen per lane (weno_recon).
-__device__ __forceinline__ double flux_face(const DevGrid& g, int axis, int uf, const double* __restrict__ f, long c,
-                                            long s, int ix, double advec)
+// weno_flux_nug::fx/fy/fz with iqmin..kqmax (weno_flux_nug.cpp:136-313) at the face between the
+// cells v[q] and v[q + 1] of the line; the x upwind-from-above stencil repeats f(i+2)
+// (weno_flux_nug.cpp:288-295).  The side is chosen per lane (weno_axis).
+__device__ __forceinline__ double flux_face(const DevGrid& g, int axis, int uf, const double* v, int ix, double advec)
 {
     const bool minus = advec > 0.0;
     if(!minus && !(advec < 0.0)) return 0.0;
@@ -100,10 +221,9 @@ __device__ __forceinline__ double flux_face(const DevGrid& g, int axis, int uf, 
     const double* I = axis == 0 ? g.isfT + (long)(uf * 18) * st + ip : g.isf[axis] + (size_t)ip * 36 + uf * 18;
     const double* C = axis == 0 ? g.cfT + (long)(uf * 6) * st + ip : g.cf[axis] + (size_t)ip * 12 + uf * 6;
     const double* Q = axis == 0 ? g.qfT + (long)(uf * 12) * st + ip : g.qf[axis] + (size_t)ip * 24 + uf * 12;
-    const double fm1 = f[c - s], f0 = f[c], fp1 = f[c + s], fp2 = f[c + 2 * s];
-    const double fo = f[minus ? c - 2 * s : (axis == 0 ? c + 2 * s : c + 3 * s)];
-    return weno_recon(I, C, Q, st, minus, minus ? fo : fm1, minus ? fm1 : f0, minus ? f0 : fp1, minus ? fp1 : fp2,
-                      minus ? fp2 : fo);
+    const double fo = minus ? v[-2] : (axis == 0 ? v[2] : v[3]);
+    return weno_axis(axis, I, C, Q, st, minus, minus ? fo : v[-1], minus ? v[-1] : v[0], minus ? v[0] : v[1],
+                     minus ? v[1] : v[2], minus ? v[2] : fo);
 }
 
 // flux divergence of component ipol at cell c (weno_flux_nug.cpp:110-134) with the
@@ -137,15 +257,17 @@ __device__ __forceinline__ double flux_div(const DevGrid& g, int ipol, const dou
     const double* DY = ipol == 2 ? g.DYP : g.DYN;
     const double* DZ = ipol == 3 ? g.DZP : g.DZN;
     double fv1 = 0.0, fv2 = 0.0;
-    const double fu1 = flux_face(g, 0, ufx, q, c - 1, 1, i - 1, iv1);
-    const double fu2 = flux_face(g, 0, ufx, q, c, 1, i, iv2);
+    const Line lx = load_line(q, c, 1), lz = load_line(q, c, sxy);
+    const Line ly = g.jdir == 1 ? load_line(q, c, sx) : lx;
+    const double fu1 = flux_face(g, 0, ufx, lx.v + 2, i - 1, iv1);
+    const double fu2 = flux_face(g, 0, ufx, lx.v + 3, i, iv2);
     if(g.jdir == 1)
     {
-        fv1 = flux_face(g, 1, ufy, q, c - sx, sx, j - 1, jv1);
-        fv2 = flux_face(g, 1, ufy, q, c, sx, j, jv2);
+        fv1 = flux_face(g, 1, ufy, ly.v + 2, j - 1, jv1);
+        fv2 = flux_face(g, 1, ufy, ly.v + 3, j, jv2);
     }
-    const double fw1 = flux_face(g, 2, ufz, q, c - sxy, sxy, k - 1, kv1);
-    const double fw2 = flux_face(g, 2, ufz, q, c, sxy, k, kv2);
+    const double fw1 = flux_face(g, 2, ufz, lz.v + 2, k - 1, kv1);
+    const double fw2 = flux_face(g, 2, ufz, lz.v + 3, k, kv2);
     return -((iv2 * fu2 - iv1 * fu1) / DX[i + MARGE]) - ((jv2 * fv2 - jv1 * fv1) / DY[j + MARGE])
          - ((kv2 * fw2 - kv1 * fw1) / DZ[k + MARGE]);
 }
@@ -494,9 +616,10 @@ __device__ __forceinline__ double hj_L(const DevGrid& g, const double* __restric
     const double iadvec = 0.5 * (u[c] + u[c - 1]);
     const double jadvec = 0.5 * (v[c] + v[c - g.sx]);
     const double kadvec = 0.5 * (w[c] + w[c - g.sxy]);
-    double L = -iadvec * hj_grad(g, 0, phi_s, c, 1, i, iadvec);
-    if(g.jdir == 1) L -= jadvec * hj_grad(g, 1, phi_s, c, g.sx, j, jadvec);
-    L -= kadvec * hj_grad(g, 2, phi_s, c, g.sxy, k, kadvec);
+    const LineAt lx{phi_s + c, 1}, ly{phi_s + c, g.sx}, lz{phi_s + c, g.sxy};
+    double L = -iadvec * hj_grad(g, 0, lx, i, iadvec);
+    if(g.jdir == 1) L -= jadvec * hj_grad(g, 1, ly, j, jadvec);
+    L -= kadvec * hj_grad(g, 2, lz, k, kadvec);
     return L;
 }
 
@@ -508,12 +631,12 @@ __device__ __forceinline__ double reini_L(const DevGrid& g, const double* __rest
                                           int fsf)
 {
     const int ip = i + MARGE, jp = j + MARGE, kp = k + MARGE;
-    const double lsv = f[c];
+    const LineAt lx{f + c, 1}, ly{f + c, g.sx}, lz{f + c, g.sxy};
+    const double lsv = lx(0);
     bool active = true;
     if(fsf)
     {
-        const double n1 = f[c + 1], n2 = f[c - 1], n3 = f[c + g.sx], n4 = f[c - g.sx], n5 = f[c + g.sxy],
-                     n6 = f[c - g.sxy];
+        const double n1 = lx(1), n2 = lx(-1), n3 = ly(1), n4 = ly(-1), n5 = lz(1), n6 = lz(-1);
         active = (lsv >= 0.0 && n1 >= 0.0 && n2 >= 0.0 && n3 >= 0.0 && n4 >= 0.0 && n5 >= 0.0 && n6 >= 0.0)
               || (lsv < 0.0 && n1 < 0.0 && n2 < 0.0 && n3 < 0.0 && n4 < 0.0 && n5 < 0.0 && n6 < 0.0);
     }
@@ -526,19 +649,19 @@ __device__ __forceinline__ double reini_L(const DevGrid& g, const double* __rest
         // the side of each axis (reinidisc_f.cpp:78-104): minus, plus or none (the three tests
         // exclude each other but for the last, which zeroes the gradient); the quotients of
         // the tests are the central divided differences of the WENO stencil
-        auto axis_grad = [&](int axis, long st, int ix, const double* DP, int pp) {
-            const double dmin = (lsv - f[c - st]) / DP[pp - 1];
-            const double dplus = (f[c + st] - lsv) / DP[pp];
+        auto axis_grad = [&](int axis, const LineAt& l, int ix, const double* DP, const double* RP, int pp) {
+            const double dmin = div_width(lsv - l(-1), DP[pp - 1], RP[pp - 1]);
+            const double dplus = div_width(l(1) - lsv, DP[pp], RP[pp]);
             const bool cm = dmin * lsSig > 0.0 && dplus * lsSig > -dmin * lsSig;
             const bool cp = dplus * lsSig < 0.0 && dmin * lsSig < -dplus * lsSig;
             const bool cz = dplus * lsSig > 0.0 && dmin * lsSig < 0.0;
             double d = 0.0;
-            if((cm || cp) && !cz) d = hj_grad_dd(g, axis, f, c, st, ix, cm, dmin, dplus);
+            if((cm || cp) && !cz) d = hj_grad_dd(g, axis, l, ix, cm, dmin, dplus);
             return d;
         };
-        dx = axis_grad(0, 1, i, g.DXP, ip);
-        if(g.jdir == 1) dy = axis_grad(1, g.sx, j, g.DYP, jp);
-        dz = axis_grad(2, g.sxy, k, g.DZP, kp);
+        dx = axis_grad(0, lx, i, g.DXP, g.RDXP, ip);
+        if(g.jdir == 1) dy = axis_grad(1, ly, j, g.DYP, g.RDYP, jp);
+        dz = axis_grad(2, lz, k, g.DZP, g.RDZP, kp);
         const double dnorm = sqrt(dx * dx + dy * dy + dz * dz);
         double deltax;
         if(g.jdir == 0)

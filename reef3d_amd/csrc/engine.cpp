@@ -273,6 +273,11 @@ int Engine::build_tank(const reef_grid_desc& gd, const reef_params& p, TankBuild
         b.offinv[a] = b.inv.size();
         for(double d : h.DN[a]) b.inv.push_back(d != 0.0 ? (float)(1.0 / d) : 0.0f);
     }
+    for(int a = 0; a < 3; ++a)
+    {
+        b.offRDP[a] = b.meta.size();
+        for(double d : h.DP[a]) b.meta.push_back(d != 0.0 ? 1.0 / d : 0.0);
+    }
     // couplings of rows of one density (W1 water, W3 air) with the operations of couplings() and
     // of kb_coef32 / coupling_of
     for(int a = 0; a < 3; ++a)
@@ -397,11 +402,13 @@ int Engine::add_built(TankBuild& b, int* id)
     if(!ops.empty()) EHIP(hipMemcpy(opd, ops.data(), ops.size() * sizeof(GhostOp), hipMemcpyHostToDevice));
     const double* md = (const double*)mb;
     const double** d1[3][3] = {{&g.XP, &g.DXN, &g.DXP}, {&g.YP, &g.DYN, &g.DYP}, {&g.ZP, &g.DZN, &g.DZP}};
+    const double** rd[3] = {&g.RDXP, &g.RDYP, &g.RDZP};
     for(int a = 0; a < 3; ++a)
     {
         *d1[a][0] = md + b.offP[a];
         *d1[a][1] = md + b.offDN[a];
         *d1[a][2] = md + b.offDP[a];
+        *rd[a] = md + b.offRDP[a];
         g.qf[a] = md + b.offqf[a];
         g.cf[a] = md + b.offcf[a];
         g.isf[a] = md + b.offisf[a];

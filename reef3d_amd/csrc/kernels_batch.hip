@@ -712,15 +712,6 @@ struct NoEpi
 // What bounds it: HBM bytes.  On the 512x64x128 wave tank 91 % of the rows have one class and
 // read neither faces nor aii.
 
-// table entries through the constant address space (scalar loads at a uniform index)
-#if defined(__HIP_DEVICE_COMPILE__)
-typedef __attribute__((address_space(4))) const double CDouble;
-typedef __attribute__((address_space(4))) const float CFloat;
-#else
-typedef const double CDouble;
-typedef const float CFloat;
-#endif
-
 // the couplings of a row class along one axis at index ix
 template<class V>
 struct Pair

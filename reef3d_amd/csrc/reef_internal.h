@@ -29,6 +29,7 @@ struct DevGrid
     double psi;
     // 1-D metadata, MARGE-offset (entry i + MARGE)
     const double *DXP, *DYP, *DZP, *DXN, *DYN, *DZN, *XP, *YP, *ZP;
+    const double *RDXP, *RDYP, *RDZP;   // 1 / DXP, .. rounded to nearest
     // WENO tables per axis: qf [IP][uf][12], cf [IP][uf][6], isf [IP][uf][18]
     const double *qf[3], *cf[3], *isf[3];
     // the x tables entry-major: qfT [uf * 12 + e][IP], cfT [uf * 6 + e][IP], isfT [uf * 18 + e][IP]
