@@ -94,7 +94,8 @@ struct TankSet
 // reductions run a persistent grid over the set's work items.
 void bl_copy(const TankSet& b, int src, int dst, hipStream_t s);
 void bl_fill(const TankSet& b, int id, double v, hipStream_t s);
-void bl_ghost(const TankSet& b, int prog, int id, hipStream_t s);
+// most: operations of the largest program of the set's tanks
+void bl_ghost(const TankSet& b, int prog, int id, int most, hipStream_t s);
 void bl_hj_stage(const TankSet& b, int stage, int phi_s, int phi_n, int u, int v, int w, int out,
                  double cfac, hipStream_t s);
 void bl_reini_stage(const TankSet& b, int stage, int fs, int f0, int out, double F43, int fsf,
@@ -142,7 +143,7 @@ void bl_add32(const TankSet& b, int x, hipStream_t s);
 void bl_timestep(const TankSet& b, int u, int v, int w, double N47, int ini, hipStream_t s);
 // level-set benchmark: prescribed vortex velocity (benchmark_vortex3D) and the void
 // momentum_RK3 update of one component
-void bl_vortex_velocity(const TankSet& b, int comp, int id, double simtime, double DXM, hipStream_t s);
+void bl_vortex_velocity(const TankSet& b, double simtime, double DXM, hipStream_t s);
 void bl_void_rk3(const TankSet& b, int comp, int id, double Fv, hipStream_t s);
 // bicgstab_ijk / bicgstab_ijk_2D on each tank's explicit 7-diagonal operator (TankDev::m)
 // over the FLEXLOOP cells of var (1..3: the u / v / w grids, 4, 5: every cell), iterating

@@ -750,6 +750,13 @@ const TankHost* Engine::first_used() const
     return nullptr;
 }
 
+int Engine::most_ops(const TankSet& S, int prog) const
+{
+    int n = 0;
+    for(int p = 0; p < S.n; ++p) n = std::max(n, tanks[S.slot[p]].dev.gnops[prog]);
+    return n;
+}
+
 int Engine::ghost(int field, int kind, int gcv)
 {
     const int q = prog_index(kind, gcv);
@@ -757,7 +764,7 @@ int Engine::ghost(int field, int kind, int gcv)
     int rc;
     if((rc = sync_tables())) return rc;
     tbegin("ghost");
-    each([&](const TankSet& S) { bl_ghost(S, q, field, stream); });
+    each([&](const TankSet& S) { bl_ghost(S, q, field, most_ops(S, q), stream); });
     tend();
     return 0;
 }
@@ -862,8 +869,8 @@ int Engine::fluid_update_noalloc(int slot, double* vol2)
     const int q_ro = prog_index(4, 1);
     if(q_ro < 0) return fail(REEF_E_UNSUPPORTED, "ghost program (4, 1) not compiled");
     each([&](const TankSet& S) {
-        bl_ghost(S, q_ro, REEF_RO, stream);
-        bl_ghost(S, q_ro, REEF_VISC, stream);
+        bl_ghost(S, q_ro, REEF_RO, most_ops(S, q_ro), stream);
+        bl_ghost(S, q_ro, REEF_VISC, most_ops(S, q_ro), stream);
     });
     EHIP(hipStreamSynchronize(stream));
     return 0;
@@ -1933,15 +1940,12 @@ int Engine::vortex_step(double simtime)
     const reef_params* sp = shared();
     if(!t0 || !sp) return 0;
     const double grav[3] = {sp->W20, sp->W21, sp->W22};
-    for(int comp = 1; comp <= 3; ++comp)
-    {
-        if(comp == 2 && t0->hg.jdir == 0) continue;
-        const double Fv = 0.0 + (0.0 + grav[comp - 1] + 0.0 + 0.0) * 1.0;
-        each([&](const TankSet& S) { bl_void_rk3(S, comp, REEF_U + comp - 1, Fv, stream); });
-        if((rc = ghost(REEF_U + comp - 1, comp, 9 + comp))) return rc;
-    }
-    for(int comp = 1; comp <= 3; ++comp)
-        each([&](const TankSet& S) { bl_vortex_velocity(S, comp, REEF_U + comp - 1, simtime, t0->hg.DXM, stream); });
+    // The void momentum step: only w's.  u and v of every cell it updates, and the ghosts filled
+    // from them (u 10, v 11), are written again below by the prescribed field and its fills.
+    const double Fv = 0.0 + (0.0 + grav[2] + 0.0 + 0.0) * 1.0;
+    each([&](const TankSet& S) { bl_void_rk3(S, 3, REEF_W, Fv, stream); });
+    if((rc = ghost(REEF_W, 3, 12))) return rc;
+    each([&](const TankSet& S) { bl_vortex_velocity(S, simtime, t0->hg.DXM, stream); });
     // benchmark_vortex3D.cpp:98-100 fills u (10), v (11) and then v again with gcv 12; w's
     // ghosts keep the values of the void RK3 fill above.  Kept as the reference has it.
     if((rc = ghost(REEF_U, 1, 10))) return rc;

@@ -178,6 +178,8 @@ public:
 
     // ---- operations on every active tank
     int ghost(int field, int kind, int gcv);
+    // operations of the largest ghost program prog of a set's tanks
+    int most_ops(const TankSet& S, int prog) const;
     int convection(int ipol, int q, int u, int v, int w);
     // reini_RK3 pseudo steps with the ghost rule gcv of the level set (52 = gcval_phi for
     // F50 = 2; 50 = gcval_iniphi of the initial reinitialisation)
