@@ -35,7 +35,9 @@ typedef unsigned long long u64;
 constexpr int CG = CHIP_NT / NT;           // 256-thread groups
 static_assert(CG == 2, "groups of a block");
 constexpr unsigned ABORT = 0x80000000u;
-constexpr long WAIT_TICKS = 5000000;   // 50 ms of the 100 MHz wall clock
+// 500 ms of the 100 MHz wall clock: where a set has more blocks than the card has CUs, a tank's
+// blocks can be dispatched one tank's whole solve apart
+constexpr long WAIT_TICKS = 50000000;
 
 __device__ __forceinline__ void put_word(u64* p, u64 v)
 {
