@@ -25,6 +25,16 @@ static int check(int nx, int ny, int nz, int ty, int tz, int cpt, int ct)
     const TileShape s = make_shape(nx, ny, nz, ty, tz, cpt);
     const int NTH = 256, most = 2 * (ct / cpt);
     int used = 0;
+    {
+        // item_spread deals every item once
+        int nb = 0, b = 0;
+        std::vector<int> dealt(s.nitems, 0);
+        for(int l = 0; l < s.nitems; ++l)
+        {
+            const int it = item_spread(s, l);
+            CHECK(it >= 0 && it < s.nitems && !dealt[it]++);
+        }
+    }
     for(int nb = 1; nb <= 256 && nb <= s.nitems; nb *= 2)
     {
         int b = 0;
