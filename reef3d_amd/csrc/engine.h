@@ -66,7 +66,7 @@ struct TankHost
     TankDev dev{};                  // host copy of the table entry
     std::vector<void*> mem;         // pool blocks
     size_t bytes = 0;               // device bytes of the tank
-    std::vector<double> staging;
+    std::vector<double> staging;    // REEF_LAYOUT_REF transposition
     // on-chip solver (Engine::chip_plan): largest halo of a block with 2^q blocks, -1 unknown
     std::array<int, 9> chip_h;
     // iteration-level scheduling (start_steps / pump)
@@ -275,6 +275,19 @@ private:
     std::vector<int> solving_key_;
     std::vector<TankSet> solving_sets_;
 
+    // fields between host arrays and the device through pinned slots (move_rows)
+    struct PinnedSlot
+    {
+        double* p = nullptr;
+        hipEvent_t ev = nullptr;
+    };
+    static constexpr int XFER_LANES = 3, XFER_SLOTS = 2;   // copying threads, slots each
+    PinnedSlot xfer_[XFER_LANES][XFER_SLOTS];
+    size_t xfer_bytes_ = 0;                // of one slot
+    int xfer_lanes_ = 0;                   // lanes that have slots
+    bool have_slots(size_t bytes, int lanes);
+    void free_slots();
+    int move_rows(double* dev, const double* from, double* to, long rows, long X, long sx, bool& moved);
     int sync_tables();
     std::vector<TankSet> make_sets(const std::vector<int>& slots) const;
     int fail(int code, const std::string& m)

@@ -2719,6 +2719,22 @@ __global__ void kb_gather_states(TankSet b, BiState* __restrict__ dst)
     dst[b.slot[p]] = *T.st;
 }
 
+// Field rows between the device (sx doubles apart) and a pinned host slot (X apart), which the
+// kernel reads or writes over the bus, which bounds it (40 GB/s to the device).  The copy engine
+// was no faster for 2 MB and took 50 us more to start and to wait for.
+__global__ void __launch_bounds__(NT) kb_move_rows(double* __restrict__ dev, double* __restrict__ slot, long ndev, long X,
+                                                   long sx, int put)
+{
+    for(long e = (long)blockIdx.x * NT + threadIdx.x; e < ndev; e += (long)gridDim.x * NT)
+    {
+        const long r = (unsigned)e / (unsigned)sx, x = e - r * sx;   // a chunk has less than 2^32 doubles
+        if(put)
+            dev[e] = x < X ? slot[r * X + x] : 0.0;
+        else if(x < X)
+            slot[r * X + x] = dev[e];
+    }
+}
+
 // ------------------------------------------------------------------ level-set benchmark
 // benchmark_vortex3D::start (benchmark_vortex3D.cpp:67-96): the prescribed deformation velocity
 // at the face positions, at time simtime, of the three components.  The factors depend on one
@@ -2954,6 +2970,11 @@ static inline dim3 pgrid(const TankSet& b, int occ = OCC_FULL) { return pgrid_n(
 static inline dim3 pgrid_pw(const TankSet& b, int occ) { return pgrid_n(b.pw_items, occ); }
 static inline dim3 pgrid_direct(const TankSet& b, int occ) { return pgrid_n(b.nitems - b.pw_items, occ); }
 
+void bl_move_rows(double* dev, double* pinned, long ndev, long X, long sx, bool put, hipStream_t s)
+{
+    const unsigned blocks = (unsigned)std::min(1024L, (ndev + NT - 1) / NT);
+    hipLaunchKernelGGL(kb_move_rows, dim3(blocks), dim3(NT), 0, s, dev, pinned, ndev, X, sx, put ? 1 : 0);
+}
 void bl_copy(const TankSet& b, int src, int dst, hipStream_t s)
 {
     hipLaunchKernelGGL(kb_copy, tgrid(b), dim3(NT), 0, s, b, src, dst);
