@@ -70,15 +70,18 @@ sys.path.insert(0, ROOT)
 
 # algorithmic HBM bytes per interior cell of each solver kernel (FP64): arrays each
 # kernel must read or write once; stencil neighbours are served on chip
+# of a 3-D tank that is walked by row classes: rows of one density take the operator and the
+# Jacobi factor from tables of one axis each (about 9 % of the rows of the wave tank are mixed
+# and read them, 32 bytes per cell more)
 SOLVER_BYTES = {
-    "bicg_p": 48,   # r, p, v, aii in; p, ph out
-    "bicg_v": 48,   # ph, 3 face densities, r0 in; v out (|r|^2 comes from the x phase)
-    "bicg_t": 56,   # r, v, aii, 3 face densities in; t out
-    "bicg_x": 72,   # x, ph, r, v, aii, t, r0 in; x, r out
+    "bicg_p": 40,   # r, p, v in; p, ph out
+    "bicg_v": 24,   # ph, r0 in; v out (|r|^2 comes from the x phase)
+    "bicg_t": 24,   # r, v in; t out
+    "bicg_x": 64,   # x, ph, r, v, t, r0 in; x, r out
 }
 # the same kernels of the FP32 inner solve of the mixed-precision projection
-# mix_v: the FP32 p update fused with v = A ph (r, p, v, aii, 3 conductances, r0 in; v, p, ph out)
-SOLVER_BYTES.update({"mix_v": 44, "bicg32_t": 28, "bicg32_x": 36})
+# mix_v: the FP32 p update fused with v = A aii p (r, p, v, aii, r0 in; v, p out)
+SOLVER_BYTES.update({"mix_v": 28, "bicg32_t": 16, "bicg32_x": 32})
 HBM_PEAK_GBS = 8000.0
 TIMED_FAMILIES = ("bicg_init", "bicg_p", "bicg_v", "bicg_t", "bicg_x", "mix_init", "mix_v",
                   "bicg32_t", "bicg32_x", "mix_ru", "coef32", "add32", "hj", "reini", "momentum", "ghost",
@@ -199,7 +202,7 @@ STENCIL_BYTES = {
 # the WENO stencils are bound by VALU issue and load latency, not by HBM: FP64 flops per
 # cell (add + mul + 2 fma + trans) counted with SQ_INSTS_VALU_*_F64 on the 512x64x128 tank
 # (profiles/wave_tank_512x64x128_stencil_valu.md); the same kernels run here
-STENCIL_FP64_FLOPS = {"hj": 554.0, "reini": 733.0, "momentum": 798.0}
+STENCIL_FP64_FLOPS = {"hj": 549.0, "reini": 679.0, "momentum": 879.0}
 FP64_PEAK_TFLOPS = 78.6
 MOMENTUM_BYTES = (56 + 64 + 64) / 3.0   # q_in, u, v, w, p, phi [, q_old] in; q out
 
@@ -245,10 +248,10 @@ def hbm_copy(nbytes=1 << 30, reps=5):
 
 
 # kernel name -> the family of the bench's SOLVER_BYTES (the traffic tables of the profiles)
-TRAFFIC_KERNELS = (("kb_bicg_p<double>", "bicg_p"), ("kb_bicg_v<double, true>", "bicg_v"),
-                   ("kb_bicg_t<double, true>", "bicg_t"), ("kb_bicg_x<double>", "bicg_x"),
-                   ("kb_mix_v<true>", "mix_v"), ("kb_bicg_t<float, true>", "bicg32_t"),
-                   ("kb_bicg_x<float>", "bicg32_x"), ("kb_hj_stage", "hj"), ("kb_reini_stage", "reini"))
+TRAFFIC_KERNELS = (("kb_class_p", "bicg_p"), ("kb_class_v", "bicg_v"),
+                   ("kb_bicg_t<double, true>", "bicg_t"), ("kb_class_x<double>", "bicg_x"),
+                   ("kb_bicg_x<double>", "bicg_x"), ("kb_mix_v<true>", "mix_v"),
+                   ("kb_bicg_t<float, true>", "bicg32_t"), ("kb_class_x<float>", "bicg32_x"), ("kb_hj_stage", "hj"), ("kb_reini_stage", "reini"))
 
 
 def traffic_tables(fetch_dir, write_dir, cells=512 * 64 * 128, out_dir=None):

@@ -415,7 +415,7 @@ __device__ __forceinline__ CouplingV<float> coupling_of(const DevGrid& g, const 
 }
 
 // The grid factors of the couplings along one axis at index ix: DP(ix), DN(ix), DP(ix-1)
-// for the FP64 operator, the FP32 1/DN(ix) for the FP32 one.  The plane walk loads the
+// for the FP64 operator, the FP32 1/DN(ix) for the FP32 one.  The class walk loads the
 // x and y factors once per column and the z factors with each plane.
 template<class Op>
 struct AxisFactor;

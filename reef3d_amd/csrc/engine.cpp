@@ -116,8 +116,8 @@ void DevicePool::free(void* p)
 }
 
 // ------------------------------------------------------------------ plan
-// 64 x 4 x 1 tiles for 3-D tanks (plane walk of the solver), 64 x 1 x 4 for 2-D x-z tanks.
-// A 3-D tank gets about one work item per block of the plane-walk grid (a large tank's
+// 64 x 4 x 1 tiles for 3-D tanks (class walk of the solver), 64 x 1 x 4 for 2-D x-z tanks.
+// A 3-D tank gets about one work item per block of the class-walk grid (a large tank's
 // items are columns of several planes); a 2-D tank about 2048 items.  The plan is a
 // function of the tank alone, so its reductions are the same in any batch.
 TileShape plan_shape(const HostGrid& h, int cpt_override)
@@ -578,7 +578,7 @@ int Engine::sync_tables()
 // the launch sets of the given slots, at most SET_MAX tanks each
 std::vector<TankSet> Engine::make_sets(const std::vector<int>& slots_in) const
 {
-    // plane-walked tanks first: their items are a prefix of each set's items, so the
+    // class-walked tanks first: their items are a prefix of each set's items, so the
     // launches that take one kind of tank spread that kind's items over every XCD group
     auto pw = [&](int q) {
         const TankHost& t = tanks[q];
@@ -674,7 +674,8 @@ bool Engine::have_slots(size_t bytes, int lanes)
 // the bus while another is copied by the host; fields of 4 MB and more take up to three host
 // threads, since the first touch of the caller's pages costs more than the bus.  To the device
 // and back, before (one pageable copy of a staging array) and after: 154 kB 126 + 141
-// -> 22 + 21 us, 40 MB 4.2 + 5.4 -> 1.0 + 1.7 ms.  More threads or smaller chunks gave nothing.
+// -> 22 + 21 us, 40 MB 4.2 + 5.4 -> 1.0 + 1.7 ms (six threads
+// and chunks of 512 kB: 1.3 + 1.4 ms).
 // moved: false if there is no page-locked memory (nothing was done).
 int Engine::move_rows(double* dev, const double* from, double* to, long rows, long X, long sx, bool& moved)
 {

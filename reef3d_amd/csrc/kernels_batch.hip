@@ -75,7 +75,7 @@ __device__ __forceinline__ ItemIter set_items_spread(const TankSet& b)
     return it;
 }
 
-// the items of the plane-walked tanks (a prefix of the set) or of the others
+// the items of the class-walked tanks (a prefix of the set) or of the others
 template<bool PW>
 __device__ __forceinline__ ItemIter set_items_of(const TankSet& b)
 {
@@ -668,7 +668,7 @@ __global__ void __launch_bounds__(NT) kb_correct(TankSet b, double rw, double ra
 
 // ------------------------------------------------------------------ BiCGStab
 // Occupancy of the persistent solver kernels (waves per SIMD = blocks per CU): 8 for the
-// plane walk and the FP32 / elementwise kernels; 5 for the kernels that apply the FP64
+// FP32 / elementwise kernels; 5 for the kernels that apply the FP64
 // operator cell by cell (about 100 registers), whose grids are sized to match.
 constexpr int OCC_FULL = 8, OCC_A64 = 5;
 // class walk: 4 blocks per CU (the default plan of a 3-D tank gives it one work item per
@@ -697,7 +697,7 @@ struct NoEpi
 };
 
 // ------------------------------------------------------------------ class walk (3-D tanks)
-// Plane walk of the 3-D stencil phases (tanks with 64 x 4 x 1 tiles): a block walks up the k
+// Class walk of the 3-D stencil phases (tanks with 64 x 4 x 1 tiles): a block walks up the k
 // planes of its item's column; the operand of plane k (rows j-1 .. j+4, columns i-1 .. i+64)
 // sits in a double-buffered LDS plane (one barrier per plane), planes k-1 and k+1 of the own
 // cell in registers.
@@ -1113,7 +1113,7 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
     }
 }
 
-// Elementwise pass over an item of a plane-walked tank with aii from the row classes (mixed
+// Elementwise pass over an item of a class-walked tank with aii from the row classes (mixed
 // rows load it): load(u, c) and use(u, c, aii) for each cell, U tiles at a time so that their
 // loads are in flight together; the cells of a thread come in tile order.
 template<class V, int U, class Load, class Use>
@@ -1255,7 +1255,7 @@ __device__ __forceinline__ void row_walk(const DevGrid& g, const Op& op, const T
     }
 }
 
-__device__ __forceinline__ bool plane_walk_ok(CTank& T)
+__device__ __forceinline__ bool class_walk_ok(CTank& T)
 {
     return T.g.jdir == 1 && T.shape.ty == TY && T.shape.tz == 1;
 }
@@ -1350,7 +1350,7 @@ __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int r
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 2 || plane_walk_ok(T))
+        if(st->done || st->mode == 2 || class_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1384,7 +1384,7 @@ __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int r
     }
 }
 
-// kb_bicg_p of the plane-walked tanks, aii from the row classes: 40 bytes per cell (r, p, v / p,
+// kb_bicg_p of the class-walked tanks, aii from the row classes: 40 bytes per cell (r, p, v / p,
 // ph)
 __global__ void __launch_bounds__(NT, OCC_CX) kb_class_p(TankSet b, int x, int rhs)
 {
@@ -1448,7 +1448,7 @@ __global__ void kb_fin_p(TankSet b)
 // v = A ph; sigma = (v, r0), |v|^2 (bicgstab_ijk.cpp:151-160).  |r|^2 of the same loop is
 // the square norm of the residual the x phase (or the restart) has just formed and summed:
 // kb_fin_v takes it from the state instead of reading r again here.
-// Tanks without a plane walk; kb_class_v takes the others.
+// Tanks without a class walk; kb_class_v takes the others.
 template<class V>
 __global__ void __launch_bounds__(NT, sizeof(V) == 4 ? OCC_FULL : OCC_A64) kb_bicg_v(TankSet b, int x, int rhs)
 {
@@ -1458,7 +1458,7 @@ __global__ void __launch_bounds__(NT, sizeof(V) == 4 ? OCC_FULL : OCC_A64) kb_bi
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 3 || plane_walk_ok(T))
+        if(st->done || st->mode == 3 || class_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1514,7 +1514,7 @@ __global__ void __launch_bounds__(NT, sizeof(V) == 4 ? OCC_FULL : OCC_A64) kb_bi
     }
 }
 
-// v = A ph of the plane-walked tanks (24 bytes per cell: ph, r0 / v).  The p update stays a
+// v = A ph of the class-walked tanks (24 bytes per cell: ph, r0 / v).  The p update stays a
 // pass of its own (kb_class_p): fused into this walk, as the FP32 v phase has it, the FP64
 // operand needs r, p, v and aii at every stencil point, and the walk spills at 4 blocks per CU.
 __global__ void __launch_bounds__(NT, OCC_PW) kb_class_v(TankSet b, int x, int rhs)
@@ -1525,7 +1525,7 @@ __global__ void __launch_bounds__(NT, OCC_PW) kb_class_v(TankSet b, int x, int r
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 3 || !plane_walk_ok(T))
+        if(st->done || st->mode == 3 || !class_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1576,7 +1576,7 @@ __global__ void __launch_bounds__(NT, PW ? OCC_PW : OCC_FULL) kb_mix_v(TankSet b
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || plane_walk_ok(T) != PW)
+        if(st->done || class_walk_ok(T) != PW)
         {
             skip_tank(q, b);
             continue;
@@ -1771,7 +1771,7 @@ __global__ void __launch_bounds__(NT, PW ? OCC_PW : (sizeof(V) == 4 ? OCC_FULL :
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 1 || st->mode == 3 || plane_walk_ok(T) != PW)
+        if(st->done || st->mode == 1 || st->mode == 3 || class_walk_ok(T) != PW)
         {
             skip_tank(q, b);
             continue;
@@ -1882,7 +1882,7 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 1 || st->mode == 3 || plane_walk_ok(T))
+        if(st->done || st->mode == 1 || st->mode == 3 || class_walk_ok(T))
         {
             skip_tank(q, b);
             continue;
@@ -1929,7 +1929,7 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
     }
 }
 
-// kb_bicg_x of the plane-walked tanks, aii from the row classes: 64 bytes per cell in FP64 (x,
+// kb_bicg_x of the class-walked tanks, aii from the row classes: 64 bytes per cell in FP64 (x,
 // ph, r, v, t, r0 / x, r); FP32 forms ph = aii p from the current p
 template<class V>
 __global__ void __launch_bounds__(NT, OCC_CX) kb_class_x(TankSet b, int x, int rhs)
@@ -2966,7 +2966,7 @@ static inline dim3 pgrid_n(int nitems, int occ)
     return dim3((unsigned)std::max(8, std::min(256 * occ, (nitems + 7) / 8 * 8)));
 }
 static inline dim3 pgrid(const TankSet& b, int occ = OCC_FULL) { return pgrid_n(b.nitems, occ); }
-// the launches of one kind of tank (set_items_of): plane-walked or the others
+// the launches of one kind of tank (set_items_of): class-walked or the others
 static inline dim3 pgrid_pw(const TankSet& b, int occ) { return pgrid_n(b.pw_items, occ); }
 static inline dim3 pgrid_direct(const TankSet& b, int occ) { return pgrid_n(b.nitems - b.pw_items, occ); }
 

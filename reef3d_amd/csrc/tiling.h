@@ -24,7 +24,7 @@ namespace reef {
 
 constexpr int TILE_X = 64;
 
-// blocks per CU of the plane-walk solver kernels (256 CUs)
+// blocks per CU of the class-walk solver kernels (256 CUs)
 #define REEF_OCC_PW 4
 constexpr int PW_BLOCKS = 256 * REEF_OCC_PW;
 
@@ -40,7 +40,7 @@ struct TileShape
     // tiles whose columns split into whole items (nbz % cpt == 0, more than one chunk).
     // Item position l then stands for item (l % columns) * zslab + l / columns, so one XCD
     // group's contiguous share of the positions is a z-slab of every column: the rows of
-    // the y-neighbour tiles a plane walk stages in its halo belong to blocks of the same
+    // the y-neighbour tiles a class walk stages in its halo belong to blocks of the same
     // XCD walking the same planes at the same time, and are served by that XCD's L2.
     // Items and their reduction slots are unchanged, only the block that walks them is.
     int zslab;
