@@ -96,7 +96,7 @@ void bl_copy(const TankSet& b, int src, int dst, hipStream_t s);
 void bl_fill(const TankSet& b, int id, double v, hipStream_t s);
 // ndev doubles of device rows of sx from (put: to, with 0 in the padding) compact rows of X in
 // pinned host memory
-void bl_move_rows(double* dev, double* pinned, long ndev, long X, long sx, bool put, hipStream_t s);
+hipError_t bl_move_rows(double* dev, double* pinned, long ndev, long X, long sx, bool put, hipStream_t s);
 // most: operations of the largest program of the set's tanks
 void bl_ghost(const TankSet& b, int prog, int id, int most, hipStream_t s);
 void bl_hj_stage(const TankSet& b, int stage, int phi_s, int phi_n, int u, int v, int w, int out,

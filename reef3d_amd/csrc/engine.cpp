@@ -673,9 +673,8 @@ bool Engine::have_slots(size_t bytes, int lanes)
 // of at most 2 MB through pinned slots that a kernel reads or writes, so that one chunk crosses
 // the bus while another is copied by the host; fields of 4 MB and more take up to three host
 // threads, since the first touch of the caller's pages costs more than the bus.  To the device
-// and back, before (one pageable copy of a staging array) and after: 154 kB 126 + 141
-// -> 22 + 21 us, 40 MB 4.2 + 5.4 -> 1.0 + 1.7 ms (six threads
-// and chunks of 512 kB: 1.3 + 1.4 ms).
+// and back, before (one pageable copy of a staging array) and after: 154 kB 126 + 141 -> 22 +
+// 21 us, 40 MB 4.2 + 5.4 -> 1.0 + 1.7 ms (six threads and chunks of 512 kB: 1.3 + 1.4 ms).
 // moved: false if there is no page-locked memory (nothing was done).
 int Engine::move_rows(double* dev, const double* from, double* to, long rows, long X, long sx, bool& moved)
 {
@@ -695,8 +694,7 @@ int Engine::move_rows(double* dev, const double* from, double* to, long rows, lo
             const long r0 = c * per, n = std::min(per, rows - r0);
             // the last row ends with its X doubles: the padding after it is not the field's
             const long ndev = (n - 1) * sx + (r0 + n == rows ? X : sx);
-            bl_move_rows(dev + r0 * sx, s.p, ndev, X, sx, from != nullptr, stream);
-            hipError_t q = hipGetLastError();
+            hipError_t q = bl_move_rows(dev + r0 * sx, s.p, ndev, X, sx, from != nullptr, stream);
             if(q == hipSuccess) q = hipEventRecord(s.ev, stream);
             return q;
         };

@@ -2970,10 +2970,12 @@ static inline dim3 pgrid(const TankSet& b, int occ = OCC_FULL) { return pgrid_n(
 static inline dim3 pgrid_pw(const TankSet& b, int occ) { return pgrid_n(b.pw_items, occ); }
 static inline dim3 pgrid_direct(const TankSet& b, int occ) { return pgrid_n(b.nitems - b.pw_items, occ); }
 
-void bl_move_rows(double* dev, double* pinned, long ndev, long X, long sx, bool put, hipStream_t s)
+hipError_t bl_move_rows(double* dev, double* pinned, long ndev, long X, long sx, bool put, hipStream_t s)
 {
     const unsigned blocks = (unsigned)std::min(1024L, (ndev + NT - 1) / NT);
-    hipLaunchKernelGGL(kb_move_rows, dim3(blocks), dim3(NT), 0, s, dev, pinned, ndev, X, sx, put ? 1 : 0);
+    int to_dev = put ? 1 : 0;
+    void* args[] = {&dev, &pinned, &ndev, &X, &sx, &to_dev};
+    return hipLaunchKernel(reinterpret_cast<const void*>(kb_move_rows), dim3(blocks), dim3(NT), args, 0, s);
 }
 void bl_copy(const TankSet& b, int src, int dst, hipStream_t s)
 {
