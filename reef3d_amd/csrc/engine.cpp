@@ -568,6 +568,7 @@ int Engine::sync_tables()
     for(int m = 0; m < 2; ++m) all_chip_[m] = chip_plan(act, m != 0);
     solving_key_.clear();
     solving_sets_.clear();
+    solving_chip_ = ChipPlan();
     last_state.resize(nslot, BiState{});
     step_iters.resize(nslot, 0);
     vol.resize(2 * (size_t)nslot, 0.0);
@@ -1109,7 +1110,6 @@ int Engine::chip_blocks(TankHost& t, int per_block, bool mixed) const
 Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
 {
     ChipPlan P;
-    P.stream_all = true;
     if(chip_off_) return P;
     static const double US[2][3] = {{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}};
     struct Tank
@@ -1264,7 +1264,7 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
 int Engine::enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap)
 {
     const int m = kind == SOLVE_MIXED;
-    ChipPlan* P = cur_ == &all_ ? &all_chip_[m] : cur_ == &solving_sets_ ? &solving_chip_[m] : nullptr;
+    ChipPlan* P = cur_ == &all_ ? &all_chip_[m] : cur_ == &solving_sets_ && m == solving_mixed_ ? &solving_chip_ : nullptr;
     if(P && !chip_off_ && !P->stream_all)
     {
         int rc = chip_launch(*P, kind, x, rhs, chip_cap);
@@ -1990,11 +1990,12 @@ int Engine::pump(std::vector<int>& stepped)
         if(tanks[q].used && solving_pc(tanks[q].pc)) solving.push_back((int)q);
     if(!solving.empty())
     {
-        if(solving != solving_key_)
+        if(solving != solving_key_ || (int)mixed != solving_mixed_)
         {
             solving_sets_ = make_sets(solving);
-            solving_chip_[mixed] = chip_plan(solving, mixed);
+            solving_chip_ = chip_plan(solving, mixed);
             solving_key_ = solving;
+            solving_mixed_ = mixed;
         }
         const int ring = (int)(batch_no_++ & 1);
         cur_ = &solving_sets_;

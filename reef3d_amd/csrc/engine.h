@@ -272,7 +272,8 @@ private:
         std::vector<std::pair<int, int>> members;   // (slot, seq)
     };
     std::deque<Inflight> inflight_;
-    std::vector<int> solving_key_;
+    std::vector<int> solving_key_;         // slots and precision solving_sets_ and solving_chip_
+    int solving_mixed_ = 0;                // are of
     std::vector<TankSet> solving_sets_;
 
     // fields between host arrays and the device through pinned slots (move_rows)
@@ -326,9 +327,10 @@ private:
         std::vector<ChipSet> launches;
         std::vector<int> rest;              // slots that stream
         std::vector<TankSet> rest_sets;
-        bool stream_all = false;            // every slot streams: the caller's sets are used
+        bool stream_all = true;             // every slot streams: the caller's sets are used
     };
-    ChipPlan all_chip_[2], solving_chip_[2];   // [1]: mixed precision (FP32 vectors)
+    ChipPlan all_chip_[2];                  // of all_; [1]: mixed precision (FP32 vectors)
+    ChipPlan solving_chip_;                 // of solving_sets_, in the precision solving_mixed_
     size_t chip_tiles_ = 0;                 // tile slots the workspace holds
     // accumulator words, commit words, then the halo words of chip_tiles_ tile slots
     unsigned long long* d_chip_ = nullptr;

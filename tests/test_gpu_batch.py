@@ -211,6 +211,56 @@ def test_scheduled_run_identical_to_lockstep(precision, graphs):
             assert np.array_equal(sched[q][n], lock[q][n]), f"tank {q} {n}: scheduled != lockstep"
 
 
+# more than 2048 tiles, which the streaming phases solve: 3-D (class walk) and 2-D
+LARGE = [_tank(224, 40, 96, 0.03, 1.7, 0.05, 2.0, 0.004, 1), _tank(2049, 1, 256, 0.02, 3.0, 0.1, 3.0, 0.004, 0)]
+
+
+@pytest.mark.parametrize("tanks", [TANKS[1:2], LARGE[:1], TANKS[1:3] + LARGE[1:]], ids=["small", "large", "several"])
+@pytest.mark.parametrize("added", [0, 1, 8])
+def test_run_after_a_change_of_precision(tanks, added):
+    """A scheduled run in another precision than the run before, and back, with tanks added in
+    between (8 more outgrow the device's tank table): the bits and the iteration counts of the
+    same steps of each tank alone, in lockstep.  The same tanks solve in each run, so a launch
+    plan kept for them from the other precision would be used again."""
+    from reef3d_amd import Batch
+    runs = ["fp64", "mixed", "fp64", "mixed"]
+    more = [TANKS[2 + q % 2] for q in range(added)]
+    B = Batch()
+    print(len(tanks), added, flush=True)
+    ids = [B.add(**kw) for kw, _ in tanks]
+    for tid, (kw, f) in zip(ids, tanks):
+        _initial(B, tid, kw, f)
+    _prepare(B)
+    its = []
+    for step, precision in enumerate(runs):
+        if step == 2 and more:
+            new = [B.add(**kw) for kw, _ in more]
+            for tid, (kw, f) in zip(new, more):
+                _initial(B, tid, kw, f)
+            B.set_active(new)
+            _prepare(B)
+            B.set_active()
+            ids += new
+        B.solver_config(precision)
+        it = B.run(1)
+        its.append([it[t] for t in ids])
+    got = [{n: B.get(t, n) for n in FIELDS} for t in ids]
+    B.close()
+    for q, (kw, f) in enumerate((tanks + more)[:len(tanks) + 2]):
+        first = 0 if q < len(tanks) else 2
+        A = Batch()
+        t = A.add(**kw)
+        _initial(A, t, kw, f)
+        _prepare(A)
+        for step in range(first, len(runs)):
+            A.solver_config(runs[step])
+            it, _ = A.fc3_step()
+            assert its[step][q] == it[t] > 0, f"tank {q} run {step}"
+        for n in FIELDS:
+            assert np.array_equal(got[q][n], A.get(t, n)), f"tank {q} {n}: scheduled != lockstep"
+        A.close()
+
+
 def test_batch_refuses_differing_shared_parameters():
     """Only dt and F45 may differ between the tanks of a batch; the shared values stay
     those of the first tank added to the empty batch, also after that tank is removed."""
