@@ -142,7 +142,11 @@ int reef_ctx_create(const reef_grid_desc* grid, const reef_params* prm, reef_ctx
  * (eddyv 0); not with N48 = 1, which the reference steps with another time-step class;
  * 2 = idiff2_FS, the implicit viscous solves (idiff2_FSu.cpp:40-278, var 1..3, stop "N43",
  * default 1e-5, ini.cpp:589).  "simtime": the simulation time of the wave generator
- * (reef_wave_set; p->simtime).  Other keys: REEF_E_UNSUPPORTED. */
+ * (reef_wave_set; p->simtime).  "onchip" (no counterpart in the reference): most MiB of
+ * device memory, beside the tanks', for the solves that run in one launch with their vectors
+ * on the chip (tanks of up to 2048 tiles; default 1024, at most 100 are used); where they do
+ * not fit, or with 0, those solves run phase by phase like a large tank's, with identical
+ * results.  Other keys: REEF_E_UNSUPPORTED. */
 int reef_set_control(reef_ctx* ctx, const char* key, double value);
 void reef_ctx_destroy(reef_ctx* ctx);
 const char* reef_last_error(void);
@@ -332,7 +336,8 @@ int reef_batch_put(reef_batch* b, int tank, int field_id, const double* host, in
 int reef_batch_get(reef_batch* b, int tank, int field_id, double* host, int layout);
 int reef_batch_ghost_fill(reef_batch* b, int field_id, int kind, int gcv);
 int reef_batch_fluid_update(reef_batch* b);
-/* the keys of reef_set_control ("F49", "graphs", "N48", "N47", "D20") for every tank of the batch */
+/* the keys of reef_set_control ("F49", "graphs", "N48", "N47", "D20", "N43", "simtime",
+ * "onchip") for every tank of the batch */
 int reef_batch_control(reef_batch* b, const char* key, double value);
 int reef_batch_solver_config(reef_batch* b, int precision, double delta);
 /* Tile plans per size bucket (no counterpart in the reference).  A bucket is (jdir,

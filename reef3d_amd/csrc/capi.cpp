@@ -121,6 +121,12 @@ int control(Engine& e, const char* key, double value)
         e.n47 = value;
         return 0;
     }
+    if(std::strcmp(key, "onchip") == 0)
+    {
+        if(!(value >= 0.0)) return fail(REEF_E_ARG, "onchip must be >= 0");
+        e.set_onchip(value);
+        return 0;
+    }
     return fail(REEF_E_UNSUPPORTED, std::string("control key not supported: ") + key);
 }
 

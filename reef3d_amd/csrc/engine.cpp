@@ -1110,7 +1110,6 @@ int Engine::chip_blocks(TankHost& t, int per_block, bool mixed) const
 Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
 {
     ChipPlan P;
-    if(chip_off_) return P;
     static const double US[2][3] = {{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}};
     struct Tank
     {
@@ -1187,36 +1186,53 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
     return P;
 }
 
-// workspace of the on-chip solver for at least `tiles` tile slots
-int Engine::chip_alloc(size_t tiles)
+// The workspace of the plan's launches: false where there is no memory for it (or it is larger
+// than onchip_mib), no event, or the device does not take the kernels' LDS; the engine then
+// streams.  It is not the tanks', so it is outside the pool and its budget.
+bool Engine::chip_ready(const ChipPlan& P)
 {
-    if(d_chip_ && tiles <= chip_tiles_) return 0;
-    const int rc = chip_prepare();
-    if(rc) return fail(rc, "on-chip solver: dynamic LDS limit not accepted");
-    if(!chip_ev_) EHIP(hipEventCreateWithFlags(&chip_ev_, hipEventDisableTiming));
-    if(d_chip_)
-    {
-        EHIP(hipStreamSynchronize(stream));
-        (void)hipFree(d_chip_);
-        d_chip_ = nullptr;
-    }
+    size_t tiles = 0;
+    for(const ChipSet& S : P.launches) tiles = std::max(tiles, (size_t)S.blk0[S.n] * 2 * S.ct);
+    if(d_chip_ && tiles <= chip_tiles_) return true;
+    chip_off_ = true;
     tiles = std::max(tiles, (size_t)2048);
     const size_t bytes = ((size_t)CHIP_TANKS * CHIP_ACC_WORDS + 3 * tiles * 512) * 8 + CHIP_CTL * sizeof(unsigned);
-    EHIP(hipMalloc(&d_chip_, bytes));
+    if((double)bytes > onchip_mib * 1048576.0) return false;
+    unsigned long long* mem = nullptr;
+    if(chip_prepare() || (!chip_ev_ && hipEventCreateWithFlags(&chip_ev_, hipEventDisableTiming) != hipSuccess) ||
+       hipMalloc(&mem, bytes) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return false;
+    }
+    if(d_chip_)
+    {
+        (void)hipStreamSynchronize(stream);
+        (void)hipFree(d_chip_);
+    }
+    d_chip_ = mem;
     chip_tiles_ = tiles;
     chip_epoch_ = 1;
     chip_ctl_ = 0;
-    EHIP(hipMemsetAsync(d_chip_, 0, bytes, stream));
-    return 0;
+    if(hipMemsetAsync(d_chip_, 0, bytes, stream) != hipSuccess) return false;
+    chip_off_ = false;
+    return true;
+}
+
+void Engine::set_onchip(double mib)
+{
+    onchip_mib = mib;
+    chip_off_ = !(mib > 0.0);
+    if(!d_chip_) return;
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(d_chip_);
+    d_chip_ = nullptr;
+    chip_tiles_ = 0;
 }
 
 // the on-chip launches of the plan, each up to cap iterations
 int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
 {
-    int rc;
-    size_t tiles = 0;
-    for(const ChipSet& S : P.launches) tiles = std::max(tiles, (size_t)S.blk0[S.n] * 2 * S.ct);
-    if((rc = chip_alloc(tiles))) return rc;
     unsigned* ctl = (unsigned*)(d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS);
     unsigned long long* halo = d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS + CHIP_CTL / 2;
     int dev = 0;
@@ -1265,7 +1281,7 @@ int Engine::enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap
 {
     const int m = kind == SOLVE_MIXED;
     ChipPlan* P = cur_ == &all_ ? &all_chip_[m] : cur_ == &solving_sets_ && m == solving_mixed_ ? &solving_chip_ : nullptr;
-    if(P && !chip_off_ && !P->stream_all)
+    if(P && !chip_off_ && !P->stream_all && chip_ready(*P))
     {
         int rc = chip_launch(*P, kind, x, rhs, chip_cap);
         if(rc || P->rest.empty()) return rc;

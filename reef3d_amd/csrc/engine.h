@@ -123,6 +123,9 @@ public:
     // timing is on.
     bool graphs = false;
     void drop_graphs();
+    // most device memory, in MiB, for the workspace of the on-chip solver; 0: every solve streams
+    double onchip_mib = 1024.0;
+    void set_onchip(double mib);
     // tile plans per size bucket (jdir, floor(log2(nx ny nz))): tile rows ty x tz and
     // chunk length cpt; a bucket without an entry uses the default plan.  A tank takes the
     // plan of its bucket when it is added (and when its bucket's plan is set), so its
@@ -321,7 +324,7 @@ private:
     // On-chip solves (kernels_chip.hip).  chip_plan splits slots into launches of the on-chip
     // solver and the tanks that stay with the streaming phases; the plan of the current sets is
     // kept with them.  The workspace belongs to the engine's stream: launches of one engine
-    // follow each other, those of another engine of the process wait for them (chip_order).
+    // follow each other, those of another engine of the process wait for them (chip_launch).
     struct ChipPlan
     {
         std::vector<ChipSet> launches;
@@ -336,11 +339,13 @@ private:
     unsigned long long* d_chip_ = nullptr;
     unsigned chip_epoch_ = 0;
     int chip_ctl_ = 0;                      // next unused commit word
-    bool chip_off_ = false;                 // a launch gave up waiting: another process shares the GPU
+    // no on-chip launches: a wait ran out (another process shares the GPU), there is no workspace,
+    // or onchip_mib is 0
+    bool chip_off_ = false;
     hipEvent_t chip_ev_ = nullptr;
     int chip_blocks(TankHost& t, int per_block, bool mixed) const;
     ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);
-    int chip_alloc(size_t tiles);
+    bool chip_ready(const ChipPlan& P);
     int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);
     int enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap);
     int stream_iterations(int kind, int x, int rhs, int iters, bool lockstep);

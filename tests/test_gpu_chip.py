@@ -66,3 +66,23 @@ def test_iterations_beyond_one_launch():
         assert n == 1500
         xs.append(D.get("work0"))
     assert np.isfinite(xs[0]).all() and np.array_equal(xs[0], xs[1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_a_solve_streams_where_there_is_no_workspace(precision):
+    """A limit below the workspace (25 MiB at the least): the solve runs by the streaming phases,
+    with the same bits, and on chip again once the limit allows it."""
+    _, D, _, _ = _system(65, 5, 33, 1, seed=21)
+    solve = D.solver if precision == "fp64" else D.solver_mixed
+    D.timing(True)
+    out = []
+    for mib, launches in ((1024, 1), (1, 0), (0, 0), (1024, 1)):
+        D.set_control("onchip", mib)
+        D.timing_reset()
+        D.zero("work0")
+        print(precision, mib, flush=True)
+        r = solve("work0", "work1", -TOL, 20000)
+        assert min(D.timing_get("chip")[1], 1) == launches
+        out.append((r, D.get("work0")))
+    for r, x in out[1:]:
+        assert r == out[0][0] and np.array_equal(x, out[0][1])
