@@ -127,6 +127,12 @@ int control(Engine& e, const char* key, double value)
         e.set_onchip(value);
         return 0;
     }
+    if(std::strcmp(key, "onchip_wait") == 0)
+    {
+        if(!(value >= 0.0)) return fail(REEF_E_ARG, "onchip_wait must be >= 0");
+        e.set_onchip_wait(value);
+        return 0;
+    }
     return fail(REEF_E_UNSUPPORTED, std::string("control key not supported: ") + key);
 }
 

@@ -1219,6 +1219,26 @@ bool Engine::chip_ready(const ChipPlan& P)
     return true;
 }
 
+void Engine::set_onchip_wait(double seconds)
+{
+    onchip_wait = seconds;
+    chip_pause_ = 0;
+    chip_next_pause_ = CHIP_PAUSE;
+    chip_heard_ = chip_number_;
+}
+
+void Engine::chip_tick()
+{
+    if(chip_pause_ > 0 && --chip_pause_ == 0) chip_heard_ = chip_number_;
+}
+
+void Engine::chip_heard(const BiState& st)
+{
+    if(st.chip_fail <= chip_heard_ || chip_pause_ > 0) return;
+    chip_pause_ = chip_next_pause_;   // the solve goes on streaming
+    chip_next_pause_ = std::min(2 * chip_next_pause_, 64 * CHIP_PAUSE);
+}
+
 void Engine::set_onchip(double mib)
 {
     onchip_mib = mib;
@@ -1237,6 +1257,12 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
     unsigned long long* halo = d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS + CHIP_CTL / 2;
     int dev = 0;
     EHIP(hipGetDevice(&dev));
+    if(wall_khz_ == 0)
+    {
+        int khz = 0;
+        EHIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+        wall_khz_ = std::max(khz, 1);
+    }
     std::lock_guard<std::mutex> lk(g_chip_mu);
     auto& last = g_chip_last[dev];
     if(last.first && last.first != this) EHIP(hipStreamWaitEvent(stream, last.second, 0));
@@ -1261,6 +1287,8 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
         S.ctl = ctl + chip_ctl_;
         S.epoch = chip_epoch_;
         S.cap = cap;
+        S.wait = onchip_wait > 0.0 ? std::max(1L, (long)(std::min(onchip_wait, 1.0e6) * 1000.0 * (double)wall_khz_)) : 0;
+        S.number = ++chip_number_;
         tbegin("chip");
         bl_chip_solve(S, kind, x, rhs, stream);
         tend();
@@ -1281,7 +1309,7 @@ int Engine::enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap
 {
     const int m = kind == SOLVE_MIXED;
     ChipPlan* P = cur_ == &all_ ? &all_chip_[m] : cur_ == &solving_sets_ && m == solving_mixed_ ? &solving_chip_ : nullptr;
-    if(P && !chip_off_ && !P->stream_all && chip_ready(*P))
+    if(P && chip_on() && !P->stream_all && chip_ready(*P))
     {
         int rc = chip_launch(*P, kind, x, rhs, chip_cap);
         if(rc || P->rest.empty()) return rc;
@@ -1378,9 +1406,10 @@ int Engine::run_iterations(int kind, int x, int rhs, int maxiter)
     for(const TankSet& S : *cur_)
         for(int p = 0; p < S.n; ++p) members.push_back(S.slot[p]);
     int rc;
+    chip_tick();
     // an on-chip batch usually is the whole solve: nothing is enqueued behind it
     const ChipPlan& P = all_chip_[kind == SOLVE_MIXED];
-    auto ahead = [&] { return chip_off_ || cur_ != &all_ || P.stream_all || !P.rest.empty(); };
+    auto ahead = [&] { return !chip_on() || cur_ != &all_ || P.stream_all || !P.rest.empty(); };
     if((rc = enqueue_batch(kind, x, rhs, 0, 8))) return rc;
     bool queued = false;   // batch k is behind batch k - 1
     for(long k = 1;; ++k)
@@ -1392,7 +1421,7 @@ int Engine::run_iterations(int kind, int x, int rhs, int maxiter)
         for(int q : members)
         {
             if(!hs[q].done) all = false;
-            if(hs[q].chip_fail) chip_off_ = true;   // the solve goes on streaming
+            chip_heard(hs[q]);
         }
         if(all)
         {
@@ -1939,7 +1968,7 @@ int Engine::read_batch(const Inflight& f)
         TankHost& t = tanks[m.first];
         if(!t.used || t.seq != m.second || !solving_pc(t.pc)) continue;
         const BiState& st = hs[m.first];
-        if(st.chip_fail) chip_off_ = true;
+        chip_heard(st);
         if(!st.done) continue;
         t.iters_step += st.iter;
         last_state[m.first] = st;
@@ -1983,6 +2012,7 @@ int Engine::pump(std::vector<int>& stepped)
         rc = fc3_segment(s, mixed);
         cur_ = &all_;
         if(rc) return rc;
+        if(s < 3) chip_tick();
         for(int q : group)
         {
             TankHost& t = tanks[q];

@@ -126,6 +126,11 @@ public:
     // most device memory, in MiB, for the workspace of the on-chip solver; 0: every solve streams
     double onchip_mib = 1024.0;
     void set_onchip(double mib);
+    // seconds a block of an on-chip launch waits for another at most; 0: every launch of more
+    // than one block is given up.  500 ms: where a set has more blocks than the card has CUs, a
+    // tank's blocks can be dispatched one tank's whole solve apart.
+    double onchip_wait = 0.5;
+    void set_onchip_wait(double seconds);
     // tile plans per size bucket (jdir, floor(log2(nx ny nz))): tile rows ty x tz and
     // chunk length cpt; a bucket without an entry uses the default plan.  A tank takes the
     // plan of its bucket when it is added (and when its bucket's plan is set), so its
@@ -339,9 +344,19 @@ private:
     unsigned long long* d_chip_ = nullptr;
     unsigned chip_epoch_ = 0;
     int chip_ctl_ = 0;                      // next unused commit word
-    // no on-chip launches: a wait ran out (another process shares the GPU), there is no workspace,
-    // or onchip_mib is 0
-    bool chip_off_ = false;
+    bool chip_off_ = false;                 // no on-chip launches: no workspace, or onchip_mib is 0
+    // After a wait ran out (another process holds part of the GPU) the engine streams; the
+    // CHIP_PAUSE-th solve from then tries again, twice as many solves later after each further
+    // time up to 64 CHIP_PAUSE, so a GPU that stays shared costs one wait in thousands of solves.
+    static constexpr int CHIP_PAUSE = 64;
+    int chip_pause_ = 0;                    // solves until the next try, 0 on
+    int chip_next_pause_ = CHIP_PAUSE;
+    long chip_number_ = 0;                  // on-chip launches so far
+    long chip_heard_ = 0;                   // up to this launch, give-ups have been taken into account
+    long wall_khz_ = 0;                     // rate of the wall clock
+    bool chip_on() const { return !chip_off_ && chip_pause_ == 0; }
+    void chip_tick();                       // a solve begins
+    void chip_heard(const BiState& st);
     hipEvent_t chip_ev_ = nullptr;
     int chip_blocks(TankHost& t, int per_block, bool mixed) const;
     ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);

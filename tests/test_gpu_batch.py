@@ -261,6 +261,28 @@ def test_run_after_a_change_of_precision(tanks, added):
         A.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_scheduled_run_whose_launches_are_given_up(precision):
+    """Every on-chip launch given up (onchip_wait 0), in lockstep and scheduled: the same bits."""
+    from reef3d_amd import Batch
+    lock, it_lock = _run(TANKS, 2, precision)
+    for scheduled in (False, True):
+        B = Batch()
+        ids = [B.add(**kw) for kw, _ in TANKS]
+        for tid, (kw, f) in zip(ids, TANKS):
+            _initial(B, tid, kw, f)
+        B.solver_config(precision)
+        B.set_control("onchip_wait", 0)
+        _prepare(B)
+        print(precision, scheduled, flush=True)
+        it = B.run(2) if scheduled else [B.fc3_step()[0] for _ in range(2)][-1]
+        assert [it[t] for t in ids] == [it_lock[-1][q] for q in range(len(TANKS))]
+        for q, t in enumerate(ids):
+            for n in FIELDS:
+                assert np.array_equal(B.get(t, n), lock[q][n]), f"tank {q} {n}"
+        B.close()
+
+
 def test_batch_refuses_differing_shared_parameters():
     """Only dt and F45 may differ between the tanks of a batch; the shared values stay
     those of the first tank added to the empty batch, also after that tank is removed."""
