@@ -11,7 +11,6 @@
 namespace reef {
 
 constexpr int CHIP_NT = 512;                 // threads per block: two 256-thread groups
-constexpr int CHIP_CUS = 256;                // blocks that run at a time, one per CU
 constexpr int CHIP_BLOCKS = 256;             // blocks of a tank, at most
 constexpr int CHIP_TANKS = 64;               // tanks per launch
 constexpr int CHIP_TILES = 8192;             // tile slots of all blocks of a launch, at most
@@ -137,6 +136,29 @@ inline int chip_halo(const TileShape& s, int nb)
         }
     }
     return *std::max_element(h.begin(), h.end());
+}
+
+// Tile slots per group of the kernel variant for at most per_block tiles per block.
+inline int chip_ct(int per_block) { return std::max(2, per_block / 2); }
+
+// Blocks of a tank with at most per_block tiles each: the smallest power of two, at most 256,
+// the CUs of the card (the blocks of a tank wait for each other and need one each) and the
+// tank's items; 0 when the tank does not fit or its sums are taken in another order (a 2-D tank
+// with cpt > 1 walks its rows in the streaming v and t phases).  halo[q]: chip_halo of 2^q
+// blocks where it is known, else -1.
+inline int chip_blocks(const TileShape& s, int d3, int vsize, int per_block, int cus, int* halo)
+{
+    const int ct = chip_ct(per_block), limit = std::min(std::min(CHIP_BLOCKS, cus), s.nitems);
+    if(s.cpt > ct || (d3 == 0 && s.cpt > 1) || s.ntiles > CHIP_BLOCKS * per_block) return 0;
+    const int most = std::max(1, std::min(2 * (ct / s.cpt), per_block / s.cpt));   // items per block
+    const int hmax = chip_halo_max(d3, ct, vsize);
+    for(int q = 0, nb = 1; nb <= limit; ++q, nb *= 2)
+    {
+        if((s.nitems + nb - 1) / nb > most) continue;
+        if(halo[q] < 0) halo[q] = chip_halo(s, nb);
+        if(halo[q] <= hmax) return nb;
+    }
+    return 0;
 }
 
 }  // namespace reef

@@ -557,6 +557,13 @@ int Engine::sync_tables()
         cap_partials_ = 16 * std::max(items, (size_t)64);
         EHIP(hipMalloc(&d_partials_, sizeof(double) * cap_partials_));
     }
+    if(chip_cus_ < 0)
+    {
+        int device = 0, cus = 0;
+        EHIP(hipGetDevice(&device));
+        EHIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+        chip_cus_ = cus;
+    }
     if(!st_ev_[0])
         for(hipEvent_t& e : st_ev_) EHIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     std::vector<int> act;
@@ -1078,29 +1085,7 @@ static const char* const MIX_NAMES[4] = {"mix_v", "bicg32_t", "bicg32_x", "mix_r
 static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 
 // ------------------------------------------------------------------ on-chip solves
-// Tile slots per group of the kernel variant for at most per_block tiles per block.
-static int chip_ct(int per_block) { return std::max(2, per_block / 2); }
-
-// Blocks of tank t with at most per_block tiles each: the smallest power of two, at most 256
-// and the tank's items; 0 when the tank does not fit or its sums are taken in another order
-// (a 2-D tank with cpt > 1 walks its rows in the streaming v and t phases).
-int Engine::chip_blocks(TankHost& t, int per_block, bool mixed) const
-{
-    const TileShape& s = t.dev.shape;
-    const int ct = chip_ct(per_block), d3 = t.hg.jdir;
-    if(s.cpt > ct || (d3 == 0 && s.cpt > 1) || s.ntiles > CHIP_BLOCKS * per_block) return 0;
-    const int most = std::max(1, std::min(2 * (ct / s.cpt), per_block / s.cpt));   // items per block
-    const int hmax = chip_halo_max(d3, ct, mixed ? 4 : 8);
-    for(int q = 0, nb = 1; nb <= CHIP_BLOCKS && nb <= s.nitems; ++q, nb *= 2)
-    {
-        if((s.nitems + nb - 1) / nb > most) continue;
-        if(t.chip_h[q] < 0) t.chip_h[q] = chip_halo(s, nb);
-        if(t.chip_h[q] <= hmax) return nb;
-    }
-    return 0;
-}
-
-// On-chip launches for the slots.  A launch runs up to 256 blocks at a time, one per CU; of
+// On-chip launches for the slots.  A launch runs one block per CU at a time; of
 // more blocks the later ones start in order as CUs come free.  Few tiles per block keep an
 // iteration short, many keep more tanks on the chip at once.  The launch takes the tiles per
 // block (2, 4 or 8) with the shortest end of all tanks, estimated from the time of an iteration
@@ -1125,7 +1110,7 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
         int nb = 0, per = 2;
         for(int l = 2; l >= 0; --l)
         {
-            const int here = chip_blocks(t, 2 << l, mixed);
+            const int here = chip_blocks(t.dev.shape, t.hg.jdir, mixed ? 4 : 8, 2 << l, chip_cus_, t.chip_h.data());
             if(here) nb = here, per = l;
             k.nb[l] = nb;
             k.per[l] = per;
@@ -1143,7 +1128,7 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
     for(int l = 0; l < 3; ++l)
     {
         std::multimap<double, int> running;   // end time, blocks
-        int free_cus = CHIP_CUS;
+        int free_cus = chip_cus_;
         double now = 0.0, end = 0.0;
         for(const Tank& k : fit)
         {

@@ -339,6 +339,7 @@ private:
     };
     ChipPlan all_chip_[2];                  // of all_; [1]: mixed precision (FP32 vectors)
     ChipPlan solving_chip_;                 // of solving_sets_, in the precision solving_mixed_
+    int chip_cus_ = -1;                     // CUs of the device
     size_t chip_tiles_ = 0;                 // tile slots the workspace holds
     // accumulator words, commit words, then the halo words of chip_tiles_ tile slots
     unsigned long long* d_chip_ = nullptr;
@@ -358,7 +359,6 @@ private:
     void chip_tick();                       // a solve begins
     void chip_heard(const BiState& st);
     hipEvent_t chip_ev_ = nullptr;
-    int chip_blocks(TankHost& t, int per_block, bool mixed) const;
     ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);
     bool chip_ready(const ChipPlan& P);
     int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);

@@ -128,6 +128,20 @@ int main()
                    check(n[0], n[1], n[2], 1, 4, cpt, ct))
                     return 1;
         }
+    // no tank gets more blocks than the card has CUs; a whole card takes 2048 tiles
+    for(const auto& n : sizes)
+        for(int per = 2; per <= 2 * CHIP_CT_MAX; per *= 2)
+            for(int cus : {0, 1, 32, 38, 64, 128, 256, 304})
+            {
+                const int d3 = n[1] > 1;
+                const TileShape s = d3 ? make_shape(n[0], n[1], n[2], 4, 1, 1) : make_shape(n[0], 1, n[2], 1, 4, 1);
+                int halo[9];
+                std::fill(halo, halo + 9, -1);
+                const int nb = chip_blocks(s, d3, 4, per, cus, halo);
+                if(nb > cus || nb > CHIP_BLOCKS || (nb & (nb - 1)) || (nb && s.nitems > nb * per) ||
+                   (!nb && cus >= 256 && !d3 && s.ntiles <= CHIP_BLOCKS * per))
+                    return printf("%d %d %d: %d blocks of %d tiles on %d CUs\n", n[0], n[1], n[2], nb, per, cus), 1;
+            }
     for(int vsize = 4; vsize <= 8; vsize += 4)
         for(int d3 = 0; d3 < 2; ++d3)
             for(int ct = 2; ct <= CHIP_CT_MAX; ct *= 2)
