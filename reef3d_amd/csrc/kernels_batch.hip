@@ -1340,8 +1340,8 @@ __global__ void kb_fin_init(TankSet b)
 }
 
 // start of an iteration: the pending restart, or p = r + beta (p - w v), ph = aii p
-// (bicgstab_ijk.cpp:234-235 and precon_solve)
-template<class V>
+// (bicgstab_ijk.cpp:234-235 and precon_solve).  ALL: the class-walked tanks of the set too.
+template<class V, bool ALL>
 __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int rhs)
 {
     #pragma unroll 1
@@ -1350,7 +1350,7 @@ __global__ void __launch_bounds__(NT, OCC_A64) kb_bicg_p(TankSet b, int x, int r
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 2 || class_walk_ok(T))
+        if(st->done || st->mode == 2 || (!ALL && class_walk_ok(T)))
         {
             skip_tank(q, b);
             continue;
@@ -1872,8 +1872,10 @@ __global__ void kb_fin_t(TankSet b)
     }
 }
 
-// x and r updates, (r, r0), |r|^2 (bicgstab_ijk.cpp:223-268)
-template<class V>
+// x and r updates, (r, r0), |r|^2 (bicgstab_ijk.cpp:223-268).  ALL: the class-walked tanks of the
+// set too, for sets that hold both kinds: with a launch of its own for each kind these tanks ran
+// one after the other, and the x phase of a served stream's mixed sets took 28 us instead of 17.
+template<class V, bool ALL>
 __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int rhs)
 {
     #pragma unroll 1
@@ -1882,7 +1884,8 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
         CTank& T = tank_at(b, q.p);
         const DevGrid g = T.g;
         const BiState* st = T.st;
-        if(st->done || st->mode == 1 || st->mode == 3 || class_walk_ok(T))
+        const bool cls = class_walk_ok(T);
+        if(st->done || st->mode == 1 || st->mode == 3 || (!ALL && cls))
         {
             skip_tank(q, b);
             continue;
@@ -1891,13 +1894,17 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
         const TileWalk tw = item_walk(T, b, q);
         const V alpha = (V)st->alpha, w = (V)st->w;
         const int branch = st->branch;
+        // the FP32 class walk stores no ph, and t in the other half of v's buffer (kb_bicg_t)
+        const bool form_ph = ALL && sizeof(V) == 4 && cls;
         double vals[2] = {0.0, 0.0};
         V* __restrict__ xv = bv.x;
         V* __restrict__ r = bv.r;
         const V* __restrict__ vv = bv.v;
         const V* __restrict__ aii = bv.aii;
-        const V* __restrict__ ph = bv.ph;
+        const V* __restrict__ pv = form_ph ? bv.p : bv.ph;
         const V* __restrict__ tv = bv.t;
+        if constexpr(ALL && sizeof(V) == 4)
+            if(cls) tv = T.s[st->buf ? S_V : S_V2];
         const V* __restrict__ r0 = bv.r0;
         // independent tiles (the dot sums keep their order): unrolled so that several
         // tiles' loads are in flight
@@ -1908,16 +1915,18 @@ __global__ void __launch_bounds__(NT, OCC_FULL) kb_bicg_x(TankSet b, int x, int 
             long c;
             if(!tile_cell(g, tw, t, i, j, k, c)) continue;
             const V s = r[c] - alpha * vv[c];
+            V ph = pv[c];
+            if(form_ph) ph = ph * aii[c];
             V rn;
             if(branch)
             {
                 const V sh = s * aii[c];
-                xv[c] += alpha * ph[c] + w * sh;
+                xv[c] += alpha * ph + w * sh;
                 rn = s - w * tv[c];
             }
             else
             {
-                xv[c] += alpha * ph[c];
+                xv[c] += alpha * ph;
                 rn = s;
             }
             r[c] = rn;
@@ -3091,8 +3100,12 @@ void bl_bicg_phase(const TankSet& b, int x, int rhs, int phase, int part, hipStr
         switch(phase)
         {
             case 0:
-                if(b.has_pw) hipLaunchKernelGGL(kb_class_p, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
-                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_p<double>, grid64, dim3(NT), 0, s, b, x, rhs);
+                if(b.has_pw && b.has_direct)
+                    hipLaunchKernelGGL((kb_bicg_p<double, true>), grid64, dim3(NT), 0, s, b, x, rhs);
+                else if(b.has_pw)
+                    hipLaunchKernelGGL(kb_class_p, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                else
+                    hipLaunchKernelGGL((kb_bicg_p<double, false>), grid64, dim3(NT), 0, s, b, x, rhs);
                 break;
             case 1:
                 if(b.has_pw) hipLaunchKernelGGL(kb_class_v, pgrid_pw(b, OCC_PW), dim3(NT), 0, s, b, x, rhs);
@@ -3105,8 +3118,12 @@ void bl_bicg_phase(const TankSet& b, int x, int rhs, int phase, int part, hipStr
                     hipLaunchKernelGGL((kb_bicg_t<double, false>), pgrid_direct(b, OCC_A64), dim3(NT), 0, s, b, x, rhs);
                 break;
             default:
-                if(b.has_pw) hipLaunchKernelGGL(kb_class_x<double>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
-                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_x<double>, grid, dim3(NT), 0, s, b, x, rhs);
+                if(b.has_pw && b.has_direct)
+                    hipLaunchKernelGGL((kb_bicg_x<double, true>), grid, dim3(NT), 0, s, b, x, rhs);
+                else if(b.has_pw)
+                    hipLaunchKernelGGL(kb_class_x<double>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                else
+                    hipLaunchKernelGGL((kb_bicg_x<double, false>), grid, dim3(NT), 0, s, b, x, rhs);
                 break;
         }
         return;
@@ -3201,8 +3218,12 @@ void bl_mixed_phase(const TankSet& b, int x, int rhs, int phase, int part, hipSt
                     hipLaunchKernelGGL((kb_bicg_t<float, false>), pgrid_direct(b, OCC_FULL), dim3(NT), 0, s, b, x, rhs);
                 break;
             case 2:
-                if(b.has_pw) hipLaunchKernelGGL(kb_class_x<float>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
-                if(b.has_direct) hipLaunchKernelGGL(kb_bicg_x<float>, grid, dim3(NT), 0, s, b, x, rhs);
+                if(b.has_pw && b.has_direct)
+                    hipLaunchKernelGGL((kb_bicg_x<float, true>), grid, dim3(NT), 0, s, b, x, rhs);
+                else if(b.has_pw)
+                    hipLaunchKernelGGL(kb_class_x<float>, pgrid_pw(b, OCC_CX), dim3(NT), 0, s, b, x, rhs);
+                else
+                    hipLaunchKernelGGL((kb_bicg_x<float, false>), grid, dim3(NT), 0, s, b, x, rhs);
                 break;
             default: hipLaunchKernelGGL(kb_mix_ru, pgrid(b, OCC_A64), dim3(NT), 0, s, b, x, rhs); break;
         }

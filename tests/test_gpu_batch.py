@@ -283,6 +283,34 @@ def test_scheduled_run_whose_launches_are_given_up(precision):
         B.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("graphs", [False, True])
+def test_class_walked_and_other_tanks_in_one_launch(precision, graphs):
+    """3-D tanks with row classes and 2-D tanks in one set, all streamed and with the small ones
+    on chip, in lockstep and scheduled: the bits and iterations of each tank alone, whose phases
+    are launched for its own kind."""
+    from reef3d_amd import Batch
+    tanks = [TANKS[0], LARGE[0], TANKS[1], LARGE[1], TANKS[3]]
+    alone = [_run([t], 2, precision) for t in tanks]
+    for onchip in (0, 1024):
+        for scheduled in (False, True):
+            B = Batch()
+            ids = [B.add(**kw) for kw, _ in tanks]
+            for tid, (kw, f) in zip(ids, tanks):
+                _initial(B, tid, kw, f)
+            B.solver_config(precision)
+            B.set_control("graphs", 1 if graphs else 0)
+            B.set_control("onchip", onchip)
+            _prepare(B)
+            print(precision, graphs, onchip, scheduled, flush=True)
+            it = B.run(2) if scheduled else [B.fc3_step()[0] for _ in range(2)][-1]
+            assert [it[t] for t in ids] == [a[1][-1][0] for a in alone]
+            for q, t in enumerate(ids):
+                for n in FIELDS:
+                    assert np.array_equal(B.get(t, n), alone[q][0][0][n]), f"tank {q} {n}"
+            B.close()
+
+
 def test_batch_refuses_differing_shared_parameters():
     """Only dt and F45 may differ between the tanks of a batch; the shared values stay
     those of the first tank added to the empty batch, also after that tank is removed."""
