@@ -1089,13 +1089,54 @@ static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 // more blocks the later ones start in order as CUs come free.  Few tiles per block keep an
 // iteration short, many keep more tanks on the chip at once.  The launch takes the tiles per
 // block (2, 4 or 8) with the shortest end of all tanks, estimated from the time of an iteration
-// (measured, 2-D tanks: 11, 16 and 17.5 us with 2, 4 and 8 tiles per block, 3-D: 15, 19 and
-// 25 us) and
-// iterations in proportion to the tank's longest side, the longest first.
+// (CHIP_US) and iterations in proportion to the tank's longest side, the longest first.
+//
+// Beside that stands the end of the whole set streamed together (stream_end), whose tanks share
+// their launches.  Beside a tank that has to stream the others stream with it if that is shorter:
+// they add little to launches that are made anyway, and on chip they hold it up (three steps of a
+// mixed 2049x256 tank with three small ones: 629 ms with those on chip, 573 streamed).  A set
+// that fits as a whole is streamed where that is shorter by 13 % or more, since a streamed set
+// waits for the tank with the most iterations: the solves of one step of mixed 1150x157 tanks
+// take, on chip and streamed, 33 and 61 ms for one tank, 212 and 228 for 8, 446 and 367 for 16;
+// of mixed 192x32x64 tanks 14 and 23 for one, 221 and 202 for 16; of FP64 1150x157 tanks 29 and
+// 61 for one, 338 and 478 for 16.
+//
+// us an iteration on chip with 2, 4, 8 tiles per block, measured: [FP64, mixed][2-D, 3-D]
+static const double CHIP_US[2][2][3] = {{{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}}, {{11.5, 16.5, 20.5}, {15.0, 18.5, 22.5}}};
+// a streamed iteration, measured: its launches, then us per work item and per tile of the set
+// [FP64, mixed][2-D, 3-D] (sets of 7000 to 25 000 tiles: 0.8 to 0.9 of the sum for smaller ones)
+static const double STREAM_US = 28.0, ITEM_US[2][2] = {{0.0, 0.0119}, {0.0, 0.0114}},
+                    TILE_US[2][2] = {{0.0125, 0.0106}, {0.0076, 0.0055}};
+
+// estimated end of the tanks' streamed solves: every tank takes part in the launches until its
+// iterations, in proportion to its longest side, are done
+double Engine::stream_end(const std::vector<int>& slots, bool mixed) const
+{
+    std::vector<std::pair<int, double>> t;   // longest side, us per iteration
+    double all = 0.0;
+    for(int q : slots)
+    {
+        const HostGrid& h = tanks[q].hg;
+        const TileShape& s = tanks[q].dev.shape;
+        const double us = ITEM_US[mixed][h.jdir] * s.nitems + TILE_US[mixed][h.jdir] * s.ntiles;
+        t.emplace_back(std::max(h.nx, std::max(h.ny, h.nz)), us);
+        all += us;
+    }
+    std::sort(t.begin(), t.end());
+    double end = 0.0;
+    int at = 0;
+    for(const auto& k : t)
+    {
+        end += (k.first - at) * (STREAM_US + all);
+        at = k.first;
+        all -= k.second;
+    }
+    return end;
+}
+
 Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
 {
     ChipPlan P;
-    static const double US[2][3] = {{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}};
     struct Tank
     {
         int slot, side, per[3], nb[3];   // blocks and tiles per block for 2, 4, 8 (or the next that fits)
@@ -1121,7 +1162,6 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
             P.rest.push_back(q);
     }
     if(fit.empty()) return P;
-    P.stream_all = false;
     std::stable_sort(fit.begin(), fit.end(), [](const Tank& a, const Tank& b) { return a.side > b.side; });
     int best = 0;
     double best_end = 0.0;
@@ -1138,13 +1178,16 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
                 free_cus += running.begin()->second;
                 running.erase(running.begin());
             }
-            const double e = now + k.side * US[tanks[k.slot].hg.jdir][k.per[l]];
+            const double e = now + k.side * CHIP_US[mixed][tanks[k.slot].hg.jdir][k.per[l]];
             running.emplace(e, k.nb[l]);
             free_cus -= k.nb[l];
             end = std::max(end, e);
         }
         if(l == 0 || end < best_end) best = l, best_end = end;
     }
+    const double share = P.rest.empty() ? 0.87 : 1.0;
+    if(stream_end(slots_in, mixed) < share * (best_end + stream_end(P.rest, mixed))) return P;
+    P.stream_all = false;
     for(const Tank& k : fit)
     {
         const TankHost& t = tanks[k.slot];

@@ -359,6 +359,7 @@ private:
     void chip_tick();                       // a solve begins
     void chip_heard(const BiState& st);
     hipEvent_t chip_ev_ = nullptr;
+    double stream_end(const std::vector<int>& slots, bool mixed) const;
     ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);
     bool chip_ready(const ChipPlan& P);
     int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);

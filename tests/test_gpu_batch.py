@@ -286,9 +286,9 @@ def test_scheduled_run_whose_launches_are_given_up(precision):
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("graphs", [False, True])
 def test_class_walked_and_other_tanks_in_one_launch(precision, graphs):
-    """3-D tanks with row classes and 2-D tanks in one set, all streamed and with the small ones
-    on chip, in lockstep and scheduled: the bits and iterations of each tank alone, whose phases
-    are launched for its own kind."""
+    """3-D tanks with row classes and 2-D tanks in one set, all streamed, or the small ones on chip
+    once the large ones have ended, in lockstep and scheduled: the bits and iterations of each
+    tank alone, whose phases are launched for its own kind."""
     from reef3d_amd import Batch
     tanks = [TANKS[0], LARGE[0], TANKS[1], LARGE[1], TANKS[3]]
     alone = [_run([t], 2, precision) for t in tanks]
@@ -309,6 +309,28 @@ def test_class_walked_and_other_tanks_in_one_launch(precision, graphs):
                 for n in FIELDS:
                     assert np.array_equal(B.get(t, n), alone[q][0][0][n]), f"tank {q} {n}"
             B.close()
+
+
+def test_a_set_too_large_for_the_chip_streams_until_it_is_smaller():
+    """Twelve mixed tanks of 1344 tiles: streamed together first, on chip when few are left (the
+    iterations of a solve done partly in each form), the bits of the tanks alone."""
+    from reef3d_amd import Batch
+    tanks = [_tank(1300 - 24 * q, 1, 256, 0.02, 3.0, 0.1, 3.0 - 0.1 * q, 0.004, 0) for q in range(12)]
+    B = Batch()
+    ids = [B.add(**kw) for kw, _ in tanks]
+    for tid, (kw, f) in zip(ids, tanks):
+        _initial(B, tid, kw, f)
+    B.solver_config("mixed")
+    _prepare(B)
+    B.timing(True)
+    it = B.run(1)
+    assert B.timing_get("mix_v")[1] > 0 and B.timing_get("chip")[1] > 0
+    for q, t in enumerate(ids):
+        alone, it1 = _run([tanks[q]], 1, "mixed")
+        assert it[t] == it1[0][0]
+        for n in FIELDS:
+            assert np.array_equal(B.get(t, n), alone[0][n]), f"tank {q} {n}"
+    B.close()
 
 
 def test_batch_refuses_differing_shared_parameters():
