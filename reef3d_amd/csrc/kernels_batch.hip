@@ -943,28 +943,41 @@ __device__ __forceinline__ void class_walk(CTank& T, const DevGrid& g, const Til
             ad = ld32(aiia, k > 0 ? c - sxy : c);
         }
         fetch_raw(k, P0);
-        __syncthreads();   // the last run's entries have been read
-        for(int q = h; q < 4 * ZPLANES; q += NT)
-        {
-            const int kk = min(zk0 + (q >> 2), g.nz - 1), e = 2 * (((q >> 1) & 1) * g.nz + kk) + (q & 1);
-            S.z[q >> 2][q & 3] = T.ct[2][e];
-            if constexpr(sizeof(V) == 4) S.z32[q >> 2][q & 3] = T.ct32[2][e];
-        }
-        for(int q = h; q < CROWS * ZPLANES; q += NT)
-        {
-            const int rr = q / ZPLANES, kk = zk0 + q - rr * ZPLANES;
-            if(kk > min(kend, g.nz - 1)) continue;
+        // the classes of the run's planes, one row per wavefront and load, all in flight together:
+        // with 14 x 66 entries dealt to the threads in turn an item of one plane took as long to
+        // set up as one of 64
+        const int kl = min(kend, g.nz - 1), np = kl - zk0 + 1;
+        constexpr int RW = (CROWS + TY - 1) / TY;
+        auto row_of = [&](int rr) {
             const int jr = rr < TY ? j0 + rr : rr == TY ? j0 - 1 : rr == TY + 1 ? j0 + TY : j0 + (rr - 2) % TY;
             const int br = rr < TY + 2 ? bx : rr < 2 * TY + 2 ? bx - 1 : bx + 1;
             const int jq = max(0, min(jr, g.ny - 1)), bq = max(0, min(br, tw.s.nbx - 1));
-            S.c[rr][q - rr * ZPLANES] = T.cls[((long)bq * g.ny + jq) * g.nz + kk];
+            return T.cls + ((long)bq * g.ny + jq) * g.nz + zk0;
+        };
+        unsigned char rcl[RW];
+        #pragma unroll
+        for(int m = 0; m < RW; ++m) rcl[m] = row_of(min(row + m * TY, CROWS - 1))[min(lane, np - 1)];
+        __syncthreads();   // the last run's entries have been read
+        for(int q = h; q < 4 * np; q += NT)
+        {
+            const int e = 2 * (((q >> 1) & 1) * g.nz + zk0 + (q >> 2)) + (q & 1);
+            S.z[q >> 2][q & 3] = T.ct[2][e];
+            if constexpr(sizeof(V) == 4) S.z32[q >> 2][q & 3] = T.ct32[2][e];
+        }
+        #pragma unroll
+        for(int m = 0; m < RW; ++m)
+        {
+            const int rr = row + m * TY;
+            if(rr >= CROWS) continue;
+            if(lane < np) S.c[rr][lane] = rcl[m];
+            if(lane + TX < np) S.c[rr][lane + TX] = row_of(rr)[lane + TX];
         }
         if(h < TX)
             S.ax[h] = axis_factor(g, op, 0, min(i0 + h, g.nx - 1));
         else if(h < TX + TY)
             S.ay[h - TX] = axis_factor(g, op, 1, min(j0 + h - TX, g.ny - 1));
-        else if(h >= 2 * TX && h < 2 * TX + ZPLANES)
-            S.az[h - 2 * TX] = axis_factor(g, op, 2, min(zk0 + h - 2 * TX, g.nz - 1));
+        else if(h >= 2 * TX && h < 2 * TX + np)
+            S.az[h - 2 * TX] = axis_factor(g, op, 2, zk0 + h - 2 * TX);
         __syncthreads();
         keyC = keyN = keyH = 0;
         V d;
