@@ -335,27 +335,24 @@ __global__ void __launch_bounds__(NT) kb_fill(TankSet b, int id, double v)
     }
 }
 
-// compiled ghost program prog of every active tank on array id
+// compiled ghost program prog of tank blockIdx.y on array id
 __global__ void __launch_bounds__(NT) kb_ghost(TankSet b, int prog, int id)
 {
-    for(int tk = 0; tk < b.n; ++tk)
+    CTank& T = tank_at(b, (int)blockIdx.y);
+    const GhostOp* __restrict__ ops = T.gops[prog];
+    const int n = T.gnops[prog];
+    double* __restrict__ f = T.f[id];
+    for(int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
     {
-        CTank& T = tank_at(b, tk);
-        const GhostOp* __restrict__ ops = T.gops[prog];
-        const int n = T.gnops[prog];
-        double* __restrict__ f = T.f[id];
-        for(int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
-        {
-            const GhostOp op = ops[q];
-            double val;
-            if(op.src < 0)
-                val = 0.0;
-            else if(op.src & (1 << 30))
-                val = 0.0 + op.w * f[op.src & ~(1 << 30)];
-            else
-                val = f[op.src];
-            f[op.dst] = val;
-        }
+        const GhostOp op = ops[q];
+        double val;
+        if(op.src < 0)
+            val = 0.0;
+        else if(op.src & (1 << 30))
+            val = 0.0 + op.w * f[op.src & ~(1 << 30)];
+        else
+            val = f[op.src];
+        f[op.dst] = val;
     }
 }
 
@@ -3009,11 +3006,14 @@ void bl_fill(const TankSet& b, int id, double v, hipStream_t s)
 }
 // Two ghost operations per thread of the largest program, whose length sets the grid: 256 blocks
 // whatever the size left up to 20 dependent rounds to a thread of a large tank and idle blocks
-// to a small one (a fill at 512x64x128 16.0 -> 13.9 us, 128^3 6.9 -> 6.2).
+// to a small one (a fill at 512x64x128 16.0 -> 13.9 us, 128^3 6.9 -> 6.2).  Each tank has its
+// own row of blocks: with every block going through the tanks one after the other the tanks'
+// latencies added up (16 tanks of 700x160: 14 us with 256 blocks, 21 us with 8, now 6.7;
+// 8 of 128x64 7.5, 7.9, 6.5; one tank 6.4 either way).
 void bl_ghost(const TankSet& b, int prog, int id, int most, hipStream_t s)
 {
     const unsigned blocks = (unsigned)std::max(8, std::min(4096, (most + 2 * NT - 1) / (2 * NT)));
-    hipLaunchKernelGGL(kb_ghost, dim3(blocks), dim3(NT), 0, s, b, prog, id);
+    hipLaunchKernelGGL(kb_ghost, dim3(blocks, (unsigned)b.n), dim3(NT), 0, s, b, prog, id);
 }
 void bl_hj_stage(const TankSet& b, int stage, int phi_s, int phi_n, int u, int v, int w, int out, double cfac,
                  hipStream_t s)

@@ -333,6 +333,34 @@ def test_a_set_too_large_for_the_chip_streams_until_it_is_smaller():
     B.close()
 
 
+def test_ghost_fills_of_uneven_tanks():
+    """One fill of 1 and of many tanks from 4 to 2049 columns, 2-D and 3-D: each has the ghost
+    layers it gets alone, for every program of a step."""
+    from reef3d_amd import Batch
+    sizes = [(4, 1, 4, 0), (2049, 1, 256, 0), (65, 5, 33, 1), (12, 10, 8, 1), (130, 33, 37, 1), (64, 1, 9, 0)]
+
+    def fill(shapes, fields):
+        B = Batch()
+        ids = []
+        for nx, ny, nz, jdir in shapes:
+            f = [0.02 * np.arange(-5, n + 6, dtype=np.float64) for n in (nx, ny, nz)]
+            ids.append(B.add(nx, ny, nz, *f, 0.02, 0.02, jdir=jdir, top_group=3, g=(0.0, 0.0, -9.81)))
+        out = []
+        for name, kind, gcv in (("phi", 4, 52), ("u", 1, 10), ("v", 2, 11), ("w", 3, 12), ("press", 4, 40), ("ro", 4, 1)):
+            for t, a in zip(ids, fields):
+                B.put(t, name, a)
+            B.ghost_fill(name, kind, gcv)
+            out.append([B.get(t, name) for t in ids])
+        B.close()
+        return out
+
+    fields = [np.random.default_rng(q).standard_normal((nz + 6, ny + 6, nx + 6)) for q, (nx, ny, nz, _) in enumerate(sizes)]
+    together = fill(sizes, fields)
+    for q, s in enumerate(sizes):
+        alone = fill([s], [fields[q]])
+        assert all(np.array_equal(t[q], a[0]) for t, a in zip(together, alone)), s
+
+
 def test_batch_refuses_differing_shared_parameters():
     """Only dt and F45 may differ between the tanks of a batch; the shared values stay
     those of the first tank added to the empty batch, also after that tank is removed."""
