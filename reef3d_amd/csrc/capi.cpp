@@ -127,6 +127,12 @@ int control(Engine& e, const char* key, double value)
         e.set_onchip(value);
         return 0;
     }
+    if(std::strcmp(key, "rowclass") == 0)
+    {
+        if(value != 0.0 && value != 1.0) return fail(REEF_E_ARG, "rowclass must be 0 or 1");
+        e.set_rowclass(value != 0.0);
+        return 0;
+    }
     if(std::strcmp(key, "onchip_wait") == 0)
     {
         if(!(value >= 0.0)) return fail(REEF_E_ARG, "onchip_wait must be >= 0");

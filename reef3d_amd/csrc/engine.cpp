@@ -604,6 +604,7 @@ std::vector<TankSet> Engine::make_sets(const std::vector<int>& slots_in) const
         S.partials_ru = d_partials_ + cap_partials_ / 2;
         S.rw = shared() ? shared()->W1 : 1000.0;
         S.ra = shared() ? shared()->W3 : 1.205;
+        if(!rowclass) S.rw = S.ra = std::nan("");   // equal to no density
         const size_t b = std::min(slots.size(), a + (size_t)SET_MAX);
         int nt = 0, ni = 0;
         for(size_t q = a; q < b; ++q)

@@ -131,6 +131,13 @@ public:
     // tank's blocks can be dispatched one tank's whole solve apart.
     double onchip_wait = 0.5;
     void set_onchip_wait(double seconds);
+    // 0: every row of a 3-D tank is of mixed density class (the couplings come from the faces)
+    bool rowclass = true;
+    void set_rowclass(bool on)
+    {
+        rowclass = on;
+        dirty_ = true;
+    }
     // tile plans per size bucket (jdir, floor(log2(nx ny nz))): tile rows ty x tz and
     // chunk length cpt; a bucket without an entry uses the default plan.  A tank takes the
     // plan of its bucket when it is added (and when its bucket's plan is set), so its
