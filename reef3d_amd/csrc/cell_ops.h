@@ -47,7 +47,8 @@ __device__ __forceinline__ double div_normal(double a, double b)
 // a / d for a grid width d with r = 1 / d (rounded to nearest): the product is within 1.5 ulp,
 // the first correction makes it faithful, the second rounds correctly (Markstein 1990: with r
 // correctly rounded and q faithful, q + (a - q d) r rounds to a / d).  div_fixup gives the IEEE
-// results for infinities, NaN and zeros.  Operands below 1e-290 may differ in the last bit.  6
+// results for infinities, NaN and zeros, and the infinity of a quotient that overflows (the
+// corrections leave a NaN there).  Operands below 1e-290 may differ in the last bit.  6
 // instructions instead of 11.
 __device__ __forceinline__ double div_width(double a, double d, double r)
 {
@@ -57,8 +58,10 @@ __device__ __forceinline__ double div_width(double a, double d, double r)
     return __builtin_amdgcn_div_fixup(q, d, a);
 }
 
-// the three weights c / (a^2 (c0/a1^2 + c1/a2^2 + c2/a3^2)); the guard keeps every operand and
-// quotient of div_normal between 1e-281 and 1e281
+// the three weights c / (a^2 (c0/a1^2 + c1/a2^2 + c2/a3^2)); with the guard the squares lie
+// between 1e-140 and 1e140, the quotients of the sum between 1e-146 and 1e146, the last divisor
+// between 1e-6 (its own term of the sum) and 3e286 and the weight between 3e-293 and 1: every
+// operand and quotient of div_normal is a normal number
 __device__ __forceinline__ void weno_weights(double c0, double c1, double c2, double a1, double a2, double a3, double& w1,
                                              double& w2, double& w3)
 {

@@ -2134,10 +2134,9 @@ int Engine::vortex_step(double simtime)
     const TankHost* t0 = first_used();
     const reef_params* sp = shared();
     if(!t0 || !sp) return 0;
-    const double grav[3] = {sp->W20, sp->W21, sp->W22};
     // The void momentum step: only w's.  u and v of every cell it updates, and the ghosts filled
     // from them (u 10, v 11), are written again below by the prescribed field and its fills.
-    const double Fv = 0.0 + (0.0 + grav[2] + 0.0 + 0.0) * 1.0;
+    const double Fv = 0.0 + (0.0 + sp->W22 + 0.0 + 0.0) * 1.0;
     each([&](const TankSet& S) { bl_void_rk3(S, 3, REEF_W, Fv, stream); });
     if((rc = ghost(REEF_W, 3, 12))) return rc;
     each([&](const TankSet& S) { bl_vortex_velocity(S, simtime, t0->hg.DXM, stream); });

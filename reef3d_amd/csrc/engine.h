@@ -17,7 +17,6 @@
 #include "chip.h"
 
 #include <array>
-#include <atomic>
 #include <deque>
 #include <map>
 #include <string>

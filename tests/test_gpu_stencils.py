@@ -63,6 +63,37 @@ def test_weno_sides_and_guard(shape, sides, scale):
     assert np.array_equal(inner(D.get("phi")), inner(phi))
 
 
+@pytest.mark.parametrize("shape", [(37, 9, 21, 1), (130, 1, 33, 0)])
+def test_quotients_that_overflow(shape):
+    """Cells of +-1e307, whose differences overflow when divided by the width (0.02): infinities
+    decide the upwind side of the reinitialisation and end in NaN, cell for cell as the oracle's."""
+    nx, ny, nz, jdir = shape
+    print(shape, flush=True)
+    f, O, D = _tank(nx, ny, nz, jdir, stretch=0.1)
+    rng = np.random.default_rng(nx)
+    phi = f["phi"].copy()
+    at = rng.integers(0, [nz, ny, nx], (12, 3))
+    for q, (k, j, i) in enumerate(at):
+        inner(phi)[k, j, i] = (-1e307, 1e307, 1e305)[q % 3]
+    O.ghost(phi, 4, 52)
+    vel = [rng.standard_normal(O.shape) for _ in range(3)]
+    if not jdir:
+        vel[1][...] = 0.0
+    for kind, gcv, a in ((1, 10, vel[0]), (2, 11, vel[1]), (3, 12, vel[2])):
+        O.ghost(a, kind, gcv)
+    for n, a in zip(("phi", "u", "v", "w"), (phi, *vel)):
+        D.put(n, a)
+    L = np.zeros(O.shape)
+    O.hj(phi, *vel, L)
+    D.zero("L")
+    D.convection("phi", 4)
+    assert np.array_equal(inner(D.get("L")), inner(L), equal_nan=True)
+    O.reini(phi, 1)
+    D.reini("phi", 1)
+    assert np.isnan(phi).any() and np.isfinite(inner(phi)).any()
+    assert np.array_equal(inner(D.get("phi")), inner(phi), equal_nan=True)
+
+
 @pytest.mark.parametrize("shape", [(300, 33, 75, 1), (129, 65, 70, 1), (64, 70, 131, 1)])
 @pytest.mark.parametrize("stretch", [0.0, 0.2])
 def test_class_walk(shape, stretch):
