@@ -85,7 +85,7 @@ SOLVER_BYTES.update({"mix_v": 28, "bicg32_t": 16, "bicg32_x": 32})
 HBM_PEAK_GBS = 8000.0
 TIMED_FAMILIES = ("bicg_init", "bicg_p", "bicg_v", "bicg_t", "bicg_x", "mix_init", "mix_v",
                   "bicg32_t", "bicg32_x", "mix_ru", "coef32", "add32", "hj", "reini", "momentum", "ghost",
-                  "face_rho", "correct", "poisson_rhs", "heaviside", "copy", "flux")
+                  "face_rho", "correct", "poisson_rhs", "heaviside", "copy", "flux", "chip")
 
 
 def make_domain(cfg):
@@ -250,7 +250,7 @@ def hbm_copy(nbytes=1 << 30, reps=5):
 # kernel name -> the family of the bench's SOLVER_BYTES (the traffic tables of the profiles)
 TRAFFIC_KERNELS = (("kb_class_p", "bicg_p"), ("kb_class_v", "bicg_v"),
                    ("kb_bicg_t<double, true>", "bicg_t"), ("kb_class_x<double>", "bicg_x"),
-                   ("kb_bicg_x<double>", "bicg_x"), ("kb_mix_v<true>", "mix_v"),
+                   ("kb_bicg_x<double", "bicg_x"), ("kb_mix_v<true>", "mix_v"),
                    ("kb_bicg_t<float, true>", "bicg32_t"), ("kb_class_x<float>", "bicg32_x"), ("kb_hj_stage", "hj"), ("kb_reini_stage", "reini"))
 
 

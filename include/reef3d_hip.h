@@ -380,7 +380,12 @@ int reef_batch_timing_get(reef_batch* b, const char* name, double* ms, long* lau
 
 /* Kernel timing: the context records HIP events around its launches when enabled. */
 int reef_timing_enable(reef_ctx* ctx, int on);
-/* name: kernel family ("bicgstab", "hj", "reini", "flux", ...); returns total ms and launches */
+/* name: kernel family; returns total ms and launches.  "hj", "reini", "momentum", "flux", "ghost",
+ * "copy", "face_rho", "poisson_rhs", "correct", "heaviside", "timestep", "wave"; of solves that
+ * run phase by phase "bicg_init", "bicg_p", "bicg_v", "bicg_t", "bicg_x", in mixed precision
+ * "coef32", "mix_init", "mix_v", "bicg32_t", "bicg32_x", "mix_ru", "add32", on the caller's
+ * operator "mat_init", "mat_p", "mat_v", "mat_t", "mat_x"; "chip": the on-chip launches, which
+ * hold all phases of their solves.  A family that was not launched reads 0. */
 int reef_timing_get(reef_ctx* ctx, const char* name, double* ms, long* launches);
 int reef_timing_reset(reef_ctx* ctx);
 
