@@ -146,9 +146,9 @@ int reef_ctx_create(const reef_grid_desc* grid, const reef_params* prm, reef_ctx
  * device memory, beside the tanks', for the solves that run in one launch with their vectors
  * on the chip (tanks of up to 2048 tiles; default 1024, at most 100 are used); where they do
  * not fit, or with 0, those solves run phase by phase like a large tank's, with identical
- * results.  "onchip_wait": seconds such a launch waits for GPU time that another process
- * holds, before the solve goes on phase by phase (default 0.5; 0: every launch of several
- * blocks is given up), with identical results.  "rowclass": 1 (default) = rows of a 3-D tank
+ * results.  "onchip_giveup": 1 = every such launch of several blocks ends without a result, as
+ * it does after waiting 500 ms for GPU time that another process holds, and the solve goes on
+ * phase by phase, with identical results (default 0).  "rowclass": 1 (default) = rows of a 3-D tank
  * whose faces all have the density of water or of air take the operator from per-axis tables,
  * 0 = every row forms it from its faces, with identical results.  Other keys: REEF_E_UNSUPPORTED. */
 int reef_set_control(reef_ctx* ctx, const char* key, double value);
@@ -341,7 +341,7 @@ int reef_batch_get(reef_batch* b, int tank, int field_id, double* host, int layo
 int reef_batch_ghost_fill(reef_batch* b, int field_id, int kind, int gcv);
 int reef_batch_fluid_update(reef_batch* b);
 /* the keys of reef_set_control ("F49", "graphs", "N48", "N47", "D20", "N43", "simtime",
- * "onchip", "onchip_wait", "rowclass") for every tank of the batch */
+ * "onchip", "onchip_giveup", "rowclass") for every tank of the batch */
 int reef_batch_control(reef_batch* b, const char* key, double value);
 int reef_batch_solver_config(reef_batch* b, int precision, double delta);
 /* Tile plans per size bucket (no counterpart in the reference).  A bucket is (jdir,

@@ -133,10 +133,10 @@ int control(Engine& e, const char* key, double value)
         e.set_rowclass(value != 0.0);
         return 0;
     }
-    if(std::strcmp(key, "onchip_wait") == 0)
+    if(std::strcmp(key, "onchip_giveup") == 0)
     {
-        if(!(value >= 0.0)) return fail(REEF_E_ARG, "onchip_wait must be >= 0");
-        e.set_onchip_wait(value);
+        if(value != 0.0 && value != 1.0) return fail(REEF_E_ARG, "onchip_giveup must be 0 or 1");
+        e.set_onchip_giveup(value != 0.0);
         return 0;
     }
     return fail(REEF_E_UNSUPPORTED, std::string("control key not supported: ") + key);

@@ -16,8 +16,6 @@ struct ChipSet
     unsigned long long* acc;       // CHIP_ACC_WORDS per tank of the launch
     unsigned* ctl;                 // commit word per tank of the launch, 0 before it
     unsigned epoch;                // tag of the launch's first exchange
-    long wait;                     // ticks of the wall clock a block waits at most; 0: none starts
-    long number;                   // of the launch among its engine's, from 1
     int cap;                       // iterations at most
     int hmax;                      // largest halo of a block
     int d3, ct;                    // 3-D tanks; tile slots per group

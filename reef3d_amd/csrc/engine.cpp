@@ -1248,22 +1248,21 @@ bool Engine::chip_ready(const ChipPlan& P)
     return true;
 }
 
-void Engine::set_onchip_wait(double seconds)
+void Engine::set_onchip_giveup(bool on)
 {
-    onchip_wait = seconds;
+    onchip_giveup = on;
     chip_pause_ = 0;
     chip_next_pause_ = CHIP_PAUSE;
-    chip_heard_ = chip_number_;
 }
 
 void Engine::chip_tick()
 {
-    if(chip_pause_ > 0 && --chip_pause_ == 0) chip_heard_ = chip_number_;
+    if(chip_pause_ > 0) --chip_pause_;
 }
 
 void Engine::chip_heard(const BiState& st)
 {
-    if(st.chip_fail <= chip_heard_ || chip_pause_ > 0) return;
+    if(!st.chip_fail || chip_pause_ > 0) return;
     chip_pause_ = chip_next_pause_;   // the solve goes on streaming
     chip_next_pause_ = std::min(2 * chip_next_pause_, 64 * CHIP_PAUSE);
 }
@@ -1286,12 +1285,6 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
     unsigned long long* halo = d_chip_ + (size_t)CHIP_TANKS * CHIP_ACC_WORDS + CHIP_CTL / 2;
     int dev = 0;
     EHIP(hipGetDevice(&dev));
-    if(wall_khz_ == 0)
-    {
-        int khz = 0;
-        EHIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
-        wall_khz_ = std::max(khz, 1);
-    }
     std::lock_guard<std::mutex> lk(g_chip_mu);
     auto& last = g_chip_last[dev];
     if(last.first && last.first != this) EHIP(hipStreamWaitEvent(stream, last.second, 0));
@@ -1316,8 +1309,7 @@ int Engine::chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap)
         S.ctl = ctl + chip_ctl_;
         S.epoch = chip_epoch_;
         S.cap = cap;
-        S.wait = onchip_wait > 0.0 ? std::max(1L, (long)(std::min(onchip_wait, 1.0e6) * 1000.0 * (double)wall_khz_)) : 0;
-        S.number = ++chip_number_;
+        if(onchip_giveup) EHIP(hipMemsetD32Async(S.ctl, (int)0x80000000u, S.n, stream));
         tbegin("chip");
         bl_chip_solve(S, kind, x, rhs, stream);
         tend();

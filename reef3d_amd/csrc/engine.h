@@ -125,11 +125,9 @@ public:
     // most device memory, in MiB, for the workspace of the on-chip solver; 0: every solve streams
     double onchip_mib = 1024.0;
     void set_onchip(double mib);
-    // seconds a block of an on-chip launch waits for another at most; 0: every launch of more
-    // than one block is given up.  500 ms: where a set has more blocks than the card has CUs, a
-    // tank's blocks can be dispatched one tank's whole solve apart.
-    double onchip_wait = 0.5;
-    void set_onchip_wait(double seconds);
+    // every on-chip launch of more than one block per tank finds its abort bit set and is given up
+    bool onchip_giveup = false;
+    void set_onchip_giveup(bool on);
     // 0: every row of a 3-D tank is of mixed density class (the couplings come from the faces)
     bool rowclass = true;
     void set_rowclass(bool on)
@@ -358,11 +356,10 @@ private:
     static constexpr int CHIP_PAUSE = 64;
     int chip_pause_ = 0;                    // solves until the next try, 0 on
     int chip_next_pause_ = CHIP_PAUSE;
-    long chip_number_ = 0;                  // on-chip launches so far
-    long chip_heard_ = 0;                   // up to this launch, give-ups have been taken into account
-    long wall_khz_ = 0;                     // rate of the wall clock
     bool chip_on() const { return !chip_off_ && chip_pause_ == 0; }
     void chip_tick();                       // a solve begins
+    // after a give-up; a solve keeps its mark to its end, so one that was still streaming when the
+    // pause ended may start another
     void chip_heard(const BiState& st);
     hipEvent_t chip_ev_ = nullptr;
     double stream_end(const std::vector<int>& slots, bool mixed) const;

@@ -19,10 +19,11 @@
 // and with NB dividing 256 a block holds whole such strided subsets, so it publishes the
 // 256 / NB accumulators of its threads instead of every item's partial.
 //
-// Every wait is bounded (ChipSet::wait): a block that waits too long (another process holds
+// Every wait is bounded (WAIT_TICKS): a block that waits too long (another process holds
 // part of the GPU, so not all blocks are resident) sets the tank's abort bit, every block of
 // the tank leaves, and nothing has been stored: the vectors and the state are written only
-// after all blocks have arrived at the commit counter, which the abort bit shares.
+// after all blocks have arrived at the commit counter, which the abort bit shares.  The host can
+// set the bit before the launch (Engine::onchip_giveup).
 #include "chip.h"
 #include "cell_ops.h"
 #include "solver_state.h"
@@ -35,6 +36,9 @@ typedef unsigned long long u64;
 constexpr int CG = CHIP_NT / NT;           // 256-thread groups
 static_assert(CG == 2, "groups of a block");
 constexpr unsigned ABORT = 0x80000000u;
+// 500 ms of the 100 MHz wall clock: where a set has more blocks than the card has CUs, a tank's
+// blocks can be dispatched one tank's whole solve apart
+constexpr long WAIT_TICKS = 50000000;
 
 __device__ __forceinline__ void put_word(u64* p, u64 v)
 {
@@ -80,18 +84,18 @@ struct Wire<float>
 };
 
 // the bound of one wait: true when it has to end (the tank's abort bit is set, by another
-// block or here after `wait` ticks of the wall clock)
+// block or here after WAIT_TICKS)
 struct Guard
 {
     unsigned* ctl;
-    long t0, wait;
+    long t0;
     int spins;
-    __device__ Guard(unsigned* c, long w) : ctl(c), t0((long)wall_clock64()), wait(w), spins(0) {}
+    __device__ Guard(unsigned* c) : ctl(c), t0((long)wall_clock64()), spins(0) {}
     __device__ bool stop()
     {
         if((++spins & 63) != 0) return false;
         if(__hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & ABORT) return true;
-        if((long)wall_clock64() - t0 < wait) return false;
+        if((long)wall_clock64() - t0 < WAIT_TICKS) return false;
         __hip_atomic_fetch_or(ctl, ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return true;
     }
@@ -179,8 +183,6 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
     if(tid < CS) stile[tid] = chip_slot_tile(sh, CT, NB, b, tid);
     __syncthreads();
     if(st.done) return;
-    // no waiting at all: the tank is given up before it starts, its blocks leave at the commit
-    if(tid == 0 && NB > 1 && S.wait == 0) __hip_atomic_fetch_or(ctl, ABORT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // the neighbour tile of each face (+x, -x, +y, -y, +z, -z): in this block (its slot), in
     // another (-2), none (-1)
     if(tid < CS * 6)
@@ -392,7 +394,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             src[s] = -1;
             if(s < ns && tid + s * CHIP_NT < H) src[s] = hsrc[tid + s * CHIP_NT];
         }
-        Guard gd(ctl, S.wait);
+        Guard gd(ctl);
         for(;;)
         {
             bool ok = true;
@@ -484,7 +486,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
                 else
                 {
                     Wire<double> w[M];
-                    Guard gd(ctl, S.wait);
+                    Guard gd(ctl);
                     for(;;)
                     {
                         bool ok = true;
@@ -531,7 +533,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
                 {
                     const u64* src = cw + (size_t)((b % CHIP_COPIES) * CHIP_COPY_WORDS) + (w * M + m) * 2;
                     Wire<double> z;
-                    Guard gd(ctl, S.wait);
+                    Guard gd(ctl);
                     for(;;)
                     {
                         z.load(src);
@@ -829,7 +831,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             while(!(cur & ABORT) && (int)cur < NB)
             {
                 cur = __hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if(!(cur & ABORT) && (int)cur < NB && (long)wall_clock64() - t0 > S.wait)
+                if(!(cur & ABORT) && (int)cur < NB && (long)wall_clock64() - t0 > WAIT_TICKS)
                 {
                     // only while someone is missing: once all have arrived nobody may abort
                     unsigned want = cur;
@@ -843,7 +845,7 @@ __global__ void __launch_bounds__(CHIP_NT) kc_solve(ChipSet S, int x_, int rhs_)
             ok = !(cur & ABORT);
         }
         dead = !ok;
-        if(!ok && b == 0) T.st->chip_fail = S.number;
+        if(!ok && b == 0) T.st->chip_fail = 1;
     }
     __syncthreads();
     if(dead) return;

@@ -92,7 +92,7 @@ struct BiState
     int pending, nru;
     int buf;                           // mixed precision: current half of the FP32 p / v buffers
     long ncell;
-    long chip_fail;                    // the last on-chip launch that gave this solve up, 0 none
+    int chip_fail;                     // an on-chip launch gave up its wait: the solve goes on streaming
 };
 
 // operator of the solve: FP64 recomputes the couplings of poisson_pcorr from the face

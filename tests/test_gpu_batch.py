@@ -263,7 +263,7 @@ def test_run_after_a_change_of_precision(tanks, added):
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_scheduled_run_whose_launches_are_given_up(precision):
-    """Every on-chip launch given up (onchip_wait 0), in lockstep and scheduled: the same bits."""
+    """Every on-chip launch given up (onchip_giveup), in lockstep and scheduled: the same bits."""
     from reef3d_amd import Batch
     lock, it_lock = _run(TANKS, 2, precision)
     for scheduled in (False, True):
@@ -272,7 +272,7 @@ def test_scheduled_run_whose_launches_are_given_up(precision):
         for tid, (kw, f) in zip(ids, TANKS):
             _initial(B, tid, kw, f)
         B.solver_config(precision)
-        B.set_control("onchip_wait", 0)
+        B.set_control("onchip_giveup", 1)
         _prepare(B)
         print(precision, scheduled, flush=True)
         it = B.run(2) if scheduled else [B.fc3_step()[0] for _ in range(2)][-1]

@@ -172,9 +172,9 @@ def test_a_solve_streams_where_there_is_no_workspace(precision):
 @pytest.mark.parametrize("shape", [(64, 1, 4, 0), (1150, 1, 157, 0), (65, 5, 33, 1)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_a_launch_that_is_given_up_streams_on(shape, precision):
-    """A wait limit of 0: the blocks of a tank leave at the commit with nothing stored, and the
-    solve streams, with the same bits.  The next 63 solves stream without a launch, the 64th
-    tries again, and a limit that allows it runs on chip.  A tank of one block waits for nothing
+    """The abort bit set before a launch: the blocks of a tank leave at the latest at the commit with
+    nothing stored, and the solve streams, with the same bits.  The next 63 solves stream without a launch, the 64th
+    tries again, and without it the solves run on chip.  A tank of one block waits for nothing
     and is not given up."""
     nx, ny, nz, jdir = shape
     _, D, _, _ = _system(nx, ny, nz, jdir, seed=31)
@@ -192,7 +192,7 @@ def test_a_launch_that_is_given_up_streams_on(shape, precision):
     print(shape, precision, flush=True)
     r, x, chip, stream = run(20000)
     assert (chip, stream) == (1, 0)
-    D.set_control("onchip_wait", 0)
+    D.set_control("onchip_giveup", 1)
     r2, x2, chip, stream = run(20000)
     assert (chip, stream) == ((1, 0) if one_block else (1, 1))
     assert r2 == r and np.array_equal(x2, x)
@@ -201,6 +201,6 @@ def test_a_launch_that_is_given_up_streams_on(shape, precision):
         again = run(3)
         assert again[0] == first[0] and np.array_equal(again[1], first[1]) and again[2] == (1 if one_block else 0)
     assert run(3)[2] == 1
-    D.set_control("onchip_wait", 0.5)
+    D.set_control("onchip_giveup", 0)
     r2, x2, chip, stream = run(20000)
     assert (chip, stream) == (1, 0) and r2 == r and np.array_equal(x2, x)
