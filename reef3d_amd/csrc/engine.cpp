@@ -572,7 +572,7 @@ int Engine::sync_tables()
     all_ = make_sets(act);
     cur_ = &all_;
     for(TankHost& t : tanks) t.chip_h.fill(-1);   // plans may have changed
-    for(int m = 0; m < 2; ++m) all_chip_[m] = chip_plan(act, m != 0);
+    for(int m = 0; m < 2; ++m) all_chip_[m] = chip_plan(act, m != 0, false);
     solving_key_.clear();
     solving_sets_.clear();
     solving_chip_ = ChipPlan();
@@ -1093,21 +1093,22 @@ static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 // (CHIP_US) and iterations in proportion to the tank's longest side, the longest first.
 //
 // Beside that stands the end of the whole set streamed together (stream_end), whose tanks share
-// their launches.  Beside a tank that has to stream the others stream with it if that is shorter:
-// they add little to launches that are made anyway, and on chip they hold it up (three steps of a
-// mixed 2049x256 tank with three small ones: 629 ms with those on chip, 573 streamed).  A set
-// that fits as a whole is streamed where that is shorter by 13 % or more, since a streamed set
-// waits for the tank with the most iterations: the solves of one step of mixed 1150x157 tanks
-// take, on chip and streamed, 33 and 61 ms for one tank, 212 and 228 for 8, 446 and 367 for 16;
-// of mixed 192x32x64 tanks 14 and 23 for one, 221 and 202 for 16; of FP64 1150x157 tanks 29 and
-// 61 for one, 338 and 478 for 16.
+// their launches.  In scheduled steps, beside a tank that has to stream, the others stream with it
+// if that is shorter: they add little to launches that are made anyway, and a whole solve on chip
+// holds up the segments that the others have reached (three steps of a mixed 2049x256 tank with
+// three small ones: 629 ms with those on chip, 573 streamed).  Else a set is streamed where that
+// is shorter by 5 % or more, since a streamed set waits for the tank with the most iterations:
+// the solves of one step of mixed 1150x157 tanks take, on chip and streamed, 33 and 61 ms for one
+// tank, 212 and 228 for 8, 446 and 367 for 16; of mixed 192x32x64 tanks 14 and 23 for one, 221 and
+// 202 for 16; of FP64 1150x157 tanks 29 and 61 for one, 338 and 478 for 16.
 //
 // us an iteration on chip with 2, 4, 8 tiles per block, measured: [FP64, mixed][2-D, 3-D]
 static const double CHIP_US[2][2][3] = {{{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}}, {{11.5, 16.5, 20.5}, {15.0, 18.5, 22.5}}};
 // a streamed iteration, measured: its launches, then us per work item and per tile of the set
-// [FP64, mixed][2-D, 3-D] (sets of 7000 to 25 000 tiles: 0.8 to 0.9 of the sum for smaller ones)
-static const double STREAM_US = 28.0, ITEM_US[2][2] = {{0.0, 0.0119}, {0.0, 0.0114}},
-                    TILE_US[2][2] = {{0.0125, 0.0106}, {0.0076, 0.0055}};
+// [FP64, mixed][2-D, 3-D] (2-D sets of 2000 to 39 000 tiles with 1, 2 and 4 tiles per item within
+// 20 %, 3-D sets of 9000 to 25 000 tiles; smaller sets take less)
+static const double STREAM_US = 28.0, ITEM_US[2][2] = {{0.0040, 0.0119}, {0.0033, 0.0114}},
+                    TILE_US[2][2] = {{0.0105, 0.0106}, {0.0055, 0.0055}};
 
 // estimated end of the tanks' streamed solves: every tank takes part in the launches until its
 // iterations, in proportion to its longest side, are done
@@ -1135,7 +1136,7 @@ double Engine::stream_end(const std::vector<int>& slots, bool mixed) const
     return end;
 }
 
-Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
+Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed, bool scheduled)
 {
     ChipPlan P;
     struct Tank
@@ -1186,7 +1187,7 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed)
         }
         if(l == 0 || end < best_end) best = l, best_end = end;
     }
-    const double share = P.rest.empty() ? 0.87 : 1.0;
+    const double share = scheduled && !P.rest.empty() ? 1.0 : 0.95;
     if(stream_end(slots_in, mixed) < share * (best_end + stream_end(P.rest, mixed))) return P;
     P.stream_all = false;
     for(const Tank& k : fit)
@@ -2060,7 +2061,7 @@ int Engine::pump(std::vector<int>& stepped)
         if(solving != solving_key_ || (int)mixed != solving_mixed_)
         {
             solving_sets_ = make_sets(solving);
-            solving_chip_ = chip_plan(solving, mixed);
+            solving_chip_ = chip_plan(solving, mixed, true);
             solving_key_ = solving;
             solving_mixed_ = mixed;
         }

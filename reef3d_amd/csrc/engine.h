@@ -363,7 +363,7 @@ private:
     void chip_heard(const BiState& st);
     hipEvent_t chip_ev_ = nullptr;
     double stream_end(const std::vector<int>& slots, bool mixed) const;
-    ChipPlan chip_plan(const std::vector<int>& slots, bool mixed);
+    ChipPlan chip_plan(const std::vector<int>& slots, bool mixed, bool scheduled);
     bool chip_ready(const ChipPlan& P);
     int chip_launch(ChipPlan& P, int kind, int x, int rhs, int cap);
     int enqueue_iterations(int kind, int x, int rhs, int iters, int chip_cap);
