@@ -1090,14 +1090,16 @@ static const char* const MAT_NAMES[4] = {"mat_p", "mat_v", "mat_t", "mat_x"};
 // more blocks the later ones start in order as CUs come free.  Few tiles per block keep an
 // iteration short, many keep more tanks on the chip at once.  The launch takes the tiles per
 // block (2, 4 or 8) with the shortest end of all tanks, estimated from the time of an iteration
-// (CHIP_US) and iterations in proportion to the tank's longest side, the longest first.
+// (CHIP_US) and the tank's iterations (tank_iters), the longest first.
 //
 // Beside that stands the end of the whole set streamed together (stream_end), whose tanks share
 // their launches.  In scheduled steps, beside a tank that has to stream, the others stream with it
-// if that is shorter: they add little to launches that are made anyway, and a whole solve on chip
-// holds up the segments that the others have reached (three steps of a mixed 2049x256 tank with
-// three small ones: 629 ms with those on chip, 573 streamed).  Else a set is streamed where that
-// is shorter by 5 % or more, since a streamed set waits for the tank with the most iterations:
+// if that is shorter by 2 % or more: they add little to launches that are made anyway, and a whole
+// solve on chip holds up the segments that the others have reached (three steps of a mixed
+// 2049x256 tank with three small ones: 629 ms with those on chip, 573 streamed).  Where it is the
+// same the small tank ends sooner on chip (a 192x32x64 tank served beside 15 of up to 1792x192:
+// 2.4 s instead of 6.7, the stream 14.8 s both ways).  Else a set is streamed where that is
+// shorter by 5 % or more, since a streamed set waits for the tank with the most iterations:
 // the solves of one step of mixed 1150x157 tanks take, on chip and streamed, 33 and 61 ms for one
 // tank, 212 and 228 for 8, 446 and 367 for 16; of mixed 192x32x64 tanks 14 and 23 for one, 221 and
 // 202 for 16; of FP64 1150x157 tanks 29 and 61 for one, 338 and 478 for 16.
@@ -1110,23 +1112,27 @@ static const double CHIP_US[2][2][3] = {{{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}}
 static const double STREAM_US = 28.0, ITEM_US[2][2] = {{0.0040, 0.0119}, {0.0033, 0.0114}},
                     TILE_US[2][2] = {{0.0105, 0.0106}, {0.0055, 0.0055}};
 
+// Iterations of a solve, in units that cancel: in proportion to the geometric mean of length and
+// height (6 to 9 times that for the three mixed solves of a step of 2-D tanks of 128x64 to
+// 1700x240, 5.5 to 7 times for 3-D ones; against the longest side it was 2.3 to 6 times).
+static double tank_iters(const HostGrid& h) { return std::sqrt((double)h.nx * (double)h.nz); }
+
 // estimated end of the tanks' streamed solves: every tank takes part in the launches until its
-// iterations, in proportion to its longest side, are done
+// iterations are done
 double Engine::stream_end(const std::vector<int>& slots, bool mixed) const
 {
-    std::vector<std::pair<int, double>> t;   // longest side, us per iteration
+    std::vector<std::pair<double, double>> t;   // iterations, us per iteration
     double all = 0.0;
     for(int q : slots)
     {
         const HostGrid& h = tanks[q].hg;
         const TileShape& s = tanks[q].dev.shape;
         const double us = ITEM_US[mixed][h.jdir] * s.nitems + TILE_US[mixed][h.jdir] * s.ntiles;
-        t.emplace_back(std::max(h.nx, std::max(h.ny, h.nz)), us);
+        t.emplace_back(tank_iters(h), us);
         all += us;
     }
     std::sort(t.begin(), t.end());
-    double end = 0.0;
-    int at = 0;
+    double end = 0.0, at = 0.0;
     for(const auto& k : t)
     {
         end += (k.first - at) * (STREAM_US + all);
@@ -1141,7 +1147,9 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed,
     ChipPlan P;
     struct Tank
     {
-        int slot, side, per[3], nb[3];   // blocks and tiles per block for 2, 4, 8 (or the next that fits)
+        int slot;
+        double iters;
+        int per[3], nb[3];   // blocks and tiles per block for 2, 4, 8 (or the next that fits)
     };
     std::vector<Tank> fit;
     for(int q : slots_in)
@@ -1149,7 +1157,7 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed,
         TankHost& t = tanks[q];
         Tank k;
         k.slot = q;
-        k.side = std::max(t.hg.nx, std::max(t.hg.ny, t.hg.nz));
+        k.iters = tank_iters(t.hg);
         int nb = 0, per = 2;
         for(int l = 2; l >= 0; --l)
         {
@@ -1164,7 +1172,7 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed,
             P.rest.push_back(q);
     }
     if(fit.empty()) return P;
-    std::stable_sort(fit.begin(), fit.end(), [](const Tank& a, const Tank& b) { return a.side > b.side; });
+    std::stable_sort(fit.begin(), fit.end(), [](const Tank& a, const Tank& b) { return a.iters > b.iters; });
     int best = 0;
     double best_end = 0.0;
     for(int l = 0; l < 3; ++l)
@@ -1180,14 +1188,14 @@ Engine::ChipPlan Engine::chip_plan(const std::vector<int>& slots_in, bool mixed,
                 free_cus += running.begin()->second;
                 running.erase(running.begin());
             }
-            const double e = now + k.side * CHIP_US[mixed][tanks[k.slot].hg.jdir][k.per[l]];
+            const double e = now + k.iters * CHIP_US[mixed][tanks[k.slot].hg.jdir][k.per[l]];
             running.emplace(e, k.nb[l]);
             free_cus -= k.nb[l];
             end = std::max(end, e);
         }
         if(l == 0 || end < best_end) best = l, best_end = end;
     }
-    const double share = scheduled && !P.rest.empty() ? 1.0 : 0.95;
+    const double share = scheduled && !P.rest.empty() ? 0.98 : 0.95;
     if(stream_end(slots_in, mixed) < share * (best_end + stream_end(P.rest, mixed))) return P;
     P.stream_all = false;
     for(const Tank& k : fit)
