@@ -1112,10 +1112,10 @@ static const double CHIP_US[2][2][3] = {{{11.0, 16.0, 17.5}, {15.0, 19.0, 25.0}}
 static const double STREAM_US = 28.0, ITEM_US[2][2] = {{0.0040, 0.0119}, {0.0033, 0.0114}},
                     TILE_US[2][2] = {{0.0105, 0.0106}, {0.0055, 0.0055}};
 
-// Iterations of a solve, in units that cancel: in proportion to the geometric mean of length and
-// height (6 to 9 times that for the three mixed solves of a step of 2-D tanks of 128x64 to
-// 1700x240, 5.5 to 7 times for 3-D ones; against the longest side it was 2.3 to 6 times).
-static double tank_iters(const HostGrid& h) { return std::sqrt((double)h.nx * (double)h.nz); }
+// Iterations of a solve, in units that cancel: in proportion to the height, which lies between
+// the free surface and the bed (a step's three solves, 179 2-D tanks of 96 to 1700 columns: 15
+// per cell of height, 12 % standard deviation; against the longest side 61 %; 3-D tanks 5 to 10)
+static double tank_iters(const HostGrid& h) { return (h.jdir ? 1.0 : 1.75) * (double)h.nz; }
 
 // estimated end of the tanks' streamed solves: every tank takes part in the launches until its
 // iterations are done
